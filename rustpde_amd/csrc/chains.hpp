@@ -31,15 +31,15 @@ inline int buf_len(int nr) { return pad(nr + 6) + 1; }
 
 // A row of nr values -> LDS (element i at pad(i + 2), zeros at i in [-2, 0) and
 // [nr, nr + 4)) by the nthr threads of a group, thread tid; all loads are issued before the
-// first store.  Needs MAXQ * nthr >= nr + 6.
-template <int MAXQ>
+// first store.  Needs MAXQ * nthr >= nr + 6.  The row's values lie INC apart.
+template <int MAXQ, int INC = 1>
 __device__ __forceinline__ void stage_row(double* buf, const double* __restrict__ row, bool valid, int nr, int tid,
                                           int nthr) {
   double v[MAXQ];
 #pragma unroll
   for (int q = 0; q < MAXQ; ++q) {
     const int i = tid + q * nthr - 2;
-    v[q] = (valid && i >= 0 && i < nr) ? row[i] : 0.0;
+    v[q] = (valid && i >= 0 && i < nr) ? row[i * INC] : 0.0;
   }
 #pragma unroll
   for (int q = 0; q < MAXQ; ++q) {
@@ -49,8 +49,8 @@ __device__ __forceinline__ void stage_row(double* buf, const double* __restrict_
 }
 
 // LDS row -> HBM: row[i] = x_i, or row[i] = x_i (-1) + row[i] with `subtract` (old values
-// loaded first).  Needs MAXQ * nthr >= m.
-template <int MAXQ>
+// loaded first).  Needs MAXQ * nthr >= m.  The row's values lie INC apart.
+template <int MAXQ, int INC = 1>
 __device__ __forceinline__ void unstage_row(const double* buf, double* __restrict__ row, bool valid, int m, int tid,
                                             int nthr, bool subtract) {
 #pragma clang fp contract(off)
@@ -60,7 +60,7 @@ __device__ __forceinline__ void unstage_row(const double* buf, double* __restric
 #pragma unroll
     for (int q = 0; q < MAXQ; ++q) {
       const int i = tid + q * nthr;
-      old[q] = i < m ? row[i] : 0.0;
+      old[q] = i < m ? row[i * INC] : 0.0;
     }
   }
 #pragma unroll
@@ -68,7 +68,7 @@ __device__ __forceinline__ void unstage_row(const double* buf, double* __restric
     const int i = tid + q * nthr;
     if (i < m) {
       const double x = buf[pad(i + 2)];
-      row[i] = subtract ? x * (-1.0) + old[q] : x;
+      row[i * INC] = subtract ? x * (-1.0) + old[q] : x;
     }
   }
 }

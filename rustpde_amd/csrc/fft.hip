@@ -47,7 +47,9 @@ struct CGeo {
 // Tin: input type, V: arithmetic (and LDS) type, Tout: output type.  Columns j >= nzc are
 // zero on input (the rows a y-dealiasing cut cleared): a block whose columns all lie there
 // writes their zero spectra without loading or transforming.
-template <int L, typename Tin, typename V, typename Tout>
+// IL: the spectra are interleaved (re, im) pairs instead of split planes, written as 16-byte
+// pairs (Space2's arrays, whose callers hold them that way: no separate merge pass).
+template <int L, typename Tin, typename V, typename Tout, bool IL = false>
 __global__ __launch_bounds__((CGeo<L, sizeof(V)>::T)) void rfft_cols_kernel(const Tin* __restrict__ X, Tout* __restrict__ Y,
                                                                int cols, int cut, const V* __restrict__ tw,
                                                                long sx, long sy, int nzc) {
@@ -64,8 +66,12 @@ __global__ __launch_bounds__((CGeo<L, sizeof(V)>::T)) void rfft_cols_kernel(cons
     for (int e = tid; e < m * C; e += T) {
       const int c = e % C, k = e / C, j = j0 + c;
       if (j >= cols) continue;
-      Y[(size_t)k * cols + j] = (Tout)0;
-      Y[(size_t)(m + k) * cols + j] = (Tout)0;
+      if constexpr (IL) {
+        reinterpret_cast<fftlds::cpair<Tout>*>(Y)[(size_t)k * cols + j] = fftlds::cpair<Tout>{0, 0};
+      } else {
+        Y[(size_t)k * cols + j] = (Tout)0;
+        Y[(size_t)(m + k) * cols + j] = (Tout)0;
+      }
     }
     return;
   }
@@ -105,14 +111,18 @@ __global__ __launch_bounds__((CGeo<L, sizeof(V)>::T)) void rfft_cols_kernel(cons
       xr = 0;
       xi = 0;
     }
-    Y[(size_t)k * cols + j] = (Tout)xr;
-    Y[(size_t)(m + k) * cols + j] = (Tout)xi;
+    if constexpr (IL) {
+      reinterpret_cast<fftlds::cpair<Tout>*>(Y)[(size_t)k * cols + j] = fftlds::cpair<Tout>{(Tout)xr, (Tout)xi};
+    } else {
+      Y[(size_t)k * cols + j] = (Tout)xr;
+      Y[(size_t)(m + k) * cols + j] = (Tout)xi;
+    }
   }
 }
 
 // The work of one irfft block on columns j0 .. j0 + C - 1; FULL: all of them lie below cols
 // (every block but the last), so the column guards drop out.
-template <bool FULL, int L, typename Tin, typename V, typename Tout, int S, typename ZB>
+template <bool FULL, int L, typename Tin, typename V, typename Tout, int S, bool IL, typename ZB>
 __device__ __forceinline__ void irfft_block(const ZB& z, const Tin* __restrict__ X, Tout* __restrict__ Y, int cols,
                                             int times, double sc_d, const V* __restrict__ tw, int j0) {
 #pragma clang fp contract(off)
@@ -136,7 +146,15 @@ __device__ __forceinline__ void irfft_block(const ZB& z, const Tin* __restrict__
     const int e = tid + q * T, c = e % C, k = e / C, j = j0 + c;
     const bool ok = e < m * C && (FULL || j < cols);
     const size_t ia = ok ? (size_t)k * cols + j : 0;
-    const Tin xa = X[ia], xb = X[ia + (size_t)m * cols];
+    Tin xa, xb;
+    if constexpr (IL) {
+      const fftlds::cpair<Tin> x = reinterpret_cast<const fftlds::cpair<Tin>*>(X)[ia];
+      xa = x.r;
+      xb = x.i;
+    } else {
+      xa = X[ia];
+      xb = X[ia + (size_t)m * cols];
+    }
     va[q] = ok ? (V)xa : (V)0;
     vb[q] = ok ? (V)xb : (V)0;
   }
@@ -188,7 +206,7 @@ __device__ __forceinline__ void irfft_block(const ZB& z, const Tin* __restrict__
 // Batch entries b < split (all of them when split = 0) apply (i k)^times / sc and write Y;
 // entries b >= split read input b - split again, apply (i k)^times1 / sc1 and write Y1 (the
 // values and the x-derivatives of the same fields in one launch).
-template <int L, typename Tin, typename V, typename Tout>
+template <int L, typename Tin, typename V, typename Tout, bool IL = false>
 __global__ __launch_bounds__((CGeo<L, sizeof(V)>::T)) void irfft_cols_kernel(const Tin* __restrict__ X, Tout* __restrict__ Y,
                                                                 int cols, int times, double sc_d,
                                                                 const V* __restrict__ tw, long sx, long sy,
@@ -209,8 +227,8 @@ __global__ __launch_bounds__((CGeo<L, sizeof(V)>::T)) void irfft_cols_kernel(con
   X += sx * b;
   Y += sy * b;
   const int j0 = xcd_remap(blockIdx.x, gridDim.x) * C;
-  if (j0 + C <= cols) irfft_block<true, L, Tin, V, Tout, S>(z, X, Y, cols, times, sc_d, tw, j0);
-  else irfft_block<false, L, Tin, V, Tout, S>(z, X, Y, cols, times, sc_d, tw, j0);
+  if (j0 + C <= cols) irfft_block<true, L, Tin, V, Tout, S, IL>(z, X, Y, cols, times, sc_d, tw, j0);
+  else irfft_block<false, L, Tin, V, Tout, S, IL>(z, X, Y, cols, times, sc_d, tw, j0);
 }
 
 void check(const char* what) {
@@ -223,19 +241,19 @@ void check_n(int n) {
   if (n > 2048) throw std::invalid_argument("fft: length above 2048 exceeds the LDS budget");
 }
 
-template <int L, typename Tin, typename V, typename Tout>
+template <int L, typename Tin, typename V, typename Tout, bool IL = false>
 void launch_rfft(hipStream_t s, const Tin* X, Tout* Y, int cols, int cut, int batch, long sx, long sy, int nzc) {
   using G = CGeo<L, sizeof(V)>;
   const unsigned blocks = (unsigned)((cols + G::C - 1) / G::C);
-  RBC_LAUNCH((rfft_cols_kernel<L, Tin, V, Tout>), dim3(blocks, batch), dim3(G::T), 0, s, X, Y, cols, cut,
+  RBC_LAUNCH((rfft_cols_kernel<L, Tin, V, Tout, IL>), dim3(blocks, batch), dim3(G::T), 0, s, X, Y, cols, cut,
              twiddles<V>(L), sx, sy, nzc < 0 ? cols : nzc);
 }
-template <int L, typename Tin, typename V, typename Tout>
+template <int L, typename Tin, typename V, typename Tout, bool IL = false>
 void launch_irfft(hipStream_t s, const Tin* X, Tout* Y, int cols, int times, double sc, int batch, long sx, long sy,
                   Tout* Y1 = nullptr, int split = 0, int times1 = 0, double sc1 = 1.0) {
   using G = CGeo<L, sizeof(V)>;
   const unsigned blocks = (unsigned)((cols + G::C - 1) / G::C);
-  RBC_LAUNCH((irfft_cols_kernel<L, Tin, V, Tout>), dim3(blocks, batch), dim3(G::T), 0, s, X, Y, cols, times, sc,
+  RBC_LAUNCH((irfft_cols_kernel<L, Tin, V, Tout, IL>), dim3(blocks, batch), dim3(G::T), 0, s, X, Y, cols, times, sc,
              twiddles<V>(L), sx, sy, Y1, split, times1, sc1);
 }
 
@@ -276,6 +294,26 @@ void irfft_cols(hipStream_t s, const double* X, double* Y, int n, int cols, int 
   RBC_FFT_SWITCH(n, RBC_IRFFT)
 #undef RBC_IRFFT
   check("irfft_cols");
+}
+
+void rfft_cols_interleaved(hipStream_t s, const double* X, double* Y, int n, int cols, int batch) {
+  check_n(n);
+  if (batch < 1 || batch > 65535 || cols < 1) throw std::invalid_argument("rfft_cols_interleaved: bad batch or cols");
+  const long sx = (long)n * cols, sy = (long)(n + 2) * cols;
+#define RBC_RFFTI(LL) launch_rfft<LL, double, double, double, true>(s, X, Y, cols, n / 2 + 1, batch, sx, sy, -1)
+  RBC_FFT_SWITCH(n, RBC_RFFTI)
+#undef RBC_RFFTI
+  check("rfft_cols_interleaved");
+}
+
+void irfft_cols_interleaved(hipStream_t s, const double* X, double* Y, int n, int cols, int batch) {
+  check_n(n);
+  if (batch < 1 || batch > 65535 || cols < 1) throw std::invalid_argument("irfft_cols_interleaved: bad batch or cols");
+  const long sx = (long)(n + 2) * cols, sy = (long)n * cols;
+#define RBC_IRFFTI(LL) launch_irfft<LL, double, double, double, true>(s, X, Y, cols, 0, 1.0, batch, sx, sy)
+  RBC_FFT_SWITCH(n, RBC_IRFFTI)
+#undef RBC_IRFFTI
+  check("irfft_cols_interleaved");
 }
 
 void irfft_cols_pair(hipStream_t s, const double* X, double* Y0, double* Y1, int n, int cols, int times1, double sc1,

@@ -2030,7 +2030,7 @@ class Space {
   bool cplx;
   hipStream_t st = nullptr;
   OpCache X, Y;
-  DBuf W1, W2, W3, W9;
+  DBuf W1, W2, W3, W4;
   Space(int k0, int n0, int k1, int n1) : b0((Kind)k0, n0), b1((Kind)k1, n1), cplx(k0 == FO), X(false, 1.0), Y(true, 1.0) {
     if (k1 == FO) throw std::invalid_argument("axis 1 must be a Chebyshev basis");
     if (n0 < 6 || n1 < 6) throw std::invalid_argument("sizes must be >= 6");
@@ -2042,56 +2042,93 @@ class Space {
   int r_phys() const { return b0.n; }
   int r_spec() const { return cplx ? 2 * b0.m : b0.m; }
   int r_ortho() const { return cplx ? 2 * b0.m : b0.n; }
-  void ensure(size_t n) {
-    if (W1.n < n) { W1.alloc(n); W2.alloc(n); W3.alloc(n); W9.alloc(n); }
+  std::unique_ptr<DBand> band;  // stencil taps of a composite axis-1 basis
+  std::unique_ptr<DTdma> tdma;  // its from_ortho tables
+  const double* stencil_coef() {
+    if (b1.k == CHEB) return nullptr;
+    if (!band) {
+      band = std::make_unique<DBand>();
+      make_stencil_band(b1, *band);
+    }
+    return band->coef.p;
   }
-  // x-op with the scale used for gradients
-  const double* xop(const std::string& name, const double* in, int cols, double* out, double sc) {
+  const double* tdma_tab() {
+    if (!tdma) {
+      tdma = std::make_unique<DTdma>();
+      make_tdma(b1, *tdma);
+    }
+    return tdma->tabp.p;
+  }
+  // axis-1 bases and lengths of the row kernels (rowops.hip)
+  bool rows_ok() const { return (b1.k == CHEB || b1.k == CD || b1.k == CN) && row_ops_supported(b1.n); }
+  // x-operator on nb consecutive arrays [rows_in, cols], split planes when Fourier
+  const double* xop(const char* name, const double* in, int cols, double* out, int nb) {
+    const std::string op_name = name;
     if (b0.k == FO) {
-      if (name == "S" || name == "FO") return in;
-      if (fft_supported(b0.n) && (name == "BS" || name == "FS")) {  // real FFT kernels
-        if (name == "BS") irfft_cols(st, in, out, b0.n, cols, 0, 1.0);
-        else rfft_cols(st, in, out, b0.n, cols, b0.m);
+      if (op_name == "S" || op_name == "FO") return in;
+      if (fft_supported(b0.n) && (op_name == "BS" || op_name == "FS")) {  // real FFT kernels
+        const long sp = 2L * b0.m * cols, ph = (long)b0.n * cols;
+        if (op_name == "BS") irfft_cols(st, in, out, b0.n, cols, 0, 1.0, nb, sp, ph);
+        else rfft_cols(st, in, out, b0.n, cols, b0.m, nb, ph, sp);
         return out;
       }
-      if (name == "DS" || name == "DDS") {
-        fourier_diff(st, in, out, b0.m, cols, cols, name == "DS" ? 1 : 2, sc);
+      if (op_name == "DS" || op_name == "DDS") {
+        const size_t e = 2 * (size_t)b0.m * cols;
+        for (int b = 0; b < nb; ++b) fourier_diff(st, in + b * e, out + b * e, b0.m, cols, cols, op_name == "DS" ? 1 : 2, 1.0);
         return out;
       }
-    } else if (b0.k == CHEB && (name == "S" || name == "FO")) {
+    } else if (b0.k == CHEB && (op_name == "S" || op_name == "FO")) {
       return in;
     }
-    const DOp& op = X.get(b0, name);
-    gemm(st, op.rows, cols, op.cols, op.b.p, op.cols, in, cols, out, cols, 1.0, 0.0);
+    const DOp& op = X.get(b0, op_name);
+    gemm_mfma_batched(st, op.rows, cols, op.cols, op.b.p, op.cols, 0, in, cols, (long)op.cols * cols, out, cols,
+                      (long)op.rows * cols, nb, 1.0, 0.0);
     return out;
   }
-  std::unique_ptr<DBand> band;  // stencil taps of a composite axis-1 basis
-  const double* yop(const std::string& name, const double* in, int rows, double* out) {
-    if (b1.k == CHEB && (name == "S" || name == "FO")) return in;
+  // y-operator on `rows` consecutive real rows
+  const double* yop(const char* name, const double* in, long rows, double* out) {
+    const std::string op_name = name;
+    if (b1.k == CHEB && (op_name == "S" || op_name == "FO")) return in;
     if ((b1.k == CHEB || b1.k == CD || b1.k == CN) && cheb_y_supported(b1.n)) {  // FFT-based DCT-I
-      if (name == "BS") {
-        if (b1.k != CHEB && !band) {
-          band = std::make_unique<DBand>();
-          make_stencil_band(b1, *band);
-        }
-        cheb_y_backward(st, in, b1.m, b1.m, out, b1.n, rows, b1.n, band ? band->coef.p : nullptr,
-                        band ? band->mask.p : nullptr, 0, 1.0, nullptr, 0, 0.0);
+      if (op_name == "BS") {
+        const double* coef = stencil_coef();
+        cheb_y_backward(st, in, b1.m, b1.m, out, b1.n, (int)rows, b1.n, coef, band ? band->mask.p : nullptr, 0, 1.0,
+                        nullptr, 0, 0.0);
         return out;
       }
-      if (name == "FS" && b1.k == CHEB) {
-        cheb_y_forward(st, in, b1.n, out, b1.n, rows, b1.n, b1.n);
+      if (op_name == "FS" && (b1.k == CHEB || rows_ok())) {
+        double* to = b1.k == CHEB ? out : W3.p;
+        cheb_y_forward(st, in, b1.n, to, b1.n, (int)rows, b1.n, b1.n);
+        if (b1.k != CHEB) composite_rows(st, to, out, rows, false, b1.m, tdma_tab());
         return out;
       }
     }
-    const DOp& op = Y.get(b1, name);
-    gemm(st, rows, op.cols, op.rows, in, op.rows, op.b.p, op.cols, out, op.cols, 1.0, 0.0);
+    if (rows_ok()) {
+      if (op_name == "S" || op_name == "DS" || op_name == "DDS") {
+        ortho_rows(st, in, out, rows, false, b1.m, b1.n, stencil_coef(), op_name == "S" ? 0 : op_name == "DS" ? 1 : 2, 0, 1,
+                   1.0);
+        return out;
+      }
+      if (op_name == "FO") {
+        composite_rows(st, in, out, rows, false, b1.m, tdma_tab());
+        return out;
+      }
+    }
+    const DOp& op = Y.get(b1, op_name);
+    gemm_mfma(st, (int)rows, op.cols, op.rows, in, op.rows, op.b.p, op.cols, out, op.cols, 1.0, 0.0);
     return out;
+  }
+  // the work arrays hold up to this many doubles (512 MiB) of a batch at a time, or one field
+  // and this many rows (the dense row operators' 32-row tiles along one grid axis)
+  static constexpr size_t CHUNK_DOUBLES = (size_t)64 << 20, CHUNK_ROWS = (size_t)1 << 20;
+  static bool overlap(const double* a, size_t na, const double* b, size_t nb) {
+    const uintptr_t pa = (uintptr_t)a, pb = (uintptr_t)b;
+    return pa < pb + 8 * nb && pb < pa + 8 * na;
   }
   // generic 2-D application on device interleaved/real buffers
   void run(int op, const double* in, double* out, int batch, int d0, int d1, double s0, double s1) {
+    if (op == 4 && (d0 > 2 || d1 > 2)) throw std::invalid_argument("derivative order > 2");
     const size_t big = (size_t)std::max(r_ortho(), b0.n) * b1.n + 16;
-    ensure(big);
-    const bool in_c = cplx && op != 0, out_c = cplx && op != 1;
     int in_r, in_c1, out_r, out_c1;
     switch (op) {
       case 0: in_r = b0.n; in_c1 = b1.n; out_r = r_spec(); out_c1 = b1.m; break;
@@ -2101,46 +2138,79 @@ class Space {
       default: in_r = r_spec(); in_c1 = b1.m; out_r = r_ortho(); out_c1 = b1.n; break;
     }
     const size_t in_sz = (size_t)in_r * in_c1, out_sz = (size_t)out_r * out_c1;
-    for (int b = 0; b < batch; ++b) {
-      const double* src = in + b * in_sz;
+    // a whole chunk of the batch per launch; arrays that overlap (a transform in place) go one
+    // field at a time through the work arrays, each read before its result is written
+    const bool inplace = overlap(in, in_sz * batch, out, out_sz * batch);
+    const size_t rows = (size_t)std::max(r_ortho(), b0.n);
+    const size_t most = std::max<size_t>(1, std::min(CHUNK_DOUBLES / big, CHUNK_ROWS / rows));
+    const int chunk = inplace ? 1 : (int)std::min<size_t>((size_t)std::min(batch, 65535), most);
+    if (inplace && W4.n < big) W4.alloc(big);
+    for (DBuf* w : {&W1, &W2, &W3})
+      if (w->n < big * chunk) w->alloc(big * chunk);
+    GemmNoTune no_tune;  // a call's first use of a shape is not spent on timing tiles
+    for (int b = 0; b < batch; b += chunk) {
+      const int nb = std::min(chunk, batch - b);
       double* dst = out + b * out_sz;
-      const double* x = src;
-      if (in_c) { interleaved_to_split(st, src, W3.p, in_r / 2, in_c1); x = W3.p; }
-      const double* r = nullptr;
-      // gradient scale divides by s0^d0 s1^d1 (space2.rs:256-262); folded into the x part
-      const double sc = std::pow(s0, d0) * std::pow(s1, d1);
-      if (op == 0) {  // forward: axis 1 then axis 0
-        const double* a = yop("FS", x, b0.n, W1.p);
-        r = xop("FS", a, b1.m, W2.p, 1.0);
-      } else if (op == 1) {  // backward: axis 0 then axis 1
-        const double* a = xop("BS", x, b1.m, W1.p, 1.0);
-        r = yop("BS", a, b0.n, W2.p);
-      } else if (op == 2) {
-        const double* a = xop("S", x, b1.m, W1.p, 1.0);
-        r = yop("S", a, r_ortho(), W2.p);
-      } else if (op == 3) {
-        const double* a = xop("FO", x, b1.n, W1.p, 1.0);
-        r = yop("FO", a, r_spec(), W2.p);
-      } else {
-        if (d0 > 2 || d1 > 2) throw std::invalid_argument("derivative order > 2");
-        const char* nx_ = d0 == 0 ? "S" : d0 == 1 ? "DS" : "DDS";
-        const char* ny_ = d1 == 0 ? "S" : d1 == 1 ? "DS" : "DDS";
-        const double* a = xop(nx_, x, b1.m, W1.p, 1.0);
-        r = yop(ny_, a, r_ortho(), W2.p);
-        if (sc != 1.0) {
-          if (r != W2.p) { HIPCHECK(hipMemcpyAsync(W2.p, r, sizeof(double) * r_ortho() * b1.n, hipMemcpyDeviceToDevice, st)); r = W2.p; }
-          if (b0.k == FO) {
-            // complex division by (sc, 0): (a sc) / sc^2 per component
-            fourier_diff(st, W2.p, W2.p, b0.m, b1.n, b1.n, 0, sc);
-          } else {
-            ew_scale(st, W2.p, W2.p, 1.0 / sc, (long)r_ortho() * b1.n);
-          }
-        }
-      }
-      if (out_c) split_to_interleaved(st, r, dst, out_r / 2, out_c1);
-      else HIPCHECK(hipMemcpyAsync(dst, r, sizeof(double) * out_sz, hipMemcpyDeviceToDevice, st));
+      const double* r = apply(op, in + b * in_sz, inplace ? W4.p : dst, nb, in_r, in_c1, out_r, out_c1, d0, d1, s0, s1);
+      if (r != dst) HIPCHECK(hipMemcpyAsync(dst, r, sizeof(double) * out_sz * nb, hipMemcpyDeviceToDevice, st));
     }
     HIPCHECK(hipStreamSynchronize(st));
+  }
+  // the operation on nb fields; the result is at the returned address (dst, or an identity's input)
+  const double* apply(int op, const double* src, double* dst, int nb, int in_r, int in_c1, int out_r, int out_c1, int d0,
+                      int d1, double s0, double s1) {
+    // gradient scale divides by s0^d0 s1^d1 (space2.rs:256-262); folded into the last operator
+    const double sc = op == 4 ? std::pow(s0, d0) * std::pow(s1, d1) : 1.0;
+    const char* dn[3] = {"S", "DS", "DDS"};
+    // interleaved complex arrays at 16-byte addresses are read and written by the row and FFT
+    // kernels themselves; other addresses, lengths and bases go through split planes
+    const bool pairs = cplx && ((uintptr_t)src & 15) == 0 && ((uintptr_t)dst & 15) == 0;
+    if (pairs && rows_ok() && op >= 2) {
+      const long rows = (long)nb * b0.m;
+      if (op == 3 && b1.k == CHEB) return src;
+      if (op == 3) composite_rows(st, src, dst, rows, true, b1.m, tdma_tab());
+      else ortho_rows(st, src, dst, rows, true, b1.m, b1.n, stencil_coef(), op == 4 ? d1 : 0, op == 4 ? d0 : 0, b0.m, sc);
+      return dst;
+    }
+    if (pairs && fft_supported(b0.n) && op < 2) {
+      if (op == 0) {
+        rfft_cols_interleaved(st, yop("FS", src, (long)nb * b0.n, W1.p), dst, b0.n, b1.m, nb);
+        return dst;
+      }
+      irfft_cols_interleaved(st, src, W1.p, b0.n, b1.m, nb);
+      return yop("BS", W1.p, (long)nb * b0.n, dst);
+    }
+    const bool in_c = cplx && op != 0, out_c = cplx && op != 1;
+    const double* x = src;
+    if (in_c) {
+      interleaved_to_split(st, src, W3.p, in_r / 2, in_c1, nb);
+      x = W3.p;
+    }
+    double* last = out_c ? W2.p : dst;  // where the second operator writes
+    const double* r;
+    if (op == 0) {  // forward: axis 1 then axis 0
+      r = xop("FS", yop("FS", x, (long)nb * b0.n, W1.p), b1.m, last, nb);
+    } else if (op == 1) {  // backward: axis 0 then axis 1
+      r = yop("BS", xop("BS", x, b1.m, W1.p, nb), (long)nb * b0.n, last);
+    } else if (op == 2) {
+      r = yop("S", xop("S", x, b1.m, W1.p, nb), (long)nb * r_ortho(), last);
+    } else if (op == 3) {
+      r = yop("FO", xop("FO", x, b1.n, W1.p, nb), (long)nb * r_spec(), last);
+    } else {
+      r = yop(dn[d1], xop(dn[d0], x, b1.m, W1.p, nb), (long)nb * r_ortho(), last);
+      if (sc != 1.0) {
+        const size_t e = (size_t)r_ortho() * b1.n;
+        if (b0.k == FO) {  // complex division by (sc, 0): (a sc) / sc^2 per component
+          for (int b = 0; b < nb; ++b) fourier_diff(st, r + b * e, last + b * e, b0.m, b1.n, b1.n, 0, sc);
+        } else {
+          ew_scale(st, last, r, 1.0 / sc, (long)e * nb);
+        }
+        r = last;
+      }
+    }
+    if (!out_c) return r;
+    split_to_interleaved(st, r, dst, out_r / 2, out_c1, nb);
+    return dst;
   }
 };
 
@@ -2183,9 +2253,10 @@ class SolverDev {
       solve_mixed(rhs, out, batch);
       return;
     }
-    ensure(W1, big() * batch);
-    ensure(W2, big() * batch);
-    if (cplx) {
+    if (!cplx) {
+      ensure(W1, big() * batch);
+      ensure(W2, big() * batch);
+    } else if (!complex_rows(rhs, out, batch)) {
       ensure(IN, in_size() * batch);
       ensure(OUT, out_size() * batch);
     }
@@ -2314,12 +2385,23 @@ class SolverDev {
     if (!cplx) w.in = nullptr;
     solve_ws(rhs, out, batch, w);
   }
+  // a Fourier axis 0: the row kernel reads and writes the interleaved arrays itself.  Arrays
+  // that overlap keep the split copies: a row's result may lie on another's right-hand side.
+  bool complex_rows(const double* rhs, const double* out, int batch) const {
+    return cplx && fdma_rows_lds_supported(s->m, s->pyb.mi) &&
+           !Space::overlap(rhs, in_size() * batch, out, out_size() * batch);
+  }
   void solve_ws(const double* rhs, double* out, int batch, const Work& w) {
     const int o1 = b1.ortho(), m1 = b1.m, m0 = b0.m, ro = rows_out();
     const size_t in_sz = in_size(), out_sz = out_size();
     const double* x = rhs;
+    if (complex_rows(rhs, out, batch)) {
+      fdma_rows_lds_complex(st, rhs, o1, s->pyb.mi, out, m1, s->m, s->nsets, s->pybp.p, s->diagp.p, batch);
+      HIPCHECK(hipStreamSynchronize(st));
+      return;
+    }
     if (cplx) {  // interleaved -> split planes, per right-hand side
-      for (int b = 0; b < batch; ++b) interleaved_to_split(st, rhs + 2 * (size_t)m0 * o1 * b, w.in + in_sz * b, m0, o1);
+      interleaved_to_split(st, rhs, w.in, m0, o1, batch);
       x = w.in;
     }
     double* y = out;
@@ -2339,7 +2421,7 @@ class SolverDev {
                         m1, (long)out_sz, batch, 1.0, 0.0);
     }
     if (cplx)
-      for (int b = 0; b < batch; ++b) split_to_interleaved(st, y + out_sz * b, out + 2 * (size_t)m0 * m1 * b, m0, m1);
+      split_to_interleaved(st, y, out, m0, m1, batch);
     HIPCHECK(hipStreamSynchronize(st));
   }
   // P_y matvec and the row solves: R [nrows, ldr] -> X [nrows, ld]

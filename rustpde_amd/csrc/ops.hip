@@ -521,24 +521,37 @@ void dot_and_norm(hipStream_t s, const double* a, const double* w, int n, const 
 }
 
 // --------------------------------------------------------------------- layout changes
-__global__ void i2s_kernel(const double* __restrict__ in, double* __restrict__ out, int m, int c) {
+// batch entries (blockIdx.y) are consecutive
+__global__ void i2s_kernel(const double* __restrict__ in, double* __restrict__ out, long n) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)m * c) return;
+  if (t >= n) return;
+  in += 2 * n * blockIdx.y;
+  out += 2 * n * blockIdx.y;
   out[t] = in[2 * t];
-  out[(long)m * c + t] = in[2 * t + 1];
+  out[n + t] = in[2 * t + 1];
 }
-__global__ void s2i_kernel(const double* __restrict__ in, double* __restrict__ out, int m, int c) {
+__global__ void s2i_kernel(const double* __restrict__ in, double* __restrict__ out, long n) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)m * c) return;
+  if (t >= n) return;
+  in += 2 * n * blockIdx.y;
+  out += 2 * n * blockIdx.y;
   out[2 * t] = in[t];
-  out[2 * t + 1] = in[(long)m * c + t];
+  out[2 * t + 1] = in[n + t];
 }
-void interleaved_to_split(hipStream_t s, const double* in, double* out, int m, int c) {
-  RBC_LAUNCH(i2s_kernel, dim3(blocks_for((long)m * c, 256)), dim3(256), 0, s, in, out, m, c);
+void interleaved_to_split(hipStream_t s, const double* in, double* out, int m, int c, int batch) {
+  const long n = (long)m * c;
+  for (int b = 0; b < batch; b += 65535) {
+    const int nb = batch - b < 65535 ? batch - b : 65535;
+    RBC_LAUNCH(i2s_kernel, dim3(blocks_for(n, 256), nb), dim3(256), 0, s, in + 2 * n * b, out + 2 * n * b, n);
+  }
   check_launch("interleaved_to_split");
 }
-void split_to_interleaved(hipStream_t s, const double* in, double* out, int m, int c) {
-  RBC_LAUNCH(s2i_kernel, dim3(blocks_for((long)m * c, 256)), dim3(256), 0, s, in, out, m, c);
+void split_to_interleaved(hipStream_t s, const double* in, double* out, int m, int c, int batch) {
+  const long n = (long)m * c;
+  for (int b = 0; b < batch; b += 65535) {
+    const int nb = batch - b < 65535 ? batch - b : 65535;
+    RBC_LAUNCH(s2i_kernel, dim3(blocks_for(n, 256), nb), dim3(256), 0, s, in + 2 * n * b, out + 2 * n * b, n);
+  }
   check_launch("split_to_interleaved");
 }
 

@@ -206,6 +206,9 @@ void rfft_cols(hipStream_t s, const double* X, double* Y, int n, int cols, int c
                long sy = 0, int nzc = -1);
 void irfft_cols(hipStream_t s, const double* X, double* Y, int n, int cols, int times, double sc, int batch = 1,
                 long sx = 0, long sy = 0);
+// `batch` consecutive arrays with interleaved complex spectra [n / 2 + 1, cols]
+void rfft_cols_interleaved(hipStream_t s, const double* X, double* Y, int n, int cols, int batch);
+void irfft_cols_interleaved(hipStream_t s, const double* X, double* Y, int n, int cols, int batch);
 // values (entries [0, nin): times 0, sc 1 -> Y0) and (i k)^times1 / sc1 (-> Y1) of the same
 // nin inputs in one launch of 2 nin batch entries
 void irfft_cols_pair(hipStream_t s, const double* X, double* Y0, double* Y1, int n, int cols, int times1, double sc1,
@@ -225,6 +228,10 @@ void fdma_rows_lds(hipStream_t s, const double* R, int ldr, int nr, double* X, i
 void fdma_rows_lds_multi(hipStream_t s, const double* R, int ldr, int nr, double* X, int ld, int nrows, int m,
                          int nsets, const double* const* bandps, const double* const* diagps, int batch, long sr,
                          long sx);
+
+// The same on `batch` consecutive interleaved complex arrays, set k solving row k of each.
+void fdma_rows_lds_complex(hipStream_t s, const double* R, int ldr, int nr, double* X, int ld, int m, int nsets,
+                           const double* bandp, const double* diagp, int batch);
 
 // from_ortho of every row as tdma_y, one wavefront per row with LDS staging and the
 // tables (diag, low2, off_{i-2}, 1 / den, w) in slice order: R [rows, m + 2] -> X [rows, m].
@@ -312,7 +319,19 @@ void cheb_y_diff(hipStream_t s, const double* in, int ldi, int mi, double* out, 
                  const double* coef, double inv_sc, double beta, int batch = 1, long si = 0, long so = 0);
 
 // complex layout conversion: interleaved (re, im) [m, c] <-> split planes [2m, c]
-void interleaved_to_split(hipStream_t s, const double* in, double* out, int m, int c);
-void split_to_interleaved(hipStream_t s, const double* in, double* out, int m, int c);
+// (`batch` consecutive arrays)
+void interleaved_to_split(hipStream_t s, const double* in, double* out, int m, int c, int batch = 1);
+void split_to_interleaved(hipStream_t s, const double* in, double* out, int m, int c, int batch = 1);
+
+// Row operators on `rows` consecutive rows, real, or with cplx interleaved complex, rows of up
+// to 2048 values (rowops.hip).
+// ortho_rows: mi composite coefficients (coef: stencil taps [2][n]; null: Chebyshev, mi = n)
+// -> n Chebyshev coefficients of the d1-th derivative; complex rows first times (i k)^d0,
+// k = row mod m0, and divided by sc last, real rows times sc last.
+// composite_rows: from_ortho, m + 2 values -> m (tabp: the tables of tdma_rows_lds).
+bool row_ops_supported(int n);
+void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int mi, int n, const double* coef,
+                int d1, int d0, int m0, double sc);
+void composite_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int m, const double* tabp);
 
 }  // namespace rbc

@@ -1,0 +1,236 @@
+// Row operators of Space2 along axis 1 (y): to_ortho and derivatives of a composite or plain
+// Chebyshev row, and from_ortho, on real rows or on interleaved complex rows, FP64.
+//
+// A block of four wavefronts holds two value rows: two real rows, or the real and imaginary
+// parts of one complex row (read and written as 16-byte pairs where both parts are at hand, so
+// that the caller's interleaved arrays need no separate split pass).  Each row is two parity
+// chains, one wavefront each (chains.hpp).  The operators are bound by memory: one read of the
+// input and one write of the output.  At fourier_r2c(512) x cheb_dirichlet(513), 8 fields, one
+// d/dx, d/dy, d2/dy2, to_ortho and from_ortho each take 2,842 us in all as split copies, dense
+// FMA products and merge copies per field, and 127 us as one launch per operator over the batch
+#include <hip/hip_runtime.h>
+
+#include <stdexcept>
+#include <string>
+
+#include "chains.hpp"
+#include "ops.hpp"
+#include "wave.hpp"
+
+namespace rbc {
+
+namespace {
+
+using chains::buf_len;
+using chains::pad;
+using chains::WAVE;
+constexpr int WAVES = 4;
+
+void check(const char* what) {
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// d1 derivatives (ortho.rs:107-125) of the to_ortho stencil (composite_stencil.rs:207-229) of
+// every row, (i k)^d0 (r2c.rs:88-99) applied first and the division by sc last (complex rows;
+// real rows multiply by sc, the caller's reciprocal).  in: mi values per row, out: n.
+template <int SLICE, bool CPLX>
+__global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* __restrict__ in, double* __restrict__ out,
+                                                                 long rows, int mi, int n, int per, int bl,
+                                                                 const double* __restrict__ coef, int d1, int d0, int m0,
+                                                                 double sc) {
+#pragma clang fp contract(off)
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const int slot = w >> 1, p = w & 1, tid = p * WAVE + lane;
+  double* buf = lds + slot * bl;
+  constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
+  const long row = CPLX ? (long)blockIdx.x : 2 * (long)blockIdx.x + slot;
+  const bool valid = row < rows;
+  const double kk = CPLX && d0 > 0 ? (double)(row % m0) : 0.0;
+  {
+    double v[MAXQ];
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * 2 * WAVE - 2;
+      v[q] = 0.0;
+      if (valid && i >= 0 && i < mi) {
+        if constexpr (CPLX) {
+          const double2 c = reinterpret_cast<const double2*>(in)[row * mi + i];
+          double a = c.x, b = c.y;
+          for (int t = 0; t < d0; ++t) {  // (a + i b) (0 + i k) as num-complex
+            const double na = a * 0.0 - b * kk, nb = a * kk + b * 0.0;
+            a = na;
+            b = nb;
+          }
+          v[q] = slot ? b : a;
+        } else {
+          v[q] = in[row * mi + i];
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int j = tid + q * 2 * WAVE;
+      if (j < n + 6) buf[pad(j)] = v[q];
+    }
+  }
+  __syncthreads();
+  if (coef) {  // stencil taps, zero where absent
+    double v[MAXQ];
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * 2 * WAVE;
+      v[q] = i < n ? buf[pad(i + 2)] * coef[i] + buf[pad(i)] * coef[n + i] : 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * 2 * WAVE;
+      if (i < n) buf[pad(i + 2)] = v[q];
+    }
+    __syncthreads();
+  }
+  for (int t = 0; t < d1; ++t) {
+    // d_i = w_i + d_{i+2}, w_i = 2 (i+1) c_{i+1}; d_0 = c_1 + d_2 / 2
+    const int len = p == 0 ? (n + 1) / 2 : n / 2;
+    const int t0 = lane * per, cnt = max(0, min(per, len - t0));
+    double v[SLICE], s = 0.0;
+#pragma unroll
+    for (int q = SLICE - 1; q >= 0; --q) {
+      const int i = p + 2 * (t0 + q);
+      v[q] = q < cnt ? (i == 0 ? buf[pad(3)] : 2.0 * (double)(i + 1) * buf[pad(i + 3)]) : 0.0;
+      if (i > 0) s = s + v[q];
+    }
+    double above;
+    wave::suffix_sum(s, lane, above);
+#pragma unroll
+    for (int q = SLICE - 1; q >= 0; --q) {
+      if (q < cnt) {
+        above = (p == 0 && t0 + q == 0) ? v[q] + above / 2.0 : v[q] + above;
+        v[q] = above;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < SLICE; ++q)
+      if (q < cnt) buf[pad(p + 2 * (t0 + q) + 2)] = v[q];
+    __syncthreads();
+  }
+  if constexpr (CPLX) {
+    const double ns = sc * sc + 0.0 * 0.0;
+    for (int i = threadIdx.x; i < n; i += WAVE * WAVES) {
+      double a = lds[pad(i + 2)], b = lds[bl + pad(i + 2)];
+      if (sc != 1.0) {  // num-complex division by (sc, 0)
+        const double na = (a * sc + b * 0.0) / ns, nb = (b * sc - a * 0.0) / ns;
+        a = na;
+        b = nb;
+      }
+      reinterpret_cast<double2*>(out)[row * n + i] = double2{a, b};
+    }
+  } else {
+    if (!valid) return;
+    for (int i = tid; i < n; i += 2 * WAVE) out[row * n + i] = sc != 1.0 ? buf[pad(i + 2)] * sc : buf[pad(i + 2)];
+  }
+}
+
+// from_ortho of every row (composite_stencil.rs:250-276, linalg.rs:14-57), the recurrences of
+// tdma_rows_lds.  in: m + 2 values per row, out: m.
+template <int SLICE, bool CPLX>
+__global__ __launch_bounds__(WAVE* WAVES) void composite_rows_kernel(const double* __restrict__ in,
+                                                                     double* __restrict__ out, long rows, int m, int per,
+                                                                     int bl, const double* __restrict__ tab) {
+#pragma clang fp contract(off)
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const int slot = w >> 1, p = w & 1, tid = p * WAVE + lane, n = m + 2;
+  double* buf = lds + slot * bl;
+  constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
+  const long row = CPLX ? (long)blockIdx.x : 2 * (long)blockIdx.x + slot;
+  const bool valid = row < rows;
+  {
+    double v[MAXQ];
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * 2 * WAVE - 2;
+      v[q] = valid && i >= 0 && i < n ? (CPLX ? in[2 * (row * n + i) + slot] : in[row * n + i]) : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int j = tid + q * 2 * WAVE;
+      if (j < n + 6) buf[pad(j)] = v[q];
+    }
+  }
+  __syncthreads();
+  const int len = p == 0 ? (m + 1) / 2 : m / 2;
+  const int t0 = lane * per, cnt = max(0, min(per, len - t0));
+  double v[SLICE], c0[SLICE], c1[SLICE];
+#define TB(a, q) tab[((size_t)((a) * 2 + p) * per + (q)) * WAVE + lane]
+#pragma unroll
+  for (int q = 0; q < SLICE; ++q) {
+    c0[q] = TB(0, q);
+    c1[q] = TB(1, q);
+  }
+#pragma unroll
+  for (int q = 0; q < SLICE; ++q) {
+    const int j = p + 2 * (t0 + q) + 2;
+    v[q] = q < cnt ? buf[pad(j)] * c0[q] + buf[pad(j + 2)] * c1[q] : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < SLICE; ++q) {
+    c0[q] = TB(2, q);
+    c1[q] = TB(3, q);
+  }
+  chains::tdma_forward(v, c0, c1, lane, t0, cnt);
+#pragma unroll
+  for (int q = 0; q < SLICE; ++q) c0[q] = TB(4, q);
+#undef TB
+  chains::tdma_backward(v, c0, lane, t0, cnt, p, m);
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < SLICE; ++q)
+    if (q < cnt) buf[pad(p + 2 * (t0 + q) + 2)] = v[q];
+  __syncthreads();
+  if constexpr (CPLX) {
+    for (int i = threadIdx.x; i < m; i += WAVE * WAVES)
+      reinterpret_cast<double2*>(out)[row * m + i] = double2{lds[pad(i + 2)], lds[bl + pad(i + 2)]};
+  } else {
+    if (!valid) return;
+    for (int i = tid; i < m; i += 2 * WAVE) out[row * m + i] = buf[pad(i + 2)];
+  }
+}
+
+}  // namespace
+
+// the slices of a row of n values: at most 16 entries per lane and chain
+bool row_ops_supported(int n) { return n >= 6 && fdma_rows_lds_per(n) <= 16; }
+
+#define RBC_ROW_OP(KERNEL, CPLX, per, ...)                                                                   \
+  do {                                                                                                       \
+    const dim3 grid((unsigned)((CPLX) ? rows : (rows + 1) / 2)), block(WAVE * WAVES);                         \
+    if ((per) <= 4) RBC_LAUNCH((KERNEL<4, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
+    else if ((per) <= 8) RBC_LAUNCH((KERNEL<8, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__); \
+    else RBC_LAUNCH((KERNEL<16, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);                \
+  } while (0)
+
+void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int mi, int n, const double* coef,
+                int d1, int d0, int m0, double sc) {
+  if (!row_ops_supported(n) || mi > n || (!coef && mi != n) || d1 < 0 || d0 < 0 || (d0 > 0 && m0 < 1))
+    throw std::invalid_argument("ortho_rows: bad arguments");
+  if (rows < 1 || rows > 0x3fffffff) throw std::invalid_argument("ortho_rows: bad rows");
+  const int per = fdma_rows_lds_per(n), bl = buf_len(n);
+  if (cplx) RBC_ROW_OP(ortho_rows_kernel, true, per, in, out, rows, mi, n, per, bl, coef, d1, d0, m0, sc);
+  else RBC_ROW_OP(ortho_rows_kernel, false, per, in, out, rows, mi, n, per, bl, coef, d1, 0, 1, sc);
+  check("ortho_rows");
+}
+
+void composite_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int m, const double* tabp) {
+  if (!row_ops_supported(m + 2) || !tdma_rows_lds_supported(m)) throw std::invalid_argument("composite_rows: bad length");
+  if (rows < 1 || rows > 0x3fffffff) throw std::invalid_argument("composite_rows: bad rows");
+  const int per = fdma_rows_lds_per(m), bl = buf_len(m + 2);
+  if (cplx) RBC_ROW_OP(composite_rows_kernel, true, per, in, out, rows, m, per, bl, tabp);
+  else RBC_ROW_OP(composite_rows_kernel, false, per, in, out, rows, m, per, bl, tabp);
+  check("composite_rows");
+}
+
+}  // namespace rbc

@@ -58,6 +58,20 @@ __global__ __launch_bounds__(WAVE* WAVES, SLICE <= 8 ? 4 : 2) void fdma_rows_lds
                               tb.diag[ti], bx);
 }
 
+// The rows of blockIdx.y-th interleaved complex array [nsets, nr] -> [nsets, m], one block per
+// set.  The caller's arrays are read and written once: at fourier_r2c(256) x cheb_neumann(257),
+// 4 right-hand sides, 19 us a call with the wait for it, against 59 us with a split and a merge
+// copy per right-hand side around the solve.
+template <int SLICE>
+__global__ __launch_bounds__(WAVE* WAVES, SLICE <= 8 ? 4 : 2) void fdma_rows_complex_kernel(
+    const double* __restrict__ R, int ldr, int nr, double* __restrict__ X, int ld, int m, int nsets, int per, int bl,
+    const double* __restrict__ bandp, const double* __restrict__ diagp) {
+  extern __shared__ double lds[];
+  R += 2 * (size_t)nsets * ldr * blockIdx.y;
+  X += 2 * (size_t)nsets * ld * blockIdx.y;
+  rowsolve::fdma_block<SLICE, true>(lds, R, ldr, nr, X, ld, 2 * nsets, m, nsets, per, bl, bandp, diagp, blockIdx.x);
+}
+
 // from_ortho of a composite basis per row (composite_stencil.rs:250-276, linalg.rs:14-57):
 // d_i = p_i diag_i + p_{i+2} low2_i, then g_i = (d_i - g_{i-2} off_{i-2}) / den_i and
 // x_i = g_i - x_{i+2} w_i (x_i = g_i for the last two i), arithmetic as tdma_y.  One
@@ -184,6 +198,26 @@ void fdma_rows_lds_multi(hipStream_t s, const double* R, int ldr, int nr, double
   }
   tb.shared = 0;
   launch_rows(s, R, ldr, nr, X, ld, nrows, m, nsets, tb, batch, sr, sx);
+}
+
+void fdma_rows_lds_complex(hipStream_t s, const double* R, int ldr, int nr, double* X, int ld, int m, int nsets,
+                           const double* bandp, const double* diagp, int batch) {
+  if (!fdma_rows_lds_supported(m, nr)) throw std::invalid_argument("fdma_rows_lds_complex: unsupported row length");
+  if (nsets < 1 || batch < 1 || !bandp || !diagp) throw std::invalid_argument("fdma_rows_lds_complex: bad arguments");
+  const int per = fdma_rows_lds_per(m), bl = buf_len(nr);
+  const size_t lds = (size_t)(WAVES / 2) * bl * sizeof(double);
+  for (int b = 0; b < batch; b += 65535) {
+    const dim3 grid(nsets, batch - b < 65535 ? batch - b : 65535), block(WAVE * WAVES);
+    const double* Rb = R + 2 * (size_t)nsets * ldr * b;
+    double* Xb = X + 2 * (size_t)nsets * ld * b;
+    if (per <= 4)
+      RBC_LAUNCH(fdma_rows_complex_kernel<4>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
+    else if (per <= 8)
+      RBC_LAUNCH(fdma_rows_complex_kernel<8>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
+    else
+      RBC_LAUNCH(fdma_rows_complex_kernel<16>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
+  }
+  check("fdma_rows_lds_complex");
 }
 
 bool tdma_rows_lds_supported(int m) {

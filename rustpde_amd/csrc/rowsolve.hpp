@@ -28,7 +28,9 @@ constexpr int WAVES = 4;  // wavefronts per block: two row slots of two parity c
 // per (row, parity chain), the two chains of a row sharing an LDS buffer of bl doubles at
 // lds + slot * bl.  With nrows = 2 nsets block bx holds the rows bx and bx + nsets of set
 // bx, else the rows 2 bx and 2 bx + 1.  Every thread of the block must call it.
-template <int SLICE>
+// CPLX: the block holds the real and the imaginary part of complex row bx of set bx, rows ldr
+// and ld interleaved values apart.
+template <int SLICE, bool CPLX = false>
 __device__ __forceinline__ void fdma_block(double* lds, const double* __restrict__ R, int ldr, int nr,
                                            double* __restrict__ X, int ld, int nrows, int m, int nsets, int per,
                                            int bl, const double* __restrict__ bandp,
@@ -40,7 +42,7 @@ __device__ __forceinline__ void fdma_block(double* lds, const double* __restrict
   // rows r and r + nsets share a diagonal set: one block per set when nrows = 2 nsets
   int r, set;
   bool valid;
-  if (nrows == 2 * nsets) {
+  if (CPLX || nrows == 2 * nsets) {
     set = bx;
     r = set + slot * nsets;
     valid = true;
@@ -51,7 +53,10 @@ __device__ __forceinline__ void fdma_block(double* lds, const double* __restrict
   }
   // (1) row -> LDS: element i at pad(i + 2); i in [-2, 0) and [nr, nr + 4) read as zero
   constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
-  chains::stage_row<MAXQ>(buf, R + (size_t)r * ldr, valid, nr, p * WAVE + lane, 2 * WAVE);
+  if constexpr (CPLX)
+    chains::stage_row<MAXQ, 2>(buf, R + 2 * (size_t)bx * ldr + slot, valid, nr, p * WAVE + lane, 2 * WAVE);
+  else
+    chains::stage_row<MAXQ>(buf, R + (size_t)r * ldr, valid, nr, p * WAVE + lane, 2 * WAVE);
   __syncthreads();
   const int len = p == 0 ? (m + 1) / 2 : m / 2;
   const int t0 = lane * per;
@@ -108,7 +113,10 @@ __device__ __forceinline__ void fdma_block(double* lds, const double* __restrict
   for (int q = 0; q < SLICE; ++q)
     if (q < cnt) buf[pad(p + 2 * (t0 + q) + 2)] = v[q];
   __syncthreads();
-  chains::unstage_row<MAXQ>(buf, X + (size_t)r * ld, valid, m, p * WAVE + lane, 2 * WAVE, false);
+  if constexpr (CPLX)
+    chains::unstage_row<MAXQ, 2>(buf, X + 2 * (size_t)bx * ld + slot, valid, m, p * WAVE + lane, 2 * WAVE, false);
+  else
+    chains::unstage_row<MAXQ>(buf, X + (size_t)r * ld, valid, m, p * WAVE + lane, 2 * WAVE, false);
 }
 
 }  // namespace rowsolve
