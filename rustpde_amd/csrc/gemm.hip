@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(int M, int N, int K, con
                                                         int ldc, long sC, double alpha, double beta,
                                                         const V* __restrict__ U, int ldu, long sU, int amod, int bmod,
                                                         int umod, const V* __restrict__ A2, const TB* __restrict__ B2,
-                                                        int split, int zero00) {
+                                                        int split) {
   using MF = Mfma<V>;
   typedef typename MF::v4 v4;
   constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
@@ -168,7 +168,6 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(int M, int N, int K, con
           V v = va * acc[i][j][r];
           if (U) v = v * uv[j][r];
           if (beta != 0.0) v = v + vb * cv[j][r];
-          if (zero00 && gm == 0 && gn == 0) v = (V)0;
           C[(size_t)gm * ldc + gn] = (TC)v;
         }
       }
@@ -187,11 +186,11 @@ void launch_tile(hipStream_t s, bool timed, int M, int N, int K, const V* A, int
   if (timed) {
     RBC_LAUNCH((gemm_mfma_kernel<BM, BN, BK, V, TB, TC>), grid, dim3(256), 0, s, M, N, K, A, lda, sA, B, ldb, sB, C,
                ldc, sC, alpha, beta, U, ldu, sU, bm.a, bm.b, bm.u, static_cast<const V*>(bm.a2),
-               static_cast<const TB*>(bm.b2), bm.split, bm.zero00);
+               static_cast<const TB*>(bm.b2), bm.split);
   } else {
     hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, BK, V, TB, TC>), grid, dim3(256), 0, s, M, N, K, A, lda, sA, B, ldb,
                        sB, C, ldc, sC, alpha, beta, U, ldu, sU, bm.a, bm.b, bm.u, static_cast<const V*>(bm.a2),
-                       static_cast<const TB*>(bm.b2), bm.split, bm.zero00);
+                       static_cast<const TB*>(bm.b2), bm.split);
   }
 }
 

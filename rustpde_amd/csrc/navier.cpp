@@ -239,8 +239,128 @@ static LMat host_y(const Basis& b, const std::string& name, const LMat& in) {
   return in * build_axis_op(b, name, 1.0L).t();
 }
 
+// A dense left operator as its parity classes on the device (XOp): the kind follows from the
+// matrix, entries of the other class being exact zeros (blocks) or mirrored values equal to
+// rounding (folds; the operators of the points are built from cosines of mirrored angles).
+struct PackedOp {
+  DBuf buf;
+  XOp op;
+  size_t stride() const { return buf.n; }
+  void pack(const std::vector<double>& m, int rows, int cols) {
+    auto at = [&](int i, int j) { return m[(size_t)i * cols + j]; };
+    op = XOp{};
+    op.rows = rows;
+    op.cols = cols;
+    bool same = true, flip = true;  // nonzero only where i + j is even / odd
+    for (int i = 0; i < rows && (same || flip); ++i)
+      for (int j = 0; j < cols; ++j)
+        if (at(i, j) != 0.0) (((i + j) & 1) ? same : flip) = false;
+    // mirror signs: column j (fold out) or row i (fold in) symmetric or antisymmetric
+    auto mirrored = [&](bool out, int parity) {  // index of parity `parity` symmetric, else antisymmetric
+      const int nl = out ? cols : rows, nm = out ? rows : cols;
+      for (int l = 0; l < nl; ++l) {
+        const double sg = (l & 1) == parity ? 1.0 : -1.0;
+        double mx = 0.0, d = 0.0;
+        for (int k = 0; k < nm; ++k) {
+          const double a = out ? at(k, l) : at(l, k), b = out ? at(nm - 1 - k, l) : at(l, nm - 1 - k);
+          mx = std::max(mx, std::fabs(a));
+          d = std::max(d, std::fabs(a - sg * b));
+        }
+        if (!(d <= 2e-15 * mx)) return false;
+      }
+      return true;
+    };
+    auto half = [](int n, int c) { return (n + 1 - c) / 2; };  // indices 2k + c below n
+    std::vector<double> cls[2];
+    int ncls = 2;
+    auto fill = [&](int c, int M, int K, auto get) {  // M x K entries; the packing follows
+      op.M[c] = M;
+      op.K[c] = K;
+      cls[c].resize((size_t)M * K);
+      op.mnz[c] = 0;
+      for (int i = 0; i < M; ++i)
+        for (int k = 0; k < K; ++k) {
+          const double v = get(i, k);
+          cls[c][(size_t)i * K + k] = v;
+          if (v != 0.0) op.mnz[c] = i + 1;
+        }
+    };
+    int pe = 0;
+    if (rows >= 4 && cols >= 4 && (same || flip)) {
+      const int f = same ? 0 : 1;
+      op.kind = XOP_BLOCKS;
+      for (int c = 0; c < 2; ++c) {
+        op.r0[c] = c ^ f;
+        op.c0[c] = c;
+        fill(c, half(rows, c), half(cols, c ^ f), [&](int i, int k) { return at(2 * i + c, 2 * k + (c ^ f)); });
+      }
+      op.rstep = op.cstep = 2;
+    } else if (rows >= 4 && cols >= 4 && (mirrored(true, 0) || mirrored(true, pe = 1))) {
+      op.kind = XOP_FOLD_OUT;  // class 0: the symmetric columns, class 1: the antisymmetric ones
+      const int h = (rows + 1) / 2;
+      for (int c = 0; c < 2; ++c) {
+        op.r0[c] = c ^ pe;
+        fill(c, h, half(cols, c ^ pe), [&](int i, int k) {
+          return c == 1 && 2 * i + 1 == rows ? 0.0 : at(i, 2 * k + (c ^ pe));  // odd at the middle: zero
+        });
+      }
+      op.rstep = 2;
+    } else if (rows >= 4 && cols >= 4 && mirrored(false, 0)) {
+      op.kind = XOP_FOLD_IN;  // even rows take sums of mirrored inputs, odd rows differences
+      const int h = (cols + 1) / 2;
+      for (int c = 0; c < 2; ++c) {
+        op.c0[c] = c;
+        fill(c, half(rows, c), h, [&](int i, int k) {
+          const double v = at(2 * i + c, k);
+          return 2 * k + 1 == cols ? (c ? 0.0 : 0.5 * v) : v;  // the middle input meets itself
+        });
+      }
+      op.cstep = 2;
+    } else {
+      ncls = 1;
+      fill(0, rows, cols, [&](int i, int k) { return at(i, k); });
+    }
+    op.groups = xop_groups(std::max(op.K[0], op.K[1]));
+    const size_t size = (size_t)((op.M[0] + 63) / 64 * 64) * op.groups * 8;
+    std::vector<double> all(size * ncls, 0.0);
+    for (int c = 0; c < ncls; ++c)
+      for (int i = 0; i < op.M[c]; ++i)
+        for (int k = 0; k < op.K[c]; ++k) all[c * size + xop_index(i, k, op.groups)] = cls[c][(size_t)i * op.K[c] + k];
+    buf.alloc(all.size());
+    buf.upload(all);
+    op.a[0] = buf.p;
+    op.a[1] = ncls == 2 ? buf.p + size : nullptr;
+  }
+};
+// entries z of C_z = op B_z, arrays [cols, N] -> [rows, N] contiguous, e_in / e_out apart
+static XGemm xgemm_of(const PackedOp& p, const double* B, double* C, int N, int entries, long sB, long sC) {
+  XGemm g;
+  g.op = p.op;
+  g.a2[0] = p.op.a[0];
+  g.a2[1] = p.op.a[1];
+  g.B = B;
+  g.C = C;
+  g.N = g.ldb = g.ldc = N;
+  g.entries = entries;
+  g.sB = sB;
+  g.sC = sC;
+  return g;
+}
+
 class OpCache {
  public:
+  // the operator as a left operator's parity classes
+  const PackedOp& packed(const Basis& b, const std::string& name) {
+    std::string key = std::to_string((int)b.k) + ":" + std::to_string(b.n) + ":" + name;
+    auto it = packed_.find(key);
+    if (it != packed_.end()) return *it->second;
+    LMat m = build_axis_op(b, name, (ld)scale_);
+    auto op = std::make_unique<PackedOp>();
+    op->pack(m.to_double(), m.r, m.c);
+    const PackedOp& ref = *op;
+    packed_[key] = std::move(op);
+    return ref;
+  }
   OpCache(bool transposed, double scale) : transposed_(transposed), scale_(scale) {}
   const DOp& get(const Basis& b, const std::string& name) {
     std::string key = std::to_string((int)b.k) + ":" + std::to_string(b.n) + ":" + name;
@@ -261,6 +381,7 @@ class OpCache {
   bool transposed_;
   double scale_;
   std::map<std::string, std::unique_ptr<DOp>> ops_;
+  std::map<std::string, std::unique_ptr<PackedOp>> packed_;
 };
 
 static void upload_op(DOp& op, const LMat& m) {
@@ -284,6 +405,7 @@ struct Solver {
   std::vector<double> px;             // P_x (m x n) in double, for composing fwd * P_x
   std::vector<double> ax, cx;         // A_x, C_x (m x m) when axis 0 is not diagonal
   DOp pf, pb, py;
+  PackedOp hxp, pfp, pbp;  // hx, pf and pb as parity classes
   DBand pyb;  // P_y as a banded matvec
   std::vector<double> pyb_taps;  // its taps on the host, [4][m]
   DBuf low, dia, up1, up2;
@@ -332,8 +454,11 @@ struct Solver {
       for (size_t i = 0; i < F.a.size(); ++i) F.a[i] = fwd[i];
       for (size_t i = 0; i < P.a.size(); ++i) P.a[i] = px[i];
       for (size_t i = 0; i < Q.a.size(); ++i) Q.a[i] = bwd[i];
-      upload_op(pf, F * P);
+      const LMat FP = F * P;
+      upload_op(pf, FP);
       upload_op(pb, Q);
+      pfp.pack(FP.to_double(), FP.r, FP.c);
+      pbp.pack(Q.to_double(), Q.r, Q.c);
     }
   }
 };
@@ -351,8 +476,12 @@ static std::unique_ptr<Solver> make_solver(SKind kind, const Basis& b0, const Ba
       LMat M(m, m);
       for (size_t i = 0; i < M.a.size(); ++i) M.a[i] = (ld)((double)g.a.a[i] - (double)g.b.a[i] * c[ax]);
       LMat H = inverse(M) * g.p;  // (m x n)
-      if (ax == 0) upload_op(s->hx, H);
-      else upload_op(s->hy, H.t());
+      if (ax == 0) {
+        upload_op(s->hx, H);
+        s->hxp.pack(H.to_double(), H.r, H.c);
+      } else {
+        upload_op(s->hy, H.t());
+      }
     }
     return s;
   }
@@ -503,8 +632,9 @@ class Navier {
   int nb = 1;
   long bs = 0;
   DBuf NUARR;
-  DBuf ADIH[3][2];
-  long adi_s[3][2] = {};
+  DBuf ADIP[3];  // x: parity classes, solver[w]->hxp.stride() apart
+  DBuf ADIH[3];  // y, adi_s apart
+  long adi_s[3] = {};
   // Field batching (confined step): inside a FieldPair scope fb = 2 (or 3) and every launch
   // covers ux and uy (and temp) of every instance, batch entry z = f nb + b (field f,
   // instance b).  Each work buffer of the velocity part then holds partner slots pair_off()
@@ -632,19 +762,6 @@ class Navier {
     const int nz = nbt();
     if ((A2 || B2) && fb != 3) throw std::logic_error("GEMM: second operators need fb = 3");
     timer.begin(st, 0, 2.0 * M * N * K * nz);
-    if (gemm_zero00 && !A2 && !B2 && (use_mfma || nz > 1)) {  // the product and the pin of C(0, 0)
-      const long d = dstr();
-      BatchMod bm;
-      bm.a = sA > 0 ? nb : 0;
-      bm.b = sB > 0 ? nb : 0;
-      bm.u = nb;
-      bm.zero00 = 1;
-      gemm_mfma_batched(st, M, N, K, A, lda, sA == DATA ? d : sA, B, ldb, sB == DATA ? d : sB, C, ldc, d, nz, 1.0,
-                        beta, U, ldu, U ? bs : 0, bm);
-      timer.end(st);
-      return;
-    }
-    if (gemm_zero00) throw std::logic_error("GEMM: pinned output needs the matrix-core path");
     if (nz > 1) {
       const long d = dstr();
       BatchMod bm;
@@ -924,15 +1041,53 @@ class Navier {
       BANDX(stencil_band(b), in, out, cols, 0.0);
       return out;
     }
+    if (xg_ok()) {
+      const XGemm g = xg(X.packed(b, name), in, cols, out);
+      XGEMM(&g, 1);
+      return out;
+    }
     const DOp& op = X.get(b, name);
     GEMM(op.rows, cols, op.cols, op.b.p, op.cols, in, cols, out, cols, 0.0, nullptr, 0, 0, DATA);
     return out;
   }
-  void xmat(const DOp& op, const double* in, int cols, double* out, const double* per_inst = nullptr,
-            long sop = 0) {  // per_inst: the group's operators, sop apart
-    GEMM(op.rows, cols, op.cols, per_inst ? per_inst : op.b.p, op.cols, in, cols, out, cols, 0.0, nullptr, 0,
-         per_inst ? sop : 0, DATA);
+  void xmat(const DOp& op, const double* in, int cols, double* out) {
+    GEMM(op.rows, cols, op.cols, op.b.p, op.cols, in, cols, out, cols, 0.0, nullptr, 0, 0, DATA);
   }
+  // temp's operator for the entries from 2 nb on of a triple's product
+  void two_ops(XGemm& g, const PackedOp& t) {
+    for (int c = 0; c < 2; ++c) {
+      g.a2[c] = t.op.a[c];
+      g.op.mnz[c] = std::max(g.op.mnz[c], t.op.mnz[c]);
+    }
+    g.split = 2 * nb;
+  }
+  // the group's per-instance ADI x operators of field `which` (and of field `which2` for the
+  // entries from 2 nb on) in place of the leader's
+  void group_adi(XGemm& g, int which, int which2) {
+    const XOp& p = solver[which]->hxp.op;
+    for (int c = 0; c < 2; ++c) {
+      g.op.mnz[c] = g.op.M[c];
+      g.op.a[c] = p.a[c] ? ADIP[which].p + (p.a[c] - p.a[0]) : nullptr;
+      if (which2 >= 0) g.a2[c] = p.a[c] ? ADIP[which2].p + (p.a[c] - p.a[0]) : nullptr;
+    }
+    g.sA = (long)solver[which]->hxp.stride();
+    g.amod = nb;
+  }
+  // one left operator's product on every entry of the current field batch, its parity classes
+  // on the matrix cores
+  XGemm xg(const PackedOp& p, const double* in, int cols, double* out) {
+    return xgemm_of(p, in, out, cols, nbt(), dstr(), dstr());
+  }
+  void XGEMM(const XGemm* g, int ng) {
+    double w = 0.0;
+    for (int i = 0; i < ng; ++i)
+      for (int c = 0; c < 2; ++c) w += 2.0 * g[i].op.M[c] * g[i].op.K[c] * (double)g[i].N * g[i].entries;
+    timer.begin(st, 0, w);
+    xgemm(st, g, ng);
+    timer.end(st);
+  }
+  // matrix cores in use for x operators (RBC_OPT_MFMA 0 keeps the FMA product of one instance)
+  bool xg_ok() const { return use_mfma || nb > 1; }
   // y (axis 1): in [rows, cin] -> out [rows, cout]; out = (in Y^T) .* U + beta out
   const double* yop(const Basis& b, const std::string& name, const double* in, int rows, double* out,
                     const double* U = nullptr, double beta = 0.0) {
@@ -1048,13 +1203,27 @@ class Navier {
     if (s2.kind != ADI || bx_t.m != bx_u.m || bx_t.n != bx_u.n) return false;
     if (s0.hx.rows != s2.hx.rows || s0.hx.cols != s2.hx.cols || s0.hy.rows != s2.hy.rows || s0.hy.cols != s2.hy.cols)
       return false;
-    return nb == 1 || (adi_s[0][0] == adi_s[2][0] && adi_s[0][1] == adi_s[2][1]);
+    return xg_ok() && same_classes(s0.hxp.op, s2.hxp.op) && (nb == 1 || adi_s[0] == adi_s[2]);
   }
-  // x-transform `name` of the triple [m_x, cols] -> [rows, cols] (FP64 GEMM, fb = 3)
+  // two operators whose classes one launch can take as first and second operators
+  static bool same_classes(const XOp& a, const XOp& b) {
+    if (a.kind != b.kind || a.rows != b.rows || a.cols != b.cols) return false;
+    for (int c = 0; c < 2; ++c)
+      if (a.M[c] != b.M[c] || a.K[c] != b.K[c] || a.r0[c] != b.r0[c] || a.c0[c] != b.c0[c])
+        return false;
+    return true;
+  }
+  bool triple_ops_ok() {
+    for (const char* name : {"BS", "BDS"})
+      if (!same_classes(X.packed(bx_u, name).op, X.packed(bx_t, name).op)) return false;
+    return true;
+  }
+  // x-transform `name` of the triple [m_x, cols] -> [rows, cols] (fb = 3)
   void xop3(const std::string& name, const double* in, int cols, double* out) {
-    const DOp &ou = X.get(bx_u, name), &ot = X.get(bx_t, name);
-    if (ou.rows != ot.rows || ou.cols != ot.cols) throw std::logic_error("xop3: operator shapes differ");
-    GEMM(ou.rows, cols, ou.cols, ou.b.p, ou.cols, in, cols, out, cols, 0.0, nullptr, 0, 0, DATA, ot.b.p);
+    const PackedOp &ou = X.packed(bx_u, name), &ot = X.packed(bx_t, name);
+    XGemm g = xg(ou, in, cols, out);
+    two_ops(g, ot);
+    XGEMM(&g, 1);
   }
   void xop3_32(const std::string& name, const double* in, int cols, float* out) {
     const DOp &ou = X.get(bx_u, name), &ot = X.get(bx_t, name);
@@ -1098,14 +1267,15 @@ class Navier {
     FieldPair ft(*this, 3);
     const Solver &s0 = *solver[0], &s2 = *solver[2];
     const bool grp = nb > 1;
-    const double* ax = grp ? ADIH[0][0].p : s0.hx.b.p;
-    const double* ax2 = grp ? ADIH[2][0].p : s2.hx.b.p;
-    const double* ay = grp ? ADIH[0][1].p : s0.hy.b.p;
-    const double* ay2 = grp ? ADIH[2][1].p : s2.hy.b.p;
+    const double* ay = grp ? ADIH[0].p : s0.hy.b.p;
+    const double* ay2 = grp ? ADIH[2].p : s2.hy.b.p;
     const DOp &hx = s0.hx, &hy = s0.hy;
-    GEMM(hx.rows, ny, hx.cols, ax, hx.cols, RHS.p, ny, W1.p, ny, 0.0, nullptr, 0, grp ? adi_s[0][0] : 0, DATA, ax2);
+    XGemm g = xg(s0.hxp, RHS.p, ny, W1.p);
+    two_ops(g, s2.hxp);
+    if (grp) group_adi(g, 0, 2);
+    XGEMM(&g, 1);
     GEMM(hx.rows, hy.cols, hy.rows, W1.p, hy.rows, ay, hy.cols, UX.p, hy.cols, 0.0, nullptr, 0, DATA,
-         grp ? adi_s[0][1] : 0, nullptr, ay2);
+         grp ? adi_s[0] : 0, nullptr, ay2);
   }
   // one confined step with the field triple (navier.rs:737-765; temp's solve moves ahead of
   // the projection, which does not read temp)
@@ -1220,31 +1390,39 @@ class Navier {
   }
 
   // ------------------------------------------------------------------------ step
-  bool gemm_zero00 = false;  // the next GEMM pins C(0, 0) of every entry to 0
-  // zero00: out(0, 0) = 0 of every entry after a confined Poisson solve (formed in its last GEMM)
+  // zero00: out(0, 0) = 0 of every entry after a confined Poisson solve (formed in its last
+  // product, on the matrix cores)
   void solve(int which, double* rhs, double* out, bool zero00 = false) {
     Solver& s = *solver[which];
     const int my = s.by.m;
     if (s.kind == ADI) {
       const bool grp = nb > 1 && which < 3;  // the group's per-instance operators
-      xmat(s.hx, rhs, ny, W1.p, grp ? ADIH[which][0].p : nullptr, adi_s[which][0]);         // [mx, ny]
-      ymat(s.hy, W1.p, s.hx.rows, out, grp ? ADIH[which][1].p : nullptr, adi_s[which][1]);  // [mx, my]
+      if (xg_ok()) {  // [mx, ny]
+        XGemm g = xg(s.hxp, rhs, ny, W1.p);
+        if (grp) group_adi(g, which, -1);
+        XGEMM(&g, 1);
+      } else {
+        xmat(s.hx, rhs, ny, W1.p);
+      }
+      ymat(s.hy, W1.p, s.hx.rows, out, grp ? ADIH[which].p : nullptr, adi_s[which]);  // [mx, my]
       return;
     }
     if (!s.has_fb) {  // Fourier x: P_y then the per-wavenumber row systems
       ROWSF(rhs, ny, out, my, 2 * s.bx.m, s);
       return;
     }
+    if (xg_ok()) {  // fwd * P_x : [m0, ny], the row systems, bwd : [m0, my]
+      const XGemm f = xg(s.pfp, rhs, ny, W1.p);
+      XGEMM(&f, 1);
+      ROWSF(W1.p, ny, W2.p, my, s.pf.rows, s);
+      XGemm b = xg(s.pbp, W2.p, my, out);
+      b.zero00 = zero00 ? 1 : 0;
+      XGEMM(&b, 1);
+      return;
+    }
     xmat(s.pf, rhs, ny, W1.p);              // fwd * P_x : [m0, ny]
     ROWSF(W1.p, ny, W2.p, my, s.pf.rows, s);  // P_y and the row systems : [m0, my]
-    gemm_zero00 = zero00;
-    try {
-      xmat(s.pb, W2.p, my, out);  // bwd : [m0, my]
-    } catch (...) {
-      gemm_zero00 = false;
-      throw;
-    }
-    gemm_zero00 = false;
+    xmat(s.pb, W2.p, my, out);  // bwd : [m0, my]
   }
 
   // convective term of q with x-basis bxq (y basis cheb_dirichlet), into CONV (physical)
@@ -1736,7 +1914,7 @@ class Navier {
       return;
     }
     gpres_valid = false;
-    if (!periodic && triple_ok() && stencil2d_ok(bx_t, by_u) && stencil2d_ok(bx_u, by_u)) {
+    if (!periodic && triple_ok() && triple_ops_ok() && stencil2d_ok(bx_t, by_u) && stencil2d_ok(bx_u, by_u)) {
       update_triple();
       return;
     }
@@ -2080,9 +2258,9 @@ class Space {
     } else if (b0.k == CHEB && (op_name == "S" || op_name == "FO")) {
       return in;
     }
-    const DOp& op = X.get(b0, op_name);
-    gemm_mfma_batched(st, op.rows, cols, op.cols, op.b.p, op.cols, 0, in, cols, (long)op.cols * cols, out, cols,
-                      (long)op.rows * cols, nb, 1.0, 0.0);
+    const PackedOp& op = X.packed(b0, op_name);
+    const XGemm g = xgemm_of(op, in, out, cols, nb, (long)op.op.cols * cols, (long)op.op.rows * cols);
+    xgemm(st, &g, 1);
     return out;
   }
   // y-operator on `rows` consecutive real rows
@@ -2408,17 +2586,17 @@ class SolverDev {
     if (cplx) y = w.out;
     Solver& sv = *s;
     if (sv.kind == ADI) {
-      gemm_mfma_batched(st, sv.hx.rows, o1, sv.hx.cols, sv.hx.b.p, sv.hx.cols, 0, x, o1, (long)in_sz, w.w1, o1,
-                        (long)sv.hx.rows * o1, batch, 1.0, 0.0);
+      const XGemm g = xgemm_of(sv.hxp, x, w.w1, o1, batch, (long)in_sz, (long)sv.hx.rows * o1);
+      xgemm(st, &g, 1);
       gemm_mfma(st, batch * sv.hx.rows, m1, sv.hy.rows, w.w1, sv.hy.rows, sv.hy.b.p, sv.hy.cols, y, m1, 1.0, 0.0);
     } else if (!sv.has_fb) {
       rows_launch(x, o1, y, m1, batch * ro, sv);
     } else {
-      gemm_mfma_batched(st, sv.pf.rows, o1, sv.pf.cols, sv.pf.b.p, sv.pf.cols, 0, x, o1, (long)in_sz, w.w1, o1,
-                        (long)sv.pf.rows * o1, batch, 1.0, 0.0);
+      const XGemm f = xgemm_of(sv.pfp, x, w.w1, o1, batch, (long)in_sz, (long)sv.pf.rows * o1);
+      xgemm(st, &f, 1);
       rows_launch(w.w1, o1, w.w2, m1, batch * sv.pf.rows, sv);
-      gemm_mfma_batched(st, sv.pb.rows, m1, sv.pb.cols, sv.pb.b.p, sv.pb.cols, 0, w.w2, m1, (long)sv.pf.rows * m1, y,
-                        m1, (long)out_sz, batch, 1.0, 0.0);
+      const XGemm b = xgemm_of(sv.pbp, w.w2, y, m1, batch, (long)sv.pf.rows * m1, (long)out_sz);
+      xgemm(st, &b, 1);
     }
     if (cplx)
       split_to_interleaved(st, y, out, m0, m1, batch);
@@ -2535,15 +2713,16 @@ class Ensemble {
         for (int b = 0; b < B; ++b) nus[b] = g->navs[b]->nu;
         L.NUARR.upload(nus);
         for (int w = 0; w < 3; ++w) {  // ADI operators of ux, uy, temp per instance
-          for (int ax = 0; ax < 2; ++ax) {
-            const DOp& op0 = ax == 0 ? L.solver[w]->hx : L.solver[w]->hy;
-            const size_t sz = (size_t)op0.rows * op0.cols;
-            L.ADIH[w][ax].alloc(sz * B);
-            L.adi_s[w][ax] = (long)sz;
-            for (int b = 0; b < B; ++b) {
-              const DOp& op = ax == 0 ? g->navs[b]->solver[w]->hx : g->navs[b]->solver[w]->hy;
-              HIPCHECK(hipMemcpy(L.ADIH[w][ax].p + b * sz, op.b.p, sz * sizeof(double), hipMemcpyDeviceToDevice));
-            }
+          const size_t sp = L.solver[w]->hxp.stride(), sy = (size_t)L.solver[w]->hy.rows * L.solver[w]->hy.cols;
+          L.ADIP[w].alloc(sp * B);
+          L.ADIH[w].alloc(sy * B);
+          L.adi_s[w] = (long)sy;
+          for (int b = 0; b < B; ++b) {
+            const Solver& sb = *g->navs[b]->solver[w];
+            if (!Navier::same_classes(sb.hxp.op, L.solver[w]->hxp.op))
+              throw std::logic_error("ensemble: implicit operators of one group differ in their parity classes");
+            HIPCHECK(hipMemcpy(L.ADIP[w].p + b * sp, sb.hxp.buf.p, sp * sizeof(double), hipMemcpyDeviceToDevice));
+            HIPCHECK(hipMemcpy(L.ADIH[w].p + b * sy, sb.hy.b.p, sy * sizeof(double), hipMemcpyDeviceToDevice));
           }
         }
       }

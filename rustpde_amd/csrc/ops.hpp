@@ -50,13 +50,11 @@ struct GemmNoTune {
 // Batch-index moduli of A, B, U (0: none): entry z reads A + sA (z % a) etc.
 // Entries z >= split read A from a2 and B from b2 instead (when given; same types, strides
 // and moduli): two operators in one launch.
-// zero00: every entry's C(0, 0) is set to 0 after the product (the pseudo-pressure pin).
 struct BatchMod {
   int a = 0, b = 0, u = 0;
   int split = 0;
   const void* a2 = nullptr;
   const void* b2 = nullptr;
-  int zero00 = 0;
 };
 // Batched: operand b of batch index z starts at A + z sA, B + z sB, C + z sC, U + z sU
 // (with the moduli and the operator switch of bm applied to A, B, U).
@@ -68,6 +66,45 @@ void gemm_mfma_batched(hipStream_t s, int M, int N, int K, const double* A, int 
 void gemm_mfma_f32_batched(hipStream_t s, int M, int N, int K, const float* A, int lda, long sA, const void* B,
                            bool b_f64, int ldb, long sB, void* C, bool c_f64, int ldc, long sC, int batch, double alpha,
                            double beta, const float* U, int ldu, long sU, BatchMod bm = BatchMod{});
+
+// Dense left operators split into their two parity classes (xgemm.hip).  Class c is a matrix of
+// M[c] x K[c] entries (M[0] >= M[1]), entry (m, k) at a[c][xop_index(m, k, groups)], packed with
+// zeros to whole 64 rows and xop_groups(max K) groups of 8 k values; rows m >= mnz[c] are zero and
+// not multiplied.
+enum { XOP_DENSE, XOP_BLOCKS, XOP_FOLD_IN, XOP_FOLD_OUT };
+struct XOp {
+  const double* a[2] = {};
+  int M[2] = {}, K[2] = {}, mnz[2] = {};
+  int groups = 0;
+  int kind = XOP_DENSE;
+  int r0[2] = {}, rstep = 1;  // input row of k: r0[c] + rstep k (fold in: also cols - 1 - that)
+  int c0[2] = {}, cstep = 1;  // output row of m: c0[c] + cstep m (fold out: m and rows - 1 - m)
+  int rows = 0, cols = 0;     // of the whole operator
+};
+int xop_groups(int K);
+// the order in which a wavefront's lanes read 16 rows x 8 k values: lane 16 (k / 2 mod 4) + m mod 16
+// holds k and k + 1
+inline size_t xop_index(int m, int k, int groups) {
+  return ((((size_t)(m / 16) * groups + k / 8) * 64) + (size_t)((k / 2) % 4) * 16 + m % 16) * 2 + k % 2;
+}
+// C_z = op B_z for `entries` entries z: B at z sB (row stride ldb), C at z sC.  Entry z takes the
+// operator (z mod amod) sA further on (amod > 0: one per instance), entries >= split (split > 0)
+// the classes a2 instead.  zero00: C(0, 0) = 0 in every entry.
+struct XGemm {
+  XOp op;
+  const double* a2[2] = {};
+  int split = 0, amod = 0;
+  long sA = 0;
+  const double* B = nullptr;
+  int ldb = 0;
+  long sB = 0;
+  double* C = nullptr;
+  int ldc = 0;
+  long sC = 0;
+  int N = 0, entries = 1, zero00 = 0;
+};
+constexpr int XGEMM_GROUPS = 3;  // independent products of one launch, operators of one kind
+void xgemm(hipStream_t s, const XGemm* groups, int ng);
 
 // Banded 4-diagonal solves (offsets -2, 0, 2, 4; pre-swept as fdma.rs:73-82) of every
 // row r of X[nrows, m] with diagonal set (r % nsets); diag arrays are [nsets, m].

@@ -490,8 +490,8 @@ bool schur(Schur& s) {
 
 }  // namespace
 
-bool eig_real(const std::vector<double>& a, int n, std::vector<double>& lam, std::vector<double>& q,
-              std::vector<double>& qi, std::string& msg) {
+static bool eig_whole(const std::vector<double>& a, int n, std::vector<double>& lam, std::vector<double>& q,
+                      std::vector<double>& qi, std::string& msg) {
   // isolated columns (zero off-diagonal): exact eigenvectors e_j (LAPACK dgebal permutation)
   std::vector<int> iso(n, 0), rest;
   for (int j = 0; j < n; ++j) {
@@ -571,6 +571,44 @@ bool eig_real(const std::vector<double>& a, int n, std::vector<double>& lam, std
   LMat qinv = inverse(qs);
   q = qs.to_double();
   qi = qinv.to_double();
+  return true;
+}
+
+// A matrix that couples indices of equal parity only (the operators of the composite bases) is
+// decomposed class by class: the eigenvectors of each class hold exact zeros in the other, where
+// a decomposition of the whole matrix leaves rounding (1e-17 to 1e-9 of their largest entry at
+// n = 24 to 400), and the two halves cost a quarter of the work.
+bool eig_real(const std::vector<double>& a, int n, std::vector<double>& lam, std::vector<double>& q,
+              std::vector<double>& qi, std::string& msg) {
+  bool split = n >= 4;
+  for (int i = 0; i < n && split; ++i)
+    for (int j = (i + 1) & 1; j < n; j += 2)
+      if (a[(size_t)i * n + j] != 0.0) { split = false; break; }
+  if (!split) return eig_whole(a, n, lam, q, qi, msg);
+  struct Pair { double lam; int c, k; };
+  std::vector<Pair> pairs;
+  std::vector<double> lc[2], qc[2], qic[2];
+  int nc[2];
+  for (int c = 0; c < 2; ++c) {
+    nc[c] = (n + 1 - c) / 2;
+    std::vector<double> b((size_t)nc[c] * nc[c]);
+    for (int i = 0; i < nc[c]; ++i)
+      for (int j = 0; j < nc[c]; ++j) b[(size_t)i * nc[c] + j] = a[(size_t)(2 * i + c) * n + 2 * j + c];
+    if (!eig_whole(b, nc[c], lc[c], qc[c], qic[c], msg)) return false;
+    for (int k = 0; k < nc[c]; ++k) pairs.push_back({lc[c][k], c, k});
+  }
+  std::stable_sort(pairs.begin(), pairs.end(), [](const Pair& x, const Pair& y) { return x.lam > y.lam; });
+  lam.assign(n, 0.0);
+  q.assign((size_t)n * n, 0.0);
+  qi.assign((size_t)n * n, 0.0);
+  for (int e = 0; e < n; ++e) {
+    const int c = pairs[e].c, k = pairs[e].k;
+    lam[e] = pairs[e].lam;
+    for (int i = 0; i < nc[c]; ++i) {
+      q[(size_t)(2 * i + c) * n + e] = qc[c][(size_t)i * nc[c] + k];
+      qi[(size_t)e * n + 2 * i + c] = qic[c][(size_t)k * nc[c] + i];
+    }
+  }
   return true;
 }
 
