@@ -246,7 +246,7 @@ struct PackedOp {
   DBuf buf;
   XOp op;
   size_t stride() const { return buf.n; }
-  void pack(const std::vector<double>& m, int rows, int cols) {
+  void pack(const std::vector<double>& m, int rows, int cols) {  // row-major rows x cols
     auto at = [&](int i, int j) { return m[(size_t)i * cols + j]; };
     op = XOp{};
     op.rows = rows;
@@ -326,7 +326,7 @@ struct PackedOp {
     for (int c = 0; c < ncls; ++c)
       for (int i = 0; i < op.M[c]; ++i)
         for (int k = 0; k < op.K[c]; ++k) all[c * size + xop_index(i, k, op.groups)] = cls[c][(size_t)i * op.K[c] + k];
-    buf.alloc(all.size());
+    if (buf.n != all.size()) buf.alloc(all.size());
     buf.upload(all);
     op.a[0] = buf.p;
     op.a[1] = ncls == 2 ? buf.p + size : nullptr;
@@ -405,7 +405,21 @@ struct Solver {
   std::vector<double> px;             // P_x (m x n) in double, for composing fwd * P_x
   std::vector<double> ax, cx;         // A_x, C_x (m x m) when axis 0 is not diagonal
   DOp pf, pb, py;
-  PackedOp hxp, pfp, pbp;  // hx, pf and pb as parity classes
+  PackedOp hxp, hyp, pfp, pbp;  // hx, the y inverse, pf and pb as parity classes
+  LMat hxl;                     // hx on the host, for composing further operators with it
+  // left operators composed with bwd (the x parts of the projection): left[i] bwd
+  std::vector<LMat> left;
+  std::vector<std::unique_ptr<PackedOp>> leftp;
+  void pack_left() {
+    LMat Q((int)lam.size(), (int)lam.size());
+    for (size_t i = 0; i < Q.a.size(); ++i) Q.a[i] = bwd[i];
+    leftp.clear();
+    for (const LMat& l : left) {
+      const LMat m = l * Q;
+      leftp.push_back(std::make_unique<PackedOp>());
+      leftp.back()->pack(m.to_double(), m.r, m.c);
+    }
+  }
   DBand pyb;  // P_y as a banded matvec
   std::vector<double> pyb_taps;  // its taps on the host, [4][m]
   DBuf low, dia, up1, up2;
@@ -459,6 +473,7 @@ struct Solver {
       upload_op(pb, Q);
       pfp.pack(FP.to_double(), FP.r, FP.c);
       pbp.pack(Q.to_double(), Q.r, Q.c);
+      if (!left.empty()) pack_left();
     }
   }
 };
@@ -479,8 +494,10 @@ static std::unique_ptr<Solver> make_solver(SKind kind, const Basis& b0, const Ba
       if (ax == 0) {
         upload_op(s->hx, H);
         s->hxp.pack(H.to_double(), H.r, H.c);
+        s->hxl = H;
       } else {
         upload_op(s->hy, H.t());
+        s->hyp.pack(H.to_double(), H.r, H.c);
       }
     }
     return s;
@@ -603,11 +620,13 @@ class Navier {
   Basis bx_u, bx_t, bx_p, bx_phi, bx_f, by_u, by_p, by_phi, by_bc;
   OpCache X, Y;
   std::shared_ptr<Solver> solver[4];
+  PackedOp dhx;  // d/dx to_ortho of the velocity's implicit x inverse (confined)
   // state
   DBuf T, UX, UY, P0, P1, BC;        // spectral (split planes when periodic)
   DBuf Tv, UXv, UYv, P0v, P1v, BCv;  // physical
   // constants derived from fieldbc
   DBuf THAT_BC, DTBCX, DTBCY, GXX, GYY;
+  DBuf BCXT, BCYT;  // DTBCX, DTBCY transposed (confined: the transposed convective products)
   // the physical fieldbc gradient: d/dx identically zero, d/dy the same in every x row
   bool bc_dx_zero = false, bc_dy_xconst = false;
   // rows of THAT_BC, GXX and GYY (spectral, [rows, ny]) before which every value is +0.0
@@ -631,8 +650,11 @@ class Navier {
   // whose buffers are slots nb * bs apart; per-instance nu and ADI operators in slabs
   int nb = 1;
   long bs = 0;
+  Navier* leader = nullptr;  // ensemble instances: the handle whose graph steps the group
   DBuf NUARR;
   DBuf ADIP[3];  // x: parity classes, solver[w]->hxp.stride() apart
+  DBuf ADIYP[3];  // y: the same of solver[w]->hyp
+  DBuf DHXP;      // d/dx of the velocity's x inverse: the same of dhx
   DBuf ADIH[3];  // y, adi_s apart
   long adi_s[3] = {};
   // Field batching (confined step): inside a FieldPair scope fb = 2 (or 3) and every launch
@@ -894,7 +916,7 @@ class Navier {
   // (3 B slots), the physical values ux and uy (2 B), A, CONV, CV, RHS, W1 and W2 three
   // fields' partners (3 B) and G the two pressure gradients (2 B).
   struct Slabs {
-    static constexpr int NK = 29;
+    static constexpr int NK = 31;
     size_t F = 0;
     int B = 0;
     DBuf slab[NK];
@@ -947,7 +969,8 @@ class Navier {
       if (per) throw std::invalid_argument("ensemble instances are confined");
       if (slabs->F != full) throw std::invalid_argument("ensemble slab stride mismatch");
       DBuf* all[Slabs::NK] = {&UX, &UY, &T, &UXP, &UYP, &A, &CONV, &CV, &RHS, &W1, &W2, &G, &P0, &P1, &Tv,
-                              &UXv, &UYv, &P0v, &P1v, &THAT_BC, &DTBCX, &DTBCY, &GXX, &GYY, &THAT, &DIV, &W3, &W4, &W9};
+                              &UXv, &UYv, &P0v, &P1v, &THAT_BC, &DTBCX, &DTBCY, &GXX, &GYY, &THAT, &DIV, &W3, &W4, &W9,
+                              &BCXT, &BCYT};
       for (int k = 0; k < Slabs::NK; ++k) all[k]->view(slabs->at(k, slot), full);
     } else {
       // slot-strided buffers of the batched step (slot k at p + k FS)
@@ -964,6 +987,8 @@ class Navier {
                       &W4, &W9})
         b->alloc(full);
     }
+    if (!slabs && !per)
+      for (DBuf* b : {&BCXT, &BCYT}) b->alloc(full);
     BC.alloc((size_t)R * 2);
     BCv.alloc((size_t)nx * ny);
     RED.alloc(std::max(ny, 8) + 300);
@@ -976,6 +1001,16 @@ class Navier {
     solver[1] = make_solver(hk, bx_u, by_u, cv);
     solver[2] = make_solver(hk, bx_t, by_u, ck);
     solver[3] = share ? share->solver[3] : std::shared_ptr<Solver>(make_solver(POISSON, bx_phi, by_phi, cp));
+    if (!per) {
+      const LMat d = build_axis_op(bx_u, "DS", (ld)scale[0]);
+      const LMat m = d * solver[0]->hxl;
+      dhx.pack(m.to_double(), m.r, m.c);
+      if (!share) {
+        const LMat fo = build_axis_op(bx_u, "FO", (ld)scale[0]);
+        solver[3]->left = {fo * build_axis_op(bx_phi, "DS", (ld)scale[0]), fo * build_axis_op(bx_phi, "S", (ld)scale[0])};
+        solver[3]->pack_left();
+      }
+    }
     // averaging weights of `field` (its coordinates are not rescaled, navier.rs:500-515)
     wx_dx = cell_widths(bx_f.coords(), bx_f.fourier());
     wy_dx = cell_widths(by_p.coords(), false);
@@ -1061,16 +1096,15 @@ class Navier {
     }
     g.split = 2 * nb;
   }
-  // the group's per-instance ADI x operators of field `which` (and of field `which2` for the
-  // entries from 2 nb on) in place of the leader's
-  void group_adi(XGemm& g, int which, int which2) {
-    const XOp& p = solver[which]->hxp.op;
+  // the group's per-instance operators p (packed in `slab`, p.stride() apart) in place of the
+  // leader's, and those of slab2 for the entries from the split on
+  void group_ops(XGemm& g, const PackedOp& p, const DBuf& slab, const DBuf* slab2 = nullptr) {
     for (int c = 0; c < 2; ++c) {
       g.op.mnz[c] = g.op.M[c];
-      g.op.a[c] = p.a[c] ? ADIP[which].p + (p.a[c] - p.a[0]) : nullptr;
-      if (which2 >= 0) g.a2[c] = p.a[c] ? ADIP[which2].p + (p.a[c] - p.a[0]) : nullptr;
+      g.op.a[c] = p.op.a[c] ? slab.p + (p.op.a[c] - p.op.a[0]) : nullptr;
+      if (slab2) g.a2[c] = p.op.a[c] ? slab2->p + (p.op.a[c] - p.op.a[0]) : nullptr;
     }
-    g.sA = (long)solver[which]->hxp.stride();
+    g.sA = (long)p.stride();
     g.amod = nb;
   }
   // one left operator's product on every entry of the current field batch, its parity classes
@@ -1272,7 +1306,7 @@ class Navier {
     const DOp &hx = s0.hx, &hy = s0.hy;
     XGemm g = xg(s0.hxp, RHS.p, ny, W1.p);
     two_ops(g, s2.hxp);
-    if (grp) group_adi(g, 0, 2);
+    if (grp) group_ops(g, s0.hxp, ADIP[0], &ADIP[2]);
     XGEMM(&g, 1);
     GEMM(hx.rows, hy.cols, hy.rows, W1.p, hy.rows, ay, hy.cols, UX.p, hy.cols, 0.0, nullptr, 0, DATA,
          grp ? adi_s[0] : 0, nullptr, ay2);
@@ -1307,6 +1341,209 @@ class Navier {
     solve_pres();
     project_velocity_pair();
     update_pres();
+    time += dt;
+  }
+
+  // ------------------------------------------------- the confined FP64 step (navier.rs:737-765)
+  // The dense operators as parity-class products along x or, on transposed arrays, along y
+  // (xgemm.hip), and what lies between them as row kernels (confined.hip): 12 launches, 13 with the
+  // y transforms by DCT, where stencils, derivatives, sums and products of their own took 29.  A
+  // step takes 47 us at 64^2 (105 before), 53 us at 128 x 129 (173), 101 us at 257^2 (205).
+  // RBC_OPT_BATCH 0 runs every launch field by field with the same arithmetic.
+  bool confined_fused_ok() {
+    if (periodic || mixed || solid_on || !use_bands || !xg_ok() || !vel_same || !confined_rows_supported(nx, ny)) return false;
+    if (solver[0]->kind != ADI || solver[1]->kind != ADI || solver[2]->kind != ADI || !solver[3]->has_fb) return false;
+    if (bx_u.k != CD || by_u.k != CD || by_phi.k != CN || bx_phi.k != CN || (bx_t.k != CD && bx_t.k != CN)) return false;
+    if (!fdma_rows_lds_supported(solver[3]->m, solver[3]->pyb.mi) || solver[3]->leftp.size() != 2) return false;
+    const Solver &s0 = *solver[0], &s2 = *solver[2];
+    for (const char* name : {"BS", "BDS"}) {
+      const XOp &u = X.packed(bx_u, name).op, &t = X.packed(bx_t, name).op;
+      if (u.kind != XOP_FOLD_OUT || !same_classes(u, t)) return false;
+      if (!confined_dct() && Y.packed(by_u, name).op.kind != XOP_FOLD_OUT) return false;
+    }
+    if (X.packed(bx_f, "Fdl").op.kind != XOP_FOLD_IN) return false;
+    if (!confined_dct() && Y.packed(by_p, "Fdl").op.kind != XOP_FOLD_IN) return false;
+    if (X.packed(bx_p, "DS").op.kind != XOP_BLOCKS || dhx.op.kind != XOP_BLOCKS) return false;
+    return s0.hxp.op.kind == XOP_BLOCKS && s0.hyp.op.kind == XOP_BLOCKS && same_classes(s0.hxp.op, s2.hxp.op) &&
+           same_classes(s0.hyp.op, s2.hyp.op);
+  }
+  // the y transforms of the convective terms by DCT: above 200 points the O(n log n) kernels are
+  // ahead of the dense products (257^2, one step: 101 us by DCT, 113 us dense; 128 x 129: 62 and
+  // 53 us; 64 x 65: 58 and 47 us)
+  bool confined_dct() const { return use_dct && nb == 1 && ny > 200 && cheb_y_supported(ny); }
+  // the products `op` (temp: `opt`) of fields f0 <= f < f1: in [op.cols, N] -> out at row stride ldc
+  XGemm field_op(const PackedOp& op, const PackedOp& opt, const double* in, int N, double* out, int ldc, int f0, int f1) {
+    const long at = f0 * pair_off();
+    XGemm g = xgemm_of(f0 >= 2 ? opt : op, in + at, out + at, N, (f1 - f0) * nb, dstr(), dstr());
+    g.ldc = ldc;
+    if (f0 < 2 && f1 > 2) {
+      for (int c = 0; c < 2; ++c) {
+        g.a2[c] = opt.op.a[c];
+        g.op.mnz[c] = std::max(g.op.mnz[c], opt.op.mnz[c]);
+      }
+      g.split = (2 - f0) * nb;
+    }
+    return g;
+  }
+  // one launch where the groups' operators can share it, one each otherwise
+  void XGEMMS(const XGemm* g, int ng, bool transposed) {
+    bool one = ng > 1;
+    for (int i = 0; i < ng; ++i)
+      one = one && g[i].op.groups == g[0].op.groups && (g[i].op.kind == XOP_BLOCKS || g[i].op.kind == XOP_FOLD_OUT);
+    for (int i = 0; i < ng; i += one ? ng : 1) {
+      double w = 0.0;
+      for (int k = i; k < (one ? ng : i + 1); ++k)
+        for (int c = 0; c < 2; ++c) w += 2.0 * g[k].op.M[c] * g[k].op.K[c] * (double)g[k].N * g[k].entries;
+      timer.begin(st, 0, w);
+      if (transposed) xgemm_t(st, g + i, one ? ng : 1);
+      else xgemm(st, g + i, one ? ng : 1);
+      timer.end(st);
+    }
+  }
+  template <class F>
+  void each_field(F fn) {
+    if (use_batch) fn(0, 3);
+    else
+      for (int f = 0; f < 3; ++f) fn(f, f + 1);
+  }
+  void update_confined() {
+    const Solver &s0 = *solver[0], &s2 = *solver[2], &sp = *solver[3];
+    const int mx_ = bx_u.m, my = by_u.m;
+    const long po = pair_off(), d = dstr();
+    const bool dct = confined_dct(), grp = nb > 1;
+    ConfinedRows a{};
+    a.U = UX.p;
+    a.RHS = RHS.p;
+    a.P0 = P0.p;
+    a.DIV = DIV.p;
+    a.CV = CV.p;
+    a.G = G.p;
+    a.that_bc = THAT_BC.p;
+    a.gxx = GXX.p;
+    a.gyy = GYY.p;
+    a.TX = W2.p + po;
+    a.P1 = P1.p;
+    a.GA = CV.p;
+    a.GB = CV.p + po;
+    a.sxu = stencil_band(bx_u).coef.p;
+    a.sxt = stencil_band(bx_t).coef.p;
+    a.sxp = stencil_band(bx_phi).coef.p;
+    a.sy = stencil_band(by_u).coef.p;
+    a.syp = stencil_band(by_phi).coef.p;
+    a.tdma = tdma_tables(by_u).tabp.p;
+    a.nuarr = grp ? NUARR.p : nullptr;
+    a.nx = nx;
+    a.ny = ny;
+    a.mx = mx_;
+    a.my = my;
+    a.field = po;
+    a.stride = d;
+    a.dt = dt;
+    a.inv_dt = 1.0 / dt;
+    a.inv_scy = 1.0 / scale[1];
+    a.nu = nu;
+    const double pts = (double)nx * ny * nb;
+    // x transforms of the fields' values and x derivatives, and d/dx pres
+    const PackedOp &bs = X.packed(bx_u, "BS"), &bst = X.packed(bx_t, "BS"), &bds = X.packed(bx_u, "BDS"),
+                   &bdst = X.packed(bx_t, "BDS"), &ds = X.packed(bx_p, "DS");
+    double *val = dct ? W2.p : A.p, *der = W1.p;
+    const int ldt = dct ? my : nx;  // [nx, my], or transposed [my, nx]
+    each_field([&](int f0, int f1) {
+      XGemm g[3] = {field_op(bs, bst, UX.p, my, val, ldt, f0, f1), field_op(bds, bdst, UX.p, my, der, ldt, f0, f1),
+                    xgemm_of(ds, P0.p, G.p, ny, nb, d, d)};
+      g[2].plain = 1;
+      XGEMMS(g, f0 == 0 ? 3 : 2, !dct);
+    });
+    // products in physical space and their dealiased transforms along y, into W2 [nx, ny]
+    if (dct) {
+      const DBand& band = stencil_band(by_u);
+      each_field([&](int f0, int f1) {
+        if (f0 < 2) CHEBY_BWD_B(by_u, val + f0 * po, UXP.p + f0 * po, nx, 0, nullptr, 0.0, std::min(f1, 2) - f0);
+      });
+      each_field([&](int f0, int f1) {
+        timer.begin(st, 11, 8.0 * nx * (f1 - f0) * (2.0 * my + 2.0 * ny));
+        cheb_y_conv(st, der + f0 * po, val + f0 * po, my, my, CONV.p + f0 * po, ny, nx, ny, band.coef.p, 1.0 / scale[1],
+                    UXP.p, UYP.p, ny, f1 - f0, (long)FS, (long)FS, UXP.p, bc_dx_zero ? nullptr : DTBCX.p, UYP.p, DTBCY.p,
+                    f1 > 2 ? 2 - f0 : -1, conv3_ldf());
+        timer.end(st);
+      });
+      each_field([&](int f0, int f1) { CHEBY_FWD_B(CONV.p + f0 * po, W2.p + f0 * po, nx, ny * 2 / 3, f1 - f0); });
+    } else {
+      const PackedOp& fy = Y.packed(by_p, "Fdl");
+      ConvArgs c{};
+      c.bs = Y.packed(by_u, "BS").op;
+      c.bds = Y.packed(by_u, "BDS").op;
+      c.T = val;
+      c.D = der;
+      c.fx = BCXT.p;
+      c.fy = BCYT.p;
+      c.C = CONV.p;
+      c.nx = nx;
+      c.nb = nb;
+      c.stride = c.sf = d;
+      each_field([&](int f0, int f1) {
+        c.f0 = f0;
+        c.f1 = f1;
+        timer.begin(st, 0, 2.0 * 4.0 * 0.5 * my * pts * (f1 - f0));
+        conv_products(st, c);
+        timer.end(st);
+      });
+      each_field([&](int f0, int f1) {
+        const XGemm g = field_op(fy, fy, CONV.p, nx, W2.p, ny, f0, f1);
+        XGEMMS(&g, 1, true);
+      });
+    }
+    const PackedOp& fx = X.packed(bx_f, "Fdl");
+    each_field([&](int f0, int f1) {
+      const XGemm g = field_op(fx, fx, W2.p, ny, CV.p, ny, f0, f1);
+      XGEMMS(&g, 1, false);
+    });
+    each_field([&](int f0, int f1) {
+      a.f0 = f0;
+      a.f1 = f1;
+      timer.begin(st, 3, 8.0 * pts * 4.0 * (f1 - f0));
+      rhs_rows(st, a, nb);
+      timer.end(st);
+    });
+    // the implicit inverses along x (transposed results), with d/dx ux beside ux, then along y
+    each_field([&](int f0, int f1) {
+      XGemm g[2] = {field_op(s0.hxp, s2.hxp, RHS.p, ny, W1.p, mx_, f0, f1), xgemm_of(dhx, RHS.p, W2.p, ny, nb, d, d)};
+      if (grp) {
+        group_ops(g[0], s0.hxp, f0 >= 2 ? ADIP[2] : ADIP[0], &ADIP[2]);
+        group_ops(g[1], dhx, DHXP);
+      }
+      g[1].ldc = nx;
+      XGEMMS(g, f0 == 0 ? 2 : 1, true);
+    });
+    each_field([&](int f0, int f1) {
+      XGemm g[2] = {field_op(s0.hyp, s2.hyp, W1.p, mx_, UX.p, my, f0, f1),
+                    xgemm_of(s0.hyp, W2.p, W2.p + po, nx, nb, d, d)};
+      if (grp) {
+        group_ops(g[0], s0.hyp, f0 >= 2 ? ADIYP[2] : ADIYP[0], &ADIYP[2]);
+        group_ops(g[1], s0.hyp, ADIYP[0]);
+      }
+      g[1].ldc = my;
+      XGEMMS(g, f0 == 0 ? 2 : 1, true);
+    });
+    a.f0 = 0;
+    a.f1 = 2;
+    timer.begin(st, 3, 8.0 * pts * 3.0);
+    div_rows(st, a, nb);
+    timer.end(st);
+    // pseudo pressure: eigen-transform, row systems, back-transform with the projection's x parts
+    {
+      const XGemm f = xgemm_of(sp.pfp, DIV.p, A.p, ny, nb, d, d);
+      XGEMMS(&f, 1, false);
+      ROWSF(A.p, ny, W1.p, by_phi.m, sp.pf.rows, sp);
+      XGemm g[3] = {xgemm_of(sp.pbp, W1.p, P1.p, by_phi.m, nb, d, d),
+                    xgemm_of(*sp.leftp[0], W1.p, CV.p, by_phi.m, nb, d, d),
+                    xgemm_of(*sp.leftp[1], W1.p, CV.p + po, by_phi.m, nb, d, d)};
+      g[0].zero00 = 1;
+      XGEMMS(g, 3, false);
+    }
+    timer.begin(st, 3, 8.0 * pts * 9.0);
+    proj_rows(st, a, nb, true);
+    timer.end(st);
     time += dt;
   }
 
@@ -1369,6 +1606,16 @@ class Navier {
     THAT_BC.upload(t);
     DTBCX.upload(hdx);
     DTBCY.upload(hdy);
+    if (!periodic) {
+      std::vector<double> tx(hdx.size()), ty(hdy.size());
+      for (int i = 0; i < nx; ++i)
+        for (int j = 0; j < ny; ++j) {
+          tx[(size_t)j * nx + i] = hdx[(size_t)i * ny + j];
+          ty[(size_t)j * nx + i] = hdy[(size_t)i * ny + j];
+        }
+      BCXT.upload(tx);
+      BCYT.upload(ty);
+    }
     bc_dx_zero = std::all_of(hdx.begin(), hdx.end(), [](double v) { return v == 0.0; });
     bc_dy_xconst = true;
     for (size_t i = (size_t)ny; i < hdy.size() && bc_dy_xconst; ++i) bc_dy_xconst = hdy[i] == hdy[i % (size_t)ny];
@@ -1399,7 +1646,7 @@ class Navier {
       const bool grp = nb > 1 && which < 3;  // the group's per-instance operators
       if (xg_ok()) {  // [mx, ny]
         XGemm g = xg(s.hxp, rhs, ny, W1.p);
-        if (grp) group_adi(g, which, -1);
+        if (grp) group_ops(g, s.hxp, ADIP[which]);
         XGEMM(&g, 1);
       } else {
         xmat(s.hx, rhs, ny, W1.p);
@@ -1914,6 +2161,10 @@ class Navier {
       return;
     }
     gpres_valid = false;
+    if (confined_fused_ok()) {
+      update_confined();
+      return;
+    }
     if (!periodic && triple_ok() && triple_ops_ok() && stencil2d_ok(bx_t, by_u) && stencil2d_ok(bx_u, by_u)) {
       update_triple();
       return;
@@ -2703,6 +2954,7 @@ class Ensemble {
                                                    di.adiabatic != 0, g->slabs.get(), b, g->st,
                                                    b > 0 ? g->navs[0].get() : nullptr));
         inst[mem[b]] = g->navs.back().get();
+        inst[mem[b]]->leader = g->navs[0].get();
         group_of[mem[b]] = (int)groups.size();
       }
       Navier& L = *g->navs[0];
@@ -2722,6 +2974,16 @@ class Ensemble {
             if (!Navier::same_classes(sb.hxp.op, L.solver[w]->hxp.op))
               throw std::logic_error("ensemble: implicit operators of one group differ in their parity classes");
             HIPCHECK(hipMemcpy(L.ADIP[w].p + b * sp, sb.hxp.buf.p, sp * sizeof(double), hipMemcpyDeviceToDevice));
+            if (!Navier::same_classes(sb.hyp.op, L.solver[w]->hyp.op))
+              throw std::logic_error("ensemble: implicit operators of one group differ in their parity classes");
+            const size_t sq = sb.hyp.stride();
+            if (b == 0) L.ADIYP[w].alloc(sq * B);
+            HIPCHECK(hipMemcpy(L.ADIYP[w].p + b * sq, sb.hyp.buf.p, sq * sizeof(double), hipMemcpyDeviceToDevice));
+            if (w == 0) {
+              const size_t sd = g->navs[b]->dhx.stride();
+              if (b == 0) L.DHXP.alloc(sd * B);
+              HIPCHECK(hipMemcpy(L.DHXP.p + b * sd, g->navs[b]->dhx.buf.p, sd * sizeof(double), hipMemcpyDeviceToDevice));
+            }
             HIPCHECK(hipMemcpy(L.ADIH[w].p + b * sy, sb.hy.b.p, sy * sizeof(double), hipMemcpyDeviceToDevice));
           }
         }
@@ -3196,6 +3458,7 @@ int rbc_set_tensor(rbc_navier* h, int s, const double* lam, const double* fwd, c
     if (sv.kind == rbc::ADI) throw std::invalid_argument("solver is HholtzAdi (no tensor)");
     HIPCHECK(hipStreamSynchronize(h->n->st));
     h->n->drop_graph();
+    if (h->n->leader) h->n->leader->drop_graph();  // the operators' classes, and with them its launches, may change
     std::memcpy(sv.lam.data(), lam, sv.lam.size() * sizeof(double));
     if (sv.has_fb) {
       if (!fwd || !bwd) throw std::invalid_argument("fwd/bwd required");

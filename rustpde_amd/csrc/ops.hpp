@@ -69,7 +69,7 @@ void gemm_mfma_f32_batched(hipStream_t s, int M, int N, int K, const float* A, i
 
 // Dense left operators split into their two parity classes (xgemm.hip).  Class c is a matrix of
 // M[c] x K[c] entries (M[0] >= M[1]), entry (m, k) at a[c][xop_index(m, k, groups)], packed with
-// zeros to whole 64 rows and xop_groups(max K) groups of 8 k values; rows m >= mnz[c] are zero and
+// zeros to whole 64 rows and `groups` >= xop_groups(max K) groups of 8 k values; rows m >= mnz[c] are zero and
 // not multiplied.
 enum { XOP_DENSE, XOP_BLOCKS, XOP_FOLD_IN, XOP_FOLD_OUT };
 struct XOp {
@@ -100,11 +100,28 @@ struct XGemm {
   long sB = 0;
   double* C = nullptr;
   int ldc = 0;
+  int plain = 0;  // xgemm_t: this group's results are not transposed
   long sC = 0;
   int N = 0, entries = 1, zero00 = 0;
 };
-constexpr int XGEMM_GROUPS = 3;  // independent products of one launch, operators of one kind
+constexpr int XGEMM_GROUPS = 3;  // independent products of one launch: block and fold-out operators
 void xgemm(hipStream_t s, const XGemm* groups, int ng);
+// The same with the results transposed: C_z [N, rows] = (op B_z)^T, row stride ldc.
+void xgemm_t(hipStream_t s, const XGemm* groups, int ng);
+// The convective terms in physical space, transposed ([ny, nx], x contiguous), of fields f0 <= f < f1
+// (ux, uy, temp) of nb instances, entry f nb + b of every array at that many strides:
+//   conv_f = (bs D_f) .* (bs T_ux) + (bds T_f) .* (bs T_uy)  (conv_term.rs:35-41)
+// from the transposed y-spectral values T and x-derivatives D [my, nx]; bs and bds are the y
+// operators to the points, of the value and of its y-derivative.  temp adds u fx + v fy
+// (navier.rs:547-550, fx and fy transposed, nb entries apart by sf).
+struct ConvArgs {
+  XOp bs, bds;
+  const double *T, *D, *fx, *fy;
+  double* C;
+  int nx, nb, f0, f1;
+  long stride, sf;
+};
+void conv_products(hipStream_t s, const ConvArgs& a);
 
 // Banded 4-diagonal solves (offsets -2, 0, 2, 4; pre-swept as fdma.rs:73-82) of every
 // row r of X[nrows, m] with diagonal set (r % nsets); diag arrays are [nsets, m].
@@ -276,6 +293,24 @@ bool tdma_rows_lds_supported(int m);
 // With project the result x is subtracted instead: X = x (-1) + X.
 void tdma_rows_lds(hipStream_t s, const double* R, int ldr, double* X, int ld, int rows, int m, const double* tabp,
                    int batch = 1, long sr = 0, long sx = 0, bool project = false);
+
+// Row kernels of the confined step (confined.hip).  Arrays of instance b (grid axis y) at b stride,
+// of field f (ux, uy, temp) at f field; U [mx, my] spectral, RHS, CV, G (d/dx pres), P0, DIV and the
+// boundary terms [nx, ny], TX (d/dx ux, y-spectral) [nx, my], P1, GA, GB [mx, my]; stencil taps of
+// an axis of n values as [2][n]: sxu, sxt, sxp along x for the velocity, temperature and pseudo
+// pressure, sy, syp along y.  Fields f0 <= f < f1 are written.
+struct ConfinedRows {
+  double *U, *RHS, *P0, *DIV;
+  const double *CV, *G, *that_bc, *gxx, *gyy, *TX, *P1, *GA, *GB;
+  const double *sxu, *sxt, *sxp, *sy, *syp, *tdma, *nuarr;
+  int nx, ny, mx, my, f0, f1;
+  long field, stride;
+  double dt, inv_dt, inv_scy, nu;
+};
+bool confined_rows_supported(int nx, int ny);
+void rhs_rows(hipStream_t s, const ConfinedRows& a, int nb);
+void div_rows(hipStream_t s, const ConfinedRows& a, int nb);
+void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure);
 
 // The pressure stage of the periodic step fused per x-wavenumber (one workgroup per k):
 // divergence, Poisson rows (pseu(0,0) = 0), projection of ux and uy, pressure update.

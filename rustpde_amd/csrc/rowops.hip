@@ -16,7 +16,7 @@
 
 #include "chains.hpp"
 #include "ops.hpp"
-#include "wave.hpp"
+#include "rowdiff.hpp"
 
 namespace rbc {
 
@@ -92,32 +92,7 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
     }
     __syncthreads();
   }
-  for (int t = 0; t < d1; ++t) {
-    // d_i = w_i + d_{i+2}, w_i = 2 (i+1) c_{i+1}; d_0 = c_1 + d_2 / 2
-    const int len = p == 0 ? (n + 1) / 2 : n / 2;
-    const int t0 = lane * per, cnt = max(0, min(per, len - t0));
-    double v[SLICE], s = 0.0;
-#pragma unroll
-    for (int q = SLICE - 1; q >= 0; --q) {
-      const int i = p + 2 * (t0 + q);
-      v[q] = q < cnt ? (i == 0 ? buf[pad(3)] : 2.0 * (double)(i + 1) * buf[pad(i + 3)]) : 0.0;
-      if (i > 0) s = s + v[q];
-    }
-    double above;
-    wave::suffix_sum(s, lane, above);
-#pragma unroll
-    for (int q = SLICE - 1; q >= 0; --q) {
-      if (q < cnt) {
-        above = (p == 0 && t0 + q == 0) ? v[q] + above / 2.0 : v[q] + above;
-        v[q] = above;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < SLICE; ++q)
-      if (q < cnt) buf[pad(p + 2 * (t0 + q) + 2)] = v[q];
-    __syncthreads();
-  }
+  for (int t = 0; t < d1; ++t) rowdiff::derive<SLICE>(buf, n, per, lane, p);
   if constexpr (CPLX) {
     const double ns = sc * sc + 0.0 * 0.0;
     for (int i = threadIdx.x; i < n; i += WAVE * WAVES) {

@@ -45,6 +45,20 @@ static ld sinpi(long long p, long long q) {
   return sinl(PI_L * (ld)r / (ld)q);
 }
 
+// cos(pi r / q) and sin(pi r / q) for r = 0 .. 2 q - 1: an operator's n^2 entries take 2 q values
+struct CosTable {
+  long long q;
+  std::vector<ld> c, s;
+  explicit CosTable(long long q_, bool sines = false) : q(q_), c(2 * q_), s(sines ? 2 * q_ : 0) {
+    for (long long r = 0; r < 2 * q; ++r) {
+      c[r] = cospi(r, q);
+      if (sines) s[r] = sinpi(r, q);
+    }
+  }
+  ld cos(long long p) const { return c[p % (2 * q)]; }
+  ld sin(long long p) const { return s[p % (2 * q)]; }
+};
+
 Basis::Basis(Kind kind, int n_) : k(kind), n(n_) {
   switch (k) {
     case CHEB: m = n; break;
@@ -93,8 +107,9 @@ LMat stencil(const Basis& b) {
 // T_k(x_j) = (-1)^k cos(pi j k/(n-1))
 LMat cheb_backward(int n) {
   LMat b(n, n);
+  const CosTable t(n - 1);
   for (int j = 0; j < n; ++j)
-    for (int k = 0; k < n; ++k) b(j, k) = ((k & 1) ? -1.0L : 1.0L) * cospi((long long)j * k, n - 1);
+    for (int k = 0; k < n; ++k) b(j, k) = ((k & 1) ? -1.0L : 1.0L) * t.cos((long long)j * k);
   return b;
 }
 
@@ -102,12 +117,13 @@ LMat cheb_backward(int n) {
 // DCT1(v)_k = v_0 + (-1)^k v_{n-1} + 2 sum_{j=1}^{n-2} v_j cos(pi j k/(n-1))
 LMat cheb_forward(int n) {
   LMat f(n, n);
+  const CosTable t(n - 1);
   for (int k = 0; k < n; ++k) {
     ld h = (k == 0 || k == n - 1) ? 0.5L : 1.0L;
     ld s = ((k & 1) ? -1.0L : 1.0L) / (ld)(n - 1) * h;
     for (int j = 0; j < n; ++j) {
       ld w = (j == 0 || j == n - 1) ? 1.0L : 2.0L;
-      f(k, j) = s * w * cospi((long long)j * k, n - 1);
+      f(k, j) = s * w * t.cos((long long)j * k);
     }
   }
   return f;
@@ -225,10 +241,11 @@ LMat from_ortho(const Basis& b) {
 LMat dft_r2c(int n) {
   const int m = n / 2 + 1;
   LMat a(2 * m, n);
+  const CosTable t(n, true);
   for (int k = 0; k < m; ++k)
     for (int j = 0; j < n; ++j) {
-      a(k, j) = cospi(2LL * j * k, n);
-      a(m + k, j) = -sinpi(2LL * j * k, n);
+      a(k, j) = t.cos(2LL * j * k);
+      a(m + k, j) = -t.sin(2LL * j * k);
     }
   return a;
 }
@@ -238,12 +255,13 @@ LMat dft_r2c(int n) {
 LMat dft_c2r(int n) {
   const int m = n / 2 + 1;
   LMat a(n, 2 * m);
+  const CosTable t(n, true);
   for (int j = 0; j < n; ++j)
     for (int k = 0; k < m; ++k) {
       bool edge = (k == 0) || (n % 2 == 0 && k == n / 2);
       ld w = edge ? 1.0L : 2.0L;
-      a(j, k) = w * cospi(2LL * j * k, n) / (ld)n;
-      a(j, m + k) = edge ? 0.0L : -w * sinpi(2LL * j * k, n) / (ld)n;
+      a(j, k) = w * t.cos(2LL * j * k) / (ld)n;
+      a(j, m + k) = edge ? 0.0L : -w * t.sin(2LL * j * k) / (ld)n;
     }
   return a;
 }

@@ -44,14 +44,24 @@ __device__ __forceinline__ T pick(bool one, T a, T b) {
   return one ? b : a;
 }
 
+// TR: the result is written transposed (C^T = op B, the operands of the MFMAs exchanged so that the
+// stores stay contiguous).  A product along y is a product along x of the transposed field, so a
+// two-dimensional transform is two such products, each reading and writing whole lines.
+// NC: parity classes of a block.  Folding in, both classes use the same loads; folding out and
+// transposed both classes' results share their lines of C.
+template <int KIND, bool TR>
+constexpr int classes_of() {
+  return KIND == XOP_DENSE ? 1 : KIND == XOP_BLOCKS ? (TR ? 2 : 1) : 2;
+}
+
 // A wavefront computes 16 FM x 16 FN values.  SPLIT: the four wavefronts of a block share one
 // such tile, a quarter of the k range each; otherwise they hold 2 x 2 tiles and each runs the
-// quarters in turn.  KIND: XOP_BLOCKS (and XOP_DENSE, one class), XOP_FOLD_IN or XOP_FOLD_OUT,
-// the same for every group; NG groups.  CH: groups of 8 k values per chunk of loads.
-template <int FM, int FN, bool SPLIT, int CH, int KIND, int NG>
+// quarters in turn.  KIND: the groups' operators' (folding out, a group may hold block
+// operators too).  CH: groups of 8 k values per chunk of loads.
+template <int FM, int FN, bool SPLIT, int CH, int KIND, int NG, bool TR>
 __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
-  constexpr bool IN2 = KIND == XOP_FOLD_IN, OUT2 = KIND == XOP_FOLD_OUT;
-  constexpr int NC = OUT2 ? 2 : 1;  // classes of a block
+  constexpr bool IN2 = KIND == XOP_FOLD_IN;
+  constexpr int NC = classes_of<KIND, TR>(), ND = IN2 ? 1 : NC;  // ND: distinct sets of data loads
   constexpr int BM = 16 * FM * (SPLIT ? 1 : 2), BN = 16 * FN * (SPLIT ? 1 : 2);
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
@@ -79,7 +89,7 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
     m0 += (wid >> 1) * 16 * FM;
     n0 += (wid & 1) * 16 * FN;
   }
-  const bool halves = !OUT2 && g.op.kind != XOP_DENSE;
+  const bool halves = KIND == XOP_BLOCKS && NC == 1;
   const bool c1 = halves && (t & 1);  // the block's class
   const int z = halves ? t >> 1 : t;
   const int M = pick(c1, g.op.M[0], g.op.M[1]), N = g.N;
@@ -93,13 +103,13 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
   const long aoff = g.amod ? g.sA * (z % g.amod) : 0;
   const double *a0 = second ? g.a2[0] : g.op.a[0], *a1 = second ? g.a2[1] : g.op.a[1];
   const int G = g.op.groups;  // groups of 8 k values of a packed row, a multiple of 4 CH
-  // class c of the block (folding out: both, otherwise its own)
+  // class c of the block (both, or its own)
   const double* Ac[NC];
   int Kc[NC], r0[NC];
   bool any = false;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const bool one = OUT2 ? c == 1 : c1;
+    const bool one = NC == 2 ? c == 1 : c1;
     any = any || m0 < pick(one, g.op.mnz[0], g.op.mnz[1]);  // else past a cut: zero rows
     Kc[c] = pick(one, g.op.K[0], g.op.K[1]);
     r0[c] = pick(one, g.op.r0[0], g.op.r0[1]);
@@ -108,9 +118,10 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
   const double* Bn[FN];  // this lane's columns (past N: a column inside, never stored)
 #pragma unroll
   for (int j = 0; j < FN; ++j) Bn[j] = B + min(n0 + 16 * j + lr, N - 1);
+  const long kst = ldb;  // from one input row of the operator to the next
 
   struct Chunk {
-    double2 a[NC][CH][FM], b[NC][CH][FN], m[IN2 ? CH : 1][IN2 ? FN : 1];
+    double2 a[NC][CH][FM], b[ND][CH][FN], m[IN2 ? CH : 1][IN2 ? FN : 1];
   };
   auto load = [&](int g0, Chunk& x) {  // groups g0 .. g0 + CH - 1
 #pragma unroll
@@ -120,15 +131,16 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
           x.a[c][h][i] = *reinterpret_cast<const double2*>(Ac[c] + ((size_t)i * G + g0 + h) * 128);
+        if (c >= ND) continue;
         const int k = (g0 + h) * 8 + 2 * lk;
         const int q0 = r0[c] + rs * min(k, Kc[c] - 1), q1 = r0[c] + rs * min(k + 1, Kc[c] - 1);
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          x.b[c][h][j].x = Bn[j][(long)q0 * ldb];
-          x.b[c][h][j].y = Bn[j][(long)q1 * ldb];
+          x.b[c][h][j].x = Bn[j][q0 * kst];
+          x.b[c][h][j].y = Bn[j][q1 * kst];
           if constexpr (IN2) {
-            x.m[h][j].x = Bn[j][(long)(last - q0) * ldb];
-            x.m[h][j].y = Bn[j][(long)(last - q1) * ldb];
+            x.m[h][j].x = Bn[j][(last - q0) * kst];
+            x.m[h][j].y = Bn[j][(last - q1) * kst];
           }
         }
       }
@@ -151,17 +163,18 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
         const bool ok0 = k < Kc[c], ok1 = k + 1 < Kc[c];  // the packed rows end in zeros, B does not
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          double2 b = x.b[c][h][j];
+          double2 b = x.b[c < ND ? c : 0][h][j];
           if constexpr (IN2) {
-            b.x = c1 ? b.x - x.m[h][j].x : b.x + x.m[h][j].x;
-            b.y = c1 ? b.y - x.m[h][j].y : b.y + x.m[h][j].y;
+            b.x = c ? b.x - x.m[h][j].x : b.x + x.m[h][j].x;
+            b.y = c ? b.y - x.m[h][j].y : b.y + x.m[h][j].y;
           }
           b.x = ok0 ? b.x : 0.0;
           b.y = ok1 ? b.y : 0.0;
 #pragma unroll
           for (int i = 0; i < FM; ++i) {
-            acc[c][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.a[c][h][i].x, b.x, acc[c][i][j], 0, 0, 0);
-            acc[c][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.a[c][h][i].y, b.y, acc[c][i][j], 0, 0, 0);
+            const double2 a = x.a[c][h][i];
+            acc[c][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(TR ? b.x : a.x, TR ? a.x : b.x, acc[c][i][j], 0, 0, 0);
+            acc[c][i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(TR ? b.y : a.y, TR ? a.y : b.y, acc[c][i][j], 0, 0, 0);
           }
         }
       }
@@ -237,11 +250,12 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
       clear();
     }
   }
-  const int ldc = g.ldc, rows = g.op.rows, c0 = pick(c1, g.op.c0[0], g.op.c0[1]), cs = g.op.cstep;
-  const bool pin = g.zero00 != 0;
-  auto put = [&](int row, int col, double v) {
+  const int ldc = g.ldc, rows = g.op.rows, cs = g.op.cstep;
+  const bool pin = g.zero00 != 0, out2 = KIND == XOP_FOLD_OUT && g.op.kind == XOP_FOLD_OUT;
+  const int e0 = pick(c1, g.op.c0[0], g.op.c0[1]), e1 = g.op.c0[1], M1 = g.op.M[1];
+  auto put = [&](int row, int col, double v) {  // row of the operator, column of the data
     if (pin && row == 0 && col == 0) v = 0.0;
-    C[(size_t)row * ldc + col] = v;
+    C[TR && !g.plain ? (size_t)col * ldc + row : (size_t)row * ldc + col] = v;
   };
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -249,21 +263,145 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = m0 + i * 16 + 4 * r + lk, n = n0 + j * 16 + lr;
+        const int m = m0 + i * 16 + (TR ? lr : 4 * r + lk), n = n0 + j * 16 + (TR ? 4 * r + lk : lr);
         if (m >= M || n >= N) continue;
         const double v = acc[0][i][j][r];
-        if constexpr (OUT2) {
+        if constexpr (NC == 2) {
           const double o = acc[1][i][j][r];
-          const int mirror = rows - 1 - m;
-          put(m, n, v + o);
-          if (mirror != m) put(mirror, n, v - o);
+          if (out2) {
+            const int mirror = rows - 1 - m;
+            put(m, n, v + o);
+            if (mirror != m) put(mirror, n, v - o);
+          } else {
+            put(e0 + cs * m, n, v);
+            if (m < M1) put(e1 + cs * m, n, o);
+          }
         } else {
-          put(c0 + cs * m, n, v);
+          put(e0 + cs * m, n, v);
         }
       }
 }
 
-template <int FM, int FN, bool SPLIT, int CH, int KIND, int NG>
+// conv_products: a block computes rows [m0, m0 + 16) and their mirror rows of 16 columns of one
+// field's term, its four wavefronts a quarter of the k range each: four products of two classes,
+//   u = bs T_ux, v = bs T_uy, d/dx q = bs D_q, d/dy q = bds T_q,
+// combined point by point.  u and v are formed again for each field: at the sizes where the
+// launches are short, one launch in place of four (two products of the velocity, two with an
+// epilogue, one for the boundary field's gradient) matters more than the products it repeats.
+template <int CH>
+__global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
+  int t = fftlds::xcd_remap(blockIdx.x, gridDim.x);
+  const int n0 = (t % tx) * 16;
+  t /= tx;
+  const int m0 = (t % ty) * 16, z = t / ty, b = z % a.nb, f = a.f0 + z / a.nb, N = a.nx;
+  const int col = min(n0 + lr, N - 1), G = a.bs.groups;
+  // data rows: T_ux, T_uy, D_f, T_f; their class c is row parity c ^ r0 of the operator
+  const double* src[4] = {a.T + a.stride * b + col, a.T + a.stride * (a.nb + b) + col,
+                          a.D + a.stride * (f * a.nb + b) + col, a.T + a.stride * (f * a.nb + b) + col};
+  const double* opa[2][2];  // [bs, bds][class]
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    opa[0][c] = a.bs.a[c] + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
+    opa[1][c] = a.bds.a[c] + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
+  }
+  const int Kb[2] = {a.bs.K[0], a.bs.K[1]}, Kd[2] = {a.bds.K[0], a.bds.K[1]};
+  const int rb[2] = {a.bs.r0[0], a.bs.r0[1]}, rd[2] = {a.bds.r0[0], a.bds.r0[1]};
+  struct Chunk {
+    double2 o[2][2][CH], d[4][2][CH];
+  };
+  v4d acc[4][2];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[p][c] = v4d{0, 0, 0, 0};
+  auto load = [&](int g0, Chunk& x) {
+#pragma unroll
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int k = (g0 + h) * 8 + 2 * lk;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) x.o[p][c][h] = *reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128);
+        const long b0 = (long)(rb[c] + 2 * min(k, Kb[c] - 1)) * N, b1 = (long)(rb[c] + 2 * min(k + 1, Kb[c] - 1)) * N;
+        const long d0 = (long)(rd[c] + 2 * min(k, Kd[c] - 1)) * N, d1 = (long)(rd[c] + 2 * min(k + 1, Kd[c] - 1)) * N;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) x.d[p][c][h] = double2{src[p][p == 3 ? d0 : b0], src[p][p == 3 ? d1 : b1]};
+      }
+  };
+  auto mac = [&](int g0, const Chunk& x) {
+#pragma unroll
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int k = (g0 + h) * 8 + 2 * lk;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const int K = p == 3 ? Kd[c] : Kb[c];
+          const double2 o = x.o[p == 3 ? 1 : 0][c][h];
+          const double v0 = k < K ? x.d[p][c][h].x : 0.0, v1 = k + 1 < K ? x.d[p][c][h].y : 0.0;
+          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.x, v0, acc[p][c], 0, 0, 0);
+          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.y, v1, acc[p][c], 0, 0, 0);
+        }
+      }
+  };
+  Chunk x, y;
+  const int nch = G / (4 * CH), top = G - CH, g0 = wid * nch * CH;
+  load(g0, x);
+  int n = 0;
+  for (; n + 2 <= nch; n += 2) {
+    load(min(g0 + (n + 1) * CH, top), y);
+    mac(g0 + n * CH, x);
+    load(min(g0 + (n + 2) * CH, top), x);
+    mac(g0 + (n + 1) * CH, y);
+  }
+  if (n < nch) mac(g0 + n * CH, x);
+  __shared__ v4d part[2][8][64];
+  auto put = [&](int s) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) part[s][e][lane] = acc[e >> 1][e & 1];
+  };
+  auto add = [&](int s) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e >> 1][e & 1] += part[s][e][lane];
+  };
+  if (wid & 1) put(wid >> 1);
+  __syncthreads();
+  if (!(wid & 1)) add(wid >> 1);
+  __syncthreads();
+  if (wid == 2) put(0);
+  __syncthreads();
+  if (wid != 0) return;
+  add(0);
+  const int ny = a.bs.rows;
+  double* C = a.C + a.stride * (f * a.nb + b);
+  const double *fx = a.fx + a.sf * b, *fy = a.fy + a.sf * b;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma clang fp contract(off)
+    const int m = m0 + 4 * r + lk, nn = n0 + lr;
+    if (m >= a.bs.M[0] || nn >= N) continue;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+      const int row = side ? ny - 1 - m : m;
+      if (side && row == m) continue;
+      double v[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) v[p] = side ? acc[p][0][r] - acc[p][1][r] : acc[p][0][r] + acc[p][1][r];
+      const size_t at = (size_t)row * N + nn;
+      double q = v[2] * v[0];
+      q = q + v[3] * v[1];
+      if (f == 2) {
+        q = q + v[0] * fx[at];
+        q = q + v[1] * fy[at];
+      }
+      C[at] = q;
+    }
+  }
+}
+
+template <int FM, int FN, bool SPLIT, int CH, int KIND, int NG, bool TR>
 void launch(hipStream_t s, const XGemm* groups) {
   constexpr int BM = 16 * FM * (SPLIT ? 1 : 2), BN = 16 * FN * (SPLIT ? 1 : 2);
   XArgs<NG> ar{};
@@ -272,60 +410,68 @@ void launch(hipStream_t s, const XGemm* groups) {
     ar.g[i] = groups[i];
     ar.tx[i] = (groups[i].N + BN - 1) / BN;
     ar.ty[i] = (groups[i].op.M[0] + BM - 1) / BM;
-    const int ncls = KIND == XOP_FOLD_OUT || groups[i].op.kind == XOP_DENSE ? 1 : 2;
+    const int ncls = KIND == XOP_BLOCKS && classes_of<KIND, TR>() == 1 ? 2 : 1;  // blocks per tile
     total += (long)ar.tx[i] * ar.ty[i] * ncls * groups[i].entries;
     if (total > 0x7fffffffL) throw std::invalid_argument("xgemm: too many tiles");
     ar.end[i] = (int)total;
   }
-  RBC_LAUNCH((xgemm_kernel<FM, FN, SPLIT, CH, KIND, NG>), dim3((unsigned)total), dim3(256), 0, s, ar);
+  RBC_LAUNCH((xgemm_kernel<FM, FN, SPLIT, CH, KIND, NG, TR>), dim3((unsigned)total), dim3(256), 0, s, ar);
 }
 
 enum { TILE_16, TILE_32, TILE_64 };
 
-template <int CH, int KIND, int NG>
+template <int CH, int KIND, int NG, bool TR>
 void launch_tile(hipStream_t s, const XGemm* groups, int tile) {
   // the larger tiles take shorter chunks: fewer registers, more wavefronts per SIMD
   constexpr int CS = CH == 4 ? 2 : CH == 3 ? 1 : CH;
   switch (tile) {
-    case TILE_16: launch<1, 1, true, CH, KIND, NG>(s, groups); break;
-    case TILE_32: launch<2, 1, true, CS, KIND, NG>(s, groups); break;
-    default: launch<2, 2, false, CS, KIND, NG>(s, groups); break;
+    case TILE_16: launch<1, 1, true, CH, KIND, NG, TR>(s, groups); break;
+    case TILE_32: launch<2, 1, true, CS, KIND, NG, TR>(s, groups); break;
+    default: launch<2, 2, false, CS, KIND, NG, TR>(s, groups); break;
   }
 }
 
-template <int CH, int KIND>
-void launch_groups(hipStream_t s, const XGemm* groups, int ng, int tile) {
-  switch (ng) {
-    case 1: launch_tile<CH, KIND, 1>(s, groups, tile); break;
-    case 2: launch_tile<CH, KIND, 2>(s, groups, tile); break;
-    default: launch_tile<CH, KIND, 3>(s, groups, tile); break;
-  }
-}
-
-template <int KIND>
-void launch_chunk(hipStream_t s, const XGemm* groups, int ng, int tile, int ch) {
+template <int KIND, int NG, bool TR>
+void launch_chunk(hipStream_t s, const XGemm* groups, int tile, int ch) {
   switch (ch) {
-    case 1: launch_groups<1, KIND>(s, groups, ng, tile); break;
-    case 2: launch_groups<2, KIND>(s, groups, ng, tile); break;
-    case 3: launch_groups<3, KIND>(s, groups, ng, tile); break;
-    default: launch_groups<4, KIND>(s, groups, ng, tile); break;
+    case 1: launch_tile<1, KIND, NG, TR>(s, groups, tile); break;
+    case 2: launch_tile<2, KIND, NG, TR>(s, groups, tile); break;
+    case 3: launch_tile<3, KIND, NG, TR>(s, groups, tile); break;
+    default: launch_tile<4, KIND, NG, TR>(s, groups, tile); break;
+  }
+}
+
+template <bool TR>
+void launch_kind(hipStream_t s, const XGemm* groups, int ng, int kind, int tile, int ch) {
+  if (ng > 1) {
+    if (kind == XOP_FOLD_OUT) launch_chunk<XOP_FOLD_OUT, XGEMM_GROUPS, TR>(s, groups, tile, ch);
+    else launch_chunk<XOP_BLOCKS, XGEMM_GROUPS, TR>(s, groups, tile, ch);
+    return;
+  }
+  switch (kind) {
+    case XOP_FOLD_IN: launch_chunk<XOP_FOLD_IN, 1, TR>(s, groups, tile, ch); break;
+    case XOP_FOLD_OUT: launch_chunk<XOP_FOLD_OUT, 1, TR>(s, groups, tile, ch); break;
+    case XOP_BLOCKS: launch_chunk<XOP_BLOCKS, 1, TR>(s, groups, tile, ch); break;
+    default: launch_chunk<XOP_DENSE, 1, TR>(s, groups, tile, ch); break;
   }
 }
 
 }  // namespace
 
 // groups of 8 k values of a packed row with K values: four equal quarters of whole chunks
-int xop_chunk(int K) {  // the chunk of 2, 3 or 4 groups that pads a quarter least
-  const int q = (K + 31) / 32;  // groups of a quarter
-  if (q <= 4) return q;
-  int best = 4;
-  for (int ch = 3; ch >= 2; --ch)
-    if ((q + ch - 1) / ch * ch < (q + best - 1) / best * best) best = ch;
-  return best;
+int xop_chunk(int groups) {  // the longest chunk of at most 4 groups that divides a quarter
+  const int q = groups / 4;
+  for (int ch = q < 4 ? q : 4; ch > 1; --ch)
+    if (q % ch == 0) return ch;
+  return 1;
 }
 int xop_groups(int K) {
-  const int q = (K + 31) / 32, ch = xop_chunk(K);
-  return 4 * ((q + ch - 1) / ch * ch);
+  const int q = (K + 31) / 32;  // groups of a quarter
+  if (q <= 4) return 4 * q;
+  int best = 4;  // the chunk of 2, 3 or 4 groups that pads the quarter least
+  for (int ch = 3; ch >= 2; --ch)
+    if ((q + ch - 1) / ch * ch < (q + best - 1) / best * best) best = ch;
+  return 4 * ((q + best - 1) / best * best);
 }
 
 // The tile follows from the launch's size, 16 x 16 tiles times groups of 8 k values (twice when
@@ -337,26 +483,54 @@ int xop_groups(int K) {
 //   64^2 x 3 (384): 2.67 / 2.79 (4.00), of which 1.66 is an empty launch.
 // Beyond a million the wavefronts of a block take a tile of their own each, 64 x 64 together, which
 // halves the loads per product: 510^2 x 64 (2.1 million) 179 us, 47 TFLOP/s, against 195 us.
-void xgemm(hipStream_t s, const XGemm* groups, int ng) {
+void conv_products(hipStream_t s, const ConvArgs& a) {
+  if (a.bs.kind != XOP_FOLD_OUT || a.bds.kind != XOP_FOLD_OUT || a.bs.groups != a.bds.groups ||
+      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.f0 < 0 || a.f1 > 3 || a.f0 >= a.f1 || a.nx < 1 || a.nb < 1)
+    throw std::invalid_argument("conv_products: bad arguments");
+  const int tx = (a.nx + 15) / 16, ty = (a.bs.M[0] + 15) / 16;
+  const long total = (long)tx * ty * a.nb * (a.f1 - a.f0);
+  if (total > 0x7fffffffL) throw std::invalid_argument("conv_products: too many tiles");
+  const dim3 grid((unsigned)total), block(256);
+  const int q = a.bs.groups / 4;  // chunks of two groups (the registers of four products in flight)
+  if (q % 2 == 0) RBC_LAUNCH(conv_kernel<2>, grid, block, 0, s, a, tx, ty);
+  else RBC_LAUNCH(conv_kernel<1>, grid, block, 0, s, a, tx, ty);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) throw std::runtime_error(std::string("conv_products: ") + hipGetErrorString(e));
+}
+
+static void xgemm_any(hipStream_t s, const XGemm* in, int ng, bool transposed) {
   if (ng < 1 || ng > XGEMM_GROUPS) throw std::invalid_argument("xgemm: bad group count");
-  const int kind = groups[0].op.kind == XOP_DENSE ? XOP_BLOCKS : groups[0].op.kind;
-  const int ch = xop_chunk(groups[0].op.K[0] > groups[0].op.K[1] ? groups[0].op.K[0] : groups[0].op.K[1]);
+  XGemm groups[XGEMM_GROUPS];
+  bool out = false;
   long size = 0;
   for (int i = 0; i < ng; ++i) {
-    const XGemm& g = groups[i];
+    const XGemm& g = groups[i] = in[i];
+    out = out || g.op.kind == XOP_FOLD_OUT;
     if (g.entries < 1 || g.N < 1 || g.op.M[0] < 1 || !g.B || !g.C || g.op.M[1] > g.op.M[0])
       throw std::invalid_argument("xgemm: bad sizes");
-    if ((g.op.kind == XOP_DENSE ? XOP_BLOCKS : g.op.kind) != kind || g.op.groups != groups[0].op.groups)
-      throw std::invalid_argument("xgemm: the groups' operators differ in kind or length");
+    if (g.op.groups != in[0].op.groups) throw std::invalid_argument("xgemm: the groups' operators differ in length");
     const int ncls = g.op.kind == XOP_DENSE ? 1 : 2;
     size += (long)((g.N + 15) / 16) * ((g.op.M[0] + 15) / 16) * ncls * g.entries * g.op.groups;
   }
+  if (ng > 1) {
+    for (int i = 0; i < ng; ++i)
+      if (in[i].op.kind == XOP_DENSE || in[i].op.kind == XOP_FOLD_IN ||
+          (!out && in[i].op.kind != XOP_BLOCKS))
+        throw std::invalid_argument("xgemm: these operators do not share a launch");
+    for (int i = ng; i < XGEMM_GROUPS; ++i) {  // an empty group
+      groups[i] = groups[0];
+      groups[i].entries = 0;
+    }
+  }
+  const int kind = out ? (int)XOP_FOLD_OUT : groups[0].op.kind, ch = xop_chunk(groups[0].op.groups);
   const int tile = size < 18000 ? TILE_16 : size < 1000000 ? TILE_32 : TILE_64;
-  if (kind == XOP_FOLD_IN) launch_chunk<XOP_FOLD_IN>(s, groups, ng, tile, ch);
-  else if (kind == XOP_FOLD_OUT) launch_chunk<XOP_FOLD_OUT>(s, groups, ng, tile, ch);
-  else launch_chunk<XOP_BLOCKS>(s, groups, ng, tile, ch);
+  if (transposed) launch_kind<true>(s, groups, ng, kind, tile, ch);
+  else launch_kind<false>(s, groups, ng, kind, tile, ch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw std::runtime_error(std::string("xgemm: ") + hipGetErrorString(e));
 }
+
+void xgemm(hipStream_t s, const XGemm* groups, int ng) { xgemm_any(s, groups, ng, false); }
+void xgemm_t(hipStream_t s, const XGemm* groups, int ng) { xgemm_any(s, groups, ng, true); }
 
 }  // namespace rbc
