@@ -54,6 +54,24 @@ constexpr int classes_of() {
   return KIND == XOP_DENSE ? 1 : KIND == XOP_BLOCKS ? (TR ? 2 : 1) : 2;
 }
 
+// (q0 + q1) + (q2 + q3) of the four wavefronts' partial tiles e < NE, in LDS: get(e, r) gives the
+// calling wavefront's register r of tile e, put(e, v) takes the sum of register wid.
+template <int NE, class Get, class Put>
+__device__ __forceinline__ void add_quarters(double* part, int wid, int lane, Get get, Put put) {
+#pragma unroll
+  for (int e = 0; e < NE; ++e)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[((e * 4 + wid) * 4 + r) * 64 + lane] = get(e, r);
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    double q[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) q[w] = part[((e * 4 + w) * 4 + wid) * 64 + lane];
+    put(e, (q[0] + q[1]) + (q[2] + q[3]));
+  }
+}
+
 // A wavefront computes 16 FM x 16 FN values.  SPLIT: the four wavefronts of a block share one
 // such tile, a quarter of the k range each; otherwise they hold 2 x 2 tiles and each runs the
 // quarters in turn.  KIND: the groups' operators' (folding out, a group may hold block
@@ -202,31 +220,20 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
       }
     }
   };
+  // the values a lane writes: register r of its MFMA results, all four of them or, with the k range
+  // split, the wavefront's own r (each wavefront adds and stores a quarter of the tile)
+  constexpr int RN = SPLIT ? 1 : 4;
+  double res[NC][FM][FN][RN];
   if constexpr (SPLIT) {
-    // partial sums of the quarters through LDS, lanes side by side
-    __shared__ v4d part[2][NC * FM * FN][64];
     const int g0 = wid * nch * CH;
     clear();
     if (any) {
       load(g0, x);
       quarter(g0);
     }
-    auto put = [&](int s) {
-#pragma unroll
-      for (int e = 0; e < NC * FM * FN; ++e) part[s][e][lane] = acc[e / (FM * FN)][e / FN % FM][e % FN];
-    };
-    auto add = [&](int s) {
-#pragma unroll
-      for (int e = 0; e < NC * FM * FN; ++e) acc[e / (FM * FN)][e / FN % FM][e % FN] += part[s][e][lane];
-    };
-    if (wid & 1) put(wid >> 1);
-    __syncthreads();
-    if (!(wid & 1)) add(wid >> 1);
-    __syncthreads();
-    if (wid == 2) put(0);
-    __syncthreads();
-    if (wid != 0) return;
-    add(0);
+    __shared__ double part[NC * FM * FN * 16 * 64];
+    add_quarters<NC * FM * FN>(part, wid, lane, [&](int e, int r) { return acc[e / (FM * FN)][e / FN % FM][e % FN][r]; },
+                               [&](int e, double v) { res[e / (FM * FN)][e / FN % FM][e % FN][0] = v; });
   } else {
     v4d sum[NC][FM][FN], pair[NC][FM][FN];
     if (any) {
@@ -249,6 +256,14 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
     } else {
       clear();
     }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) res[c][i][j][SPLIT ? 0 : r] = acc[c][i][j][r];
   }
   const int ldc = g.ldc, rows = g.op.rows, cs = g.op.cstep;
   const bool pin = g.zero00 != 0, out2 = KIND == XOP_FOLD_OUT && g.op.kind == XOP_FOLD_OUT;
@@ -262,12 +277,13 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
+      for (int q = 0; q < RN; ++q) {
+        const int r = SPLIT ? wid : q;
         const int m = m0 + i * 16 + (TR ? lr : 4 * r + lk), n = n0 + j * 16 + (TR ? 4 * r + lk : lr);
         if (m >= M || n >= N) continue;
-        const double v = acc[0][i][j][r];
+        const double v = res[0][i][j][q];
         if constexpr (NC == 2) {
-          const double o = acc[1][i][j][r];
+          const double o = res[1][i][j][q];
           if (out2) {
             const int mirror = rows - 1 - m;
             put(m, n, v + o);
@@ -282,38 +298,46 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
       }
 }
 
-// conv_products: a block computes rows [m0, m0 + 16) and their mirror rows of 16 columns of one
-// field's term, its four wavefronts a quarter of the k range each: four products of two classes,
-//   u = bs T_ux, v = bs T_uy, d/dx q = bs D_q, d/dy q = bds T_q,
-// combined point by point.  u and v are formed again for each field: at the sizes where the
-// launches are short, one launch in place of four (two products of the velocity, two with an
-// epilogue, one for the boundary field's gradient) matters more than the products it repeats.
-template <int CH>
+// conv_products: a block computes rows [m0, m0 + 16) and their mirror rows of 16 columns, its four
+// wavefronts a quarter of the k range each: the products
+//   u = bs T_ux, v = bs T_uy, and per field d/dx q = bs D_q, d/dy q = bds T_q,
+// of two parity classes each, combined point by point.  NF = 1: one field per block, u and v formed
+// again for each; NF = 3: the three fields in one block (8 products in place of 12, on 16 tiles of
+// accumulators per wavefront, so one block per CU).  One launch in place of four (the velocity, two
+// products with an epilogue, the boundary field's gradient).
+template <int CH, int NF>
 __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
+  constexpr int ND = NF == 3 ? 6 : 4, NP = NF == 3 ? 8 : 4;  // data arrays, products
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   int t = fftlds::xcd_remap(blockIdx.x, gridDim.x);
   const int n0 = (t % tx) * 16;
   t /= tx;
-  const int m0 = (t % ty) * 16, z = t / ty, b = z % a.nb, f = a.f0 + z / a.nb, N = a.nx;
+  const int m0 = (t % ty) * 16, z = t / ty, b = z % a.nb, f = NF == 3 ? 0 : a.f0 + z / a.nb, N = a.nx;
   const int col = min(n0 + lr, N - 1), G = a.bs.groups;
-  // data rows: T_ux, T_uy, D_f, T_f; their class c is row parity c ^ r0 of the operator
-  const double* src[4] = {a.T + a.stride * b + col, a.T + a.stride * (a.nb + b) + col,
-                          a.D + a.stride * (f * a.nb + b) + col, a.T + a.stride * (f * a.nb + b) + col};
+  // NF = 1: T_ux, T_uy, D_f, T_f; NF = 3: T and D of the three fields
+  const double* src[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const int ff = NF == 3 ? i % 3 : i < 2 ? i : f;
+    src[i] = (NF == 3 ? i < 3 : i != 2) ? a.T : a.D;
+    src[i] += a.stride * (ff * a.nb + b) + col;
+  }
   const double* opa[2][2];  // [bs, bds][class]
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     opa[0][c] = a.bs.a[c] + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
     opa[1][c] = a.bds.a[c] + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
   }
-  const int Kb[2] = {a.bs.K[0], a.bs.K[1]}, Kd[2] = {a.bds.K[0], a.bds.K[1]};
-  const int rb[2] = {a.bs.r0[0], a.bs.r0[1]}, rd[2] = {a.bds.r0[0], a.bds.r0[1]};
+  // rows of row parity p: 2 k + p below cols; class c of bs takes parity rb[c], of bds rd[c]
+  const int Kp[2] = {a.bs.r0[0] == 0 ? a.bs.K[0] : a.bs.K[1], a.bs.r0[0] == 0 ? a.bs.K[1] : a.bs.K[0]};
+  const int b0 = a.bs.r0[0], d0 = a.bds.r0[0];  // parity of class 0
   struct Chunk {
-    double2 o[2][2][CH], d[4][2][CH];
+    double2 o[2][2][CH], d[ND][2][CH];  // [operator][class], [array][row parity]
   };
-  v4d acc[4][2];
+  v4d acc[NP][2];
 #pragma unroll
-  for (int p = 0; p < 4; ++p)
+  for (int p = 0; p < NP; ++p)
 #pragma unroll
     for (int c = 0; c < 2; ++c) acc[p][c] = v4d{0, 0, 0, 0};
   auto load = [&](int g0, Chunk& x) {
@@ -324,27 +348,35 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
         const int k = (g0 + h) * 8 + 2 * lk;
 #pragma unroll
         for (int p = 0; p < 2; ++p) x.o[p][c][h] = *reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128);
-        const long b0 = (long)(rb[c] + 2 * min(k, Kb[c] - 1)) * N, b1 = (long)(rb[c] + 2 * min(k + 1, Kb[c] - 1)) * N;
-        const long d0 = (long)(rd[c] + 2 * min(k, Kd[c] - 1)) * N, d1 = (long)(rd[c] + 2 * min(k + 1, Kd[c] - 1)) * N;
+        const long q0 = (long)(c + 2 * min(k, Kp[c] - 1)) * N, q1 = (long)(c + 2 * min(k + 1, Kp[c] - 1)) * N;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) x.d[p][c][h] = double2{src[p][p == 3 ? d0 : b0], src[p][p == 3 ? d1 : b1]};
+        for (int i = 0; i < ND; ++i) x.d[i][c][h] = double2{src[i][q0], src[i][q1]};
       }
   };
+  // operator and data array of product p
+  auto op_of = [](int p) { return NF == 3 ? p >= 5 : p == 3; };
+  auto data_of = [](int p) { return NF == 3 ? (p < 2 ? p : p < 5 ? p + 1 : p - 5) : p; };
   auto mac = [&](int g0, const Chunk& x) {
 #pragma unroll
-    for (int h = 0; h < CH; ++h)
+    for (int h = 0; h < CH; ++h) {
+      const int k = (g0 + h) * 8 + 2 * lk;
+      double2 d[ND][2];
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int k = (g0 + h) * 8 + 2 * lk;
+      for (int i = 0; i < ND; ++i)
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
-          const int K = p == 3 ? Kd[c] : Kb[c];
-          const double2 o = x.o[p == 3 ? 1 : 0][c][h];
-          const double v0 = k < K ? x.d[p][c][h].x : 0.0, v1 = k + 1 < K ? x.d[p][c][h].y : 0.0;
+        for (int c = 0; c < 2; ++c)
+          d[i][c] = double2{k < Kp[c] ? x.d[i][c][h].x : 0.0, k + 1 < Kp[c] ? x.d[i][c][h].y : 0.0};
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const double2 o = x.o[op_of(p) ? 1 : 0][c][h];
+          const bool odd = (c ^ (op_of(p) ? d0 : b0)) != 0;
+          const double v0 = odd ? d[data_of(p)][1].x : d[data_of(p)][0].x, v1 = odd ? d[data_of(p)][1].y : d[data_of(p)][0].y;
           acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.x, v0, acc[p][c], 0, 0, 0);
           acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.y, v1, acc[p][c], 0, 0, 0);
         }
-      }
+    }
   };
   Chunk x, y;
   const int nch = G / (4 * CH), top = G - CH, g0 = wid * nch * CH;
@@ -357,46 +389,36 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
     mac(g0 + (n + 1) * CH, y);
   }
   if (n < nch) mac(g0 + n * CH, x);
-  __shared__ v4d part[2][8][64];
-  auto put = [&](int s) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) part[s][e][lane] = acc[e >> 1][e & 1];
-  };
-  auto add = [&](int s) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e >> 1][e & 1] += part[s][e][lane];
-  };
-  if (wid & 1) put(wid >> 1);
-  __syncthreads();
-  if (!(wid & 1)) add(wid >> 1);
-  __syncthreads();
-  if (wid == 2) put(0);
-  __syncthreads();
-  if (wid != 0) return;
-  add(0);
   const int ny = a.bs.rows;
-  double* C = a.C + a.stride * (f * a.nb + b);
-  const double *fx = a.fx + a.sf * b, *fy = a.fy + a.sf * b;
+  double res[NP][2];
+  __shared__ double part[8 * 16 * 64];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
+  for (int h = 0; h < NP / 4; ++h) {  // four products at a time through LDS
+    if (h) __syncthreads();
+    add_quarters<8>(part, wid, lane, [&](int e, int r) { return acc[4 * h + (e >> 1)][e & 1][r]; },
+                    [&](int e, double v) { res[4 * h + (e >> 1)][e & 1] = v; });
+  }
+  const int m = m0 + 4 * wid + lk, nn = n0 + lr;
+  if (m >= a.bs.M[0] || nn >= N) return;
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
 #pragma clang fp contract(off)
-    const int m = m0 + 4 * r + lk, nn = n0 + lr;
-    if (m >= a.bs.M[0] || nn >= N) continue;
+    const int row = side ? ny - 1 - m : m;
+    if (side && row == m) continue;
+    double v[NP];
 #pragma unroll
-    for (int side = 0; side < 2; ++side) {
-      const int row = side ? ny - 1 - m : m;
-      if (side && row == m) continue;
-      double v[4];
+    for (int p = 0; p < NP; ++p) v[p] = side ? res[p][0] - res[p][1] : res[p][0] + res[p][1];
+    const size_t at = (size_t)row * N + nn;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) v[p] = side ? acc[p][0][r] - acc[p][1][r] : acc[p][0][r] + acc[p][1][r];
-      const size_t at = (size_t)row * N + nn;
-      double q = v[2] * v[0];
-      q = q + v[3] * v[1];
-      if (f == 2) {
-        q = q + v[0] * fx[at];
-        q = q + v[1] * fy[at];
+    for (int i = 0; i < NF; ++i) {
+      const int ff = NF == 3 ? i : f;
+      double q = (NF == 3 ? v[2 + i] : v[2]) * v[0];
+      q = q + (NF == 3 ? v[5 + i] : v[3]) * v[1];
+      if (ff == 2) {
+        q = q + v[0] * a.fx[a.sf * b + at];
+        q = q + v[1] * a.fy[a.sf * b + at];
       }
-      C[at] = q;
+      a.C[a.stride * (ff * a.nb + b) + at] = q;
     }
   }
 }
@@ -474,30 +496,38 @@ int xop_groups(int K) {
   return 4 * ((q + best - 1) / best * best);
 }
 
+void conv_products(hipStream_t s, const ConvArgs& a) {
+  if (a.bs.kind != XOP_FOLD_OUT || a.bds.kind != XOP_FOLD_OUT || a.bs.groups != a.bds.groups ||
+      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.f0 < 0 || a.f1 > 3 || a.f0 >= a.f1 || a.nx < 1 || a.nb < 1)
+    throw std::invalid_argument("conv_products: bad arguments");
+  if (a.bs.rstep != 2 || a.bds.rstep != 2) throw std::invalid_argument("conv_products: bad operators");
+  const int tx = (a.nx + 15) / 16, ty = (a.bs.M[0] + 15) / 16;
+  const long tiles = (long)tx * ty * a.nb;
+  // the three fields in one block where their tiles, times groups of 8 k values, fill the chip anyway
+  // (one / three fields per block: 128^2, 1 instance (256): 5.7 / 8.9 us, 3 (768): 10.0 / 9.4; 192^2,
+  // 1 (864): 7.6 / 10.8; 64^2, 36 (1,152): 10.6 / 11.0; 96^2, 12 (1,728): 14.8 / 9.1; 257^2, 1 (2,448):
+  // 17.7 / 15.3; 128^2, 36 (9,216): 61 / 40).  A wavefront per tile with the whole k range is no faster
+  // (192^2, 36: 85 us against 100, but 32 against 38 at 12 and 11 against 30 at 3).
+  const bool three = a.f0 == 0 && a.f1 == 3 && tiles * a.bs.groups >= 1200;
+  const long total = tiles * (three ? 1 : a.f1 - a.f0);
+  if (total > 0x7fffffffL) throw std::invalid_argument("conv_products: too many tiles");
+  const dim3 grid((unsigned)total), block(256);
+  if (three) RBC_LAUNCH((conv_kernel<1, 3>), grid, block, 0, s, a, tx, ty);
+  else if (a.bs.groups / 4 % 2 == 0) RBC_LAUNCH((conv_kernel<2, 1>), grid, block, 0, s, a, tx, ty);
+  else RBC_LAUNCH((conv_kernel<1, 1>), grid, block, 0, s, a, tx, ty);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) throw std::runtime_error(std::string("conv_products: ") + hipGetErrorString(e));
+}
+
 // The tile follows from the launch's size, 16 x 16 tiles times groups of 8 k values (twice when
 // folding out), us per launch on MI355X in a graph of such launches, 16 x 16 against 32 x 16 with the
 // k range split over a block's four wavefronts, and the staged kernel it replaces (full operator):
 //   128^2 x 12 entries, blocks (6,144):   3.41 / 3.51  (5.65)     192^2 x 3 (5,184):  3.54 / 3.74  (7.38)
 //   128^2 x 36 (18,432):                  5.76 / 5.34  (9.04)     257^2 x 3 (22,032): 6.50 / 5.81  (10.3)
 //   192^2 x 36 (62,208):                  12.3 / 10.2  (19.0)     257^2 x 36 (264,384): 36.8 / 28.8  (45.6)
-//   64^2 x 3 (384): 2.67 / 2.79 (4.00), of which 1.66 is an empty launch.
+//   64^2 x 3 (384): 2.47 / 2.79 (4.00), of which 1.66 is an empty launch.
 // Beyond a million the wavefronts of a block take a tile of their own each, 64 x 64 together, which
 // halves the loads per product: 510^2 x 64 (2.1 million) 179 us, 47 TFLOP/s, against 195 us.
-void conv_products(hipStream_t s, const ConvArgs& a) {
-  if (a.bs.kind != XOP_FOLD_OUT || a.bds.kind != XOP_FOLD_OUT || a.bs.groups != a.bds.groups ||
-      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.f0 < 0 || a.f1 > 3 || a.f0 >= a.f1 || a.nx < 1 || a.nb < 1)
-    throw std::invalid_argument("conv_products: bad arguments");
-  const int tx = (a.nx + 15) / 16, ty = (a.bs.M[0] + 15) / 16;
-  const long total = (long)tx * ty * a.nb * (a.f1 - a.f0);
-  if (total > 0x7fffffffL) throw std::invalid_argument("conv_products: too many tiles");
-  const dim3 grid((unsigned)total), block(256);
-  const int q = a.bs.groups / 4;  // chunks of two groups (the registers of four products in flight)
-  if (q % 2 == 0) RBC_LAUNCH(conv_kernel<2>, grid, block, 0, s, a, tx, ty);
-  else RBC_LAUNCH(conv_kernel<1>, grid, block, 0, s, a, tx, ty);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) throw std::runtime_error(std::string("conv_products: ") + hipGetErrorString(e));
-}
-
 static void xgemm_any(hipStream_t s, const XGemm* in, int ng, bool transposed) {
   if (ng < 1 || ng > XGEMM_GROUPS) throw std::invalid_argument("xgemm: bad group count");
   XGemm groups[XGEMM_GROUPS];
