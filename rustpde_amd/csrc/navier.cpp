@@ -632,7 +632,7 @@ class Navier {
   // rows of THAT_BC, GXX and GYY (spectral, [rows, ny]) before which every value is +0.0
   int bc_rows = 0;
   // workspaces
-  DBuf THAT, UXP, UYP, A, G, CONV, CV, RHS, DIV, W1, W2, W3, W4, W9, RED;
+  DBuf THAT, UXP, UYP, A, G, CONV, CV, RHS, DIV, W1, W2, W3, W4, W9, RED, NRM;
   std::vector<double> wx_dx, wy_dx;  // cell widths of `field` (unscaled, field.rs:135-163)
   double len0 = 0, len1 = 0;
   DBuf DX0, DX1;
@@ -992,6 +992,7 @@ class Navier {
     BC.alloc((size_t)R * 2);
     BCv.alloc((size_t)nx * ny);
     RED.alloc(std::max(ny, 8) + 300);
+    NRM.alloc(SUM_SQUARES_PART);
     // solvers
     const double cv[2] = {dt * nu / std::pow(scale[0], 2.0), dt * nu / std::pow(scale[1], 2.0)};
     const double ck[2] = {dt * ka / std::pow(scale[0], 2.0), dt * ka / std::pow(scale[1], 2.0)};
@@ -1023,6 +1024,7 @@ class Navier {
   }
   ~Navier() {
     drop_graph();
+    if (norm_host) (void)hipHostFree(norm_host);
     if (st && owns_stream) (void)hipStreamDestroy(st);
   }
 
@@ -1406,11 +1408,8 @@ class Navier {
     else
       for (int f = 0; f < 3; ++f) fn(f, f + 1);
   }
-  void update_confined() {
-    const Solver &s0 = *solver[0], &s2 = *solver[2], &sp = *solver[3];
-    const int mx_ = bx_u.m, my = by_u.m;
-    const long po = pair_off(), d = dstr();
-    const bool dct = confined_dct(), grp = nb > 1;
+  ConfinedRows confined_rows() {
+    const long po = pair_off();
     ConfinedRows a{};
     a.U = UX.p;
     a.RHS = RHS.p;
@@ -1431,17 +1430,25 @@ class Navier {
     a.sy = stencil_band(by_u).coef.p;
     a.syp = stencil_band(by_phi).coef.p;
     a.tdma = tdma_tables(by_u).tabp.p;
-    a.nuarr = grp ? NUARR.p : nullptr;
+    a.nuarr = nb > 1 ? NUARR.p : nullptr;
     a.nx = nx;
     a.ny = ny;
-    a.mx = mx_;
-    a.my = my;
+    a.mx = bx_u.m;
+    a.my = by_u.m;
     a.field = po;
-    a.stride = d;
+    a.stride = dstr();
     a.dt = dt;
     a.inv_dt = 1.0 / dt;
     a.inv_scy = 1.0 / scale[1];
     a.nu = nu;
+    return a;
+  }
+  void update_confined() {
+    const Solver &s0 = *solver[0], &s2 = *solver[2], &sp = *solver[3];
+    const int mx_ = bx_u.m, my = by_u.m;
+    const long po = pair_off(), d = dstr();
+    const bool dct = confined_dct(), grp = nb > 1;
+    ConfinedRows a = confined_rows();
     const double pts = (double)nx * ny * nb;
     // x transforms of the fields' values and x derivatives, and d/dx pres
     const PackedOp &bs = X.packed(bx_u, "BS"), &bst = X.packed(bx_t, "BS"), &bds = X.packed(bx_u, "BDS"),
@@ -2444,11 +2451,29 @@ class Navier {
     HIPCHECK(hipMemcpy(STA[which].p, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice));
   }
   double div_norm() {
-    divergence(G.p);
     const long no = (long)rows_ortho(bx_u) * ny;
-    dot_and_norm(st, nullptr, nullptr, 0, G.p, no, RED.p);
-    std::vector<double> r = RED.download(2);
-    return std::sqrt(r[1]);
+    // one product and one row kernel in place of five launches (not an ensemble's instance, whose ux
+    // and uy lie in slabs of their group)
+    if (nb == 1 && UY.p == UX.p + pair_off() && confined_fused_ok()) {
+      XGemm g = xgemm_of(X.packed(bx_u, "DS"), UX.p, W2.p, by_u.m, 1, 0, 0);
+      XGEMM(&g, 1);
+      ConfinedRows a = confined_rows();
+      a.TX = W2.p;
+      a.DIV = G.p;
+      a.f1 = 2;
+      div_rows(st, a, 1);
+    } else {
+      divergence(G.p);
+    }
+    return std::sqrt(read_norm(G.p, no));
+  }
+  // sum of squares of n device values, formed into pinned host memory: no copy follows the kernel
+  double* norm_host = nullptr;
+  double read_norm(const double* v, long n) {
+    if (!norm_host) HIPCHECK(hipHostMalloc(&norm_host, 2 * sizeof(double)));
+    sum_squares(st, v, n, NRM.p, norm_host);
+    HIPCHECK(hipStreamSynchronize(st));
+    return *norm_host;
   }
 };
 

@@ -464,60 +464,47 @@ void col_weighted_sum(hipStream_t s, const double* v, int n0, int n1, const doub
   check_launch("col_weighted_sum");
 }
 
-// out[0] = sum a w (one block; n is small), out[1] = sum b^2 (grid-stride partial sums
-// per block into part[], then reduced in block 0 by a second launch)
-__global__ void dot_kernel(const double* __restrict__ a, const double* __restrict__ w, int n, double* __restrict__ out) {
+// The partial sums are added by the last block to arrive, and the result may lie in pinned host memory:
+// one launch in place of three operations (two launches and a copy to pageable memory).  Launches bound
+// it: a confined 64^2 run under integrate(), which tests exit() after each step, takes 73 us per step
+// (101 before, with the divergence in five launches).  The counter, at part[NSUM], returns to zero for
+// the next call.
+constexpr int NSUM = SUM_SQUARES_PART - 1;
+__global__ __launch_bounds__(256) void sum_squares_kernel(const double* __restrict__ b, long n, double* __restrict__ part,
+                                                          double* __restrict__ out) {
   __shared__ double red[256];
-  const int t = threadIdx.x;
-  double s = 0.0;
-  for (int i = t; i < n; i += 256) s += a[i] * w[i];
-  red[t] = s;
-  __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
-    if (t < h) red[t] += red[t + h];
-    __syncthreads();
-  }
-  if (t == 0) out[0] = red[0];
-}
-__global__ void sumsq_partial_kernel(const double* __restrict__ b, long nb, double* __restrict__ part) {
-  __shared__ double red[256];
+  __shared__ bool last;
   const int t = threadIdx.x;
   double q = 0.0;
-  for (long i = (long)blockIdx.x * 256 + t; i < nb; i += (long)gridDim.x * 256) q += b[i] * b[i];
+  for (long i = (long)blockIdx.x * 256 + t; i < n; i += (long)gridDim.x * 256) q += b[i] * b[i];
   red[t] = q;
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
     if (t < h) red[t] += red[t + h];
     __syncthreads();
   }
-  if (t == 0) part[blockIdx.x] = red[0];
-}
-__global__ void sum_kernel(const double* __restrict__ part, int np, double* __restrict__ out) {
-  __shared__ double red[256];
-  const int t = threadIdx.x;
-  double q = 0.0;
-  for (int i = t; i < np; i += 256) q += part[i];
-  red[t] = q;
+  unsigned* count = reinterpret_cast<unsigned*>(part + NSUM);
+  if (t == 0) {
+    __hip_atomic_store(part + blockIdx.x, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  red[t] = t < (int)gridDim.x ? __hip_atomic_load(part + t, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
     if (t < h) red[t] += red[t + h];
     __syncthreads();
   }
-  if (t == 0) *out = red[0];
+  if (t == 0) {
+    *out = red[0];
+    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
-void dot_and_norm(hipStream_t s, const double* a, const double* w, int n, const double* b, long nb, double* out) {
-  if (a) {
-    RBC_LAUNCH(dot_kernel, dim3(1), dim3(256), 0, s, a, w, n, out);
-    check_launch("dot");
-  }
-  if (b) {
-    // partial sums land in out[2 .. 2 + 256); the caller's buffer holds >= 258 doubles
-    const int np = 256;
-    RBC_LAUNCH(sumsq_partial_kernel, dim3(np), dim3(256), 0, s, b, nb, out + 2);
-    check_launch("sumsq_partial");
-    RBC_LAUNCH(sum_kernel, dim3(1), dim3(256), 0, s, out + 2, np, out + 1);
-    check_launch("sum");
-  }
+void sum_squares(hipStream_t s, const double* b, long n, double* part, double* out) {
+  const unsigned blocks = n < 256L * NSUM ? blocks_for(n > 0 ? n : 1, 256) : NSUM;
+  RBC_LAUNCH(sum_squares_kernel, dim3(blocks), dim3(256), 0, s, b, n, part, out);
+  check_launch("sum_squares");
 }
 
 // --------------------------------------------------------------------- layout changes

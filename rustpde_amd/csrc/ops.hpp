@@ -230,9 +230,10 @@ void ew_update_pres_group(hipStream_t s, double* p, const double* div, const dou
 
 // Weighted column sums: out[j] = sum_i v[i, j] * w[i]  (i sequential, as average.rs:25-34)
 void col_weighted_sum(hipStream_t s, const double* v, int n0, int n1, const double* w, double* out);
-// out[0] = sum_j a[j] * w[j] if a, out[1] = sum of squares of b[0..nb) if b; out must
-// hold >= 258 doubles (out[2..258) receives per-block partial sums)
-void dot_and_norm(hipStream_t s, const double* a, const double* w, int n, const double* b, long nb, double* out);
+// *out (device or pinned host memory) = sum of squares of b[0..n); part holds SUM_SQUARES_PART doubles,
+// zero before the first call and used by one call at a time
+constexpr int SUM_SQUARES_PART = 257;
+void sum_squares(hipStream_t s, const double* b, long n, double* part, double* out);
 // v = sqrt(a^2 + b^2) * f
 void ew_solid_damp(hipStream_t s, double* conv, const double* mask, const double* q, const double* bc,
                    const double* val, double c, long n);
