@@ -626,7 +626,7 @@ class Navier {
   DBuf Tv, UXv, UYv, P0v, P1v, BCv;  // physical
   // constants derived from fieldbc
   DBuf THAT_BC, DTBCX, DTBCY, GXX, GYY;
-  DBuf BCXT, BCYT;  // DTBCX, DTBCY transposed (confined: the transposed convective products)
+  DBuf BCXT, BCYT;  // DTBCX, DTBCY transposed, for the transposed convective products
   // the physical fieldbc gradient: d/dx identically zero, d/dy the same in every x row
   bool bc_dx_zero = false, bc_dy_xconst = false;
   // rows of THAT_BC, GXX and GYY (spectral, [rows, ny]) before which every value is +0.0
@@ -987,7 +987,7 @@ class Navier {
                       &W4, &W9})
         b->alloc(full);
     }
-    if (!slabs && !per)
+    if (!slabs && (!per || dense_sizes()))
       for (DBuf* b : {&BCXT, &BCYT}) b->alloc(full);
     BC.alloc((size_t)R * 2);
     BCv.alloc((size_t)nx * ny);
@@ -1391,7 +1391,9 @@ class Navier {
   void XGEMMS(const XGemm* g, int ng, bool transposed) {
     bool one = ng > 1;
     for (int i = 0; i < ng; ++i)
-      one = one && g[i].op.groups == g[0].op.groups && (g[i].op.kind == XOP_BLOCKS || g[i].op.kind == XOP_FOLD_OUT);
+      one = one && g[i].op.groups == g[0].op.groups &&
+            (g[0].op.kind == XOP_DENSE ? g[i].op.kind == XOP_DENSE
+                                       : g[i].op.kind == XOP_BLOCKS || g[i].op.kind == XOP_FOLD_OUT);
     for (int i = 0; i < ng; i += one ? ng : 1) {
       double w = 0.0;
       for (int k = i; k < (one ? ng : i + 1); ++k)
@@ -1443,25 +1445,12 @@ class Navier {
     a.nu = nu;
     return a;
   }
-  void update_confined() {
-    const Solver &s0 = *solver[0], &s2 = *solver[2], &sp = *solver[3];
-    const int mx_ = bx_u.m, my = by_u.m;
+  // the convective terms in physical space from the x-transformed values and x derivatives of the three
+  // fields (dct: [nx, my], otherwise transposed), and their dealiased transforms along y into W2 [nx, ny]
+  void conv_y(double* val, double* der, bool dct) {
+    const int my = by_u.m;
     const long po = pair_off(), d = dstr();
-    const bool dct = confined_dct(), grp = nb > 1;
-    ConfinedRows a = confined_rows();
     const double pts = (double)nx * ny * nb;
-    // x transforms of the fields' values and x derivatives, and d/dx pres
-    const PackedOp &bs = X.packed(bx_u, "BS"), &bst = X.packed(bx_t, "BS"), &bds = X.packed(bx_u, "BDS"),
-                   &bdst = X.packed(bx_t, "BDS"), &ds = X.packed(bx_p, "DS");
-    double *val = dct ? W2.p : A.p, *der = W1.p;
-    const int ldt = dct ? my : nx;  // [nx, my], or transposed [my, nx]
-    each_field([&](int f0, int f1) {
-      XGemm g[3] = {field_op(bs, bst, UX.p, my, val, ldt, f0, f1), field_op(bds, bdst, UX.p, my, der, ldt, f0, f1),
-                    xgemm_of(ds, P0.p, G.p, ny, nb, d, d)};
-      g[2].plain = 1;
-      XGEMMS(g, f0 == 0 ? 3 : 2, !dct);
-    });
-    // products in physical space and their dealiased transforms along y, into W2 [nx, ny]
     if (dct) {
       const DBand& band = stencil_band(by_u);
       each_field([&](int f0, int f1) {
@@ -1500,6 +1489,26 @@ class Navier {
         XGEMMS(&g, 1, true);
       });
     }
+  }
+  void update_confined() {
+    const Solver &s0 = *solver[0], &s2 = *solver[2], &sp = *solver[3];
+    const int mx_ = bx_u.m, my = by_u.m;
+    const long po = pair_off(), d = dstr();
+    const bool dct = confined_dct(), grp = nb > 1;
+    ConfinedRows a = confined_rows();
+    const double pts = (double)nx * ny * nb;
+    // x transforms of the fields' values and x derivatives, and d/dx pres
+    const PackedOp &bs = X.packed(bx_u, "BS"), &bst = X.packed(bx_t, "BS"), &bds = X.packed(bx_u, "BDS"),
+                   &bdst = X.packed(bx_t, "BDS"), &ds = X.packed(bx_p, "DS");
+    double *val = dct ? W2.p : A.p, *der = W1.p;
+    const int ldt = dct ? my : nx;  // [nx, my], or transposed [my, nx]
+    each_field([&](int f0, int f1) {
+      XGemm g[3] = {field_op(bs, bst, UX.p, my, val, ldt, f0, f1), field_op(bds, bdst, UX.p, my, der, ldt, f0, f1),
+                    xgemm_of(ds, P0.p, G.p, ny, nb, d, d)};
+      g[2].plain = 1;
+      XGEMMS(g, f0 == 0 ? 3 : 2, !dct);
+    });
+    conv_y(val, der, dct);
     const PackedOp& fx = X.packed(bx_f, "Fdl");
     each_field([&](int f0, int f1) {
       const XGemm g = field_op(fx, fx, W2.p, ny, CV.p, ny, f0, f1);
@@ -1613,7 +1622,7 @@ class Navier {
     THAT_BC.upload(t);
     DTBCX.upload(hdx);
     DTBCY.upload(hdy);
-    if (!periodic) {
+    if (BCXT.p) {
       std::vector<double> tx(hdx.size()), ty(hdy.size());
       for (int i = 0; i < nx; ++i)
         for (int j = 0; j < ny; ++j) {
@@ -1859,10 +1868,38 @@ class Navier {
     yop(by_u, "BS", a, nx, out);
   }
   // ----------------------------------------------------------- batched periodic step
-  bool batch_ok() const {
-    return nb == 1 && use_batch && periodic && vel_same && use_fft && fft_supported(nx) && use_dct && cheb_y_supported(ny) &&
-           use_bands && fdma_rows_lds_supported(by_u.m, by_u.n) && tdma_rows_lds_supported(by_u.m) &&
-           by_phi.n == by_u.n;
+  bool batch_ok() {
+    const bool fast = use_fft && fft_supported(nx) && use_dct && cheb_y_supported(ny);
+    return nb == 1 && use_batch && periodic && vel_same && (fast || conv_dense_ok()) && use_bands &&
+           fdma_rows_lds_supported(by_u.m, by_u.n) && tdma_rows_lds_supported(by_u.m) && by_phi.n == by_u.n;
+  }
+  // A periodic grid without fast transforms along x, or along y on a short x axis: the convective terms
+  // by products with the dense x operators, the y stage as in the confined step.  160 x 129, 50
+  // steps and their output: 12.3 ms field by field (some 45 launches a step), 2.2 ms in seven.  (With fast x transforms and a longer
+  // x axis the dense products lose: 2 nx^2 operations per column against the transform's n log n.)
+  bool dense_sizes() const {
+    return periodic && (!fft_supported(nx) || (!cheb_y_supported(ny) && nx <= 256));
+  }
+  bool conv_dense_ok() {
+    if (!dense_sizes() || !use_fuse || solid_on || !xg_ok() || by_u.k != CD) return false;
+    for (const char* name : {"BS", "BDS"}) {
+      X.packed(bx_u, name);
+      if (!confined_dct() && Y.packed(by_u, name).op.kind != XOP_FOLD_OUT) return false;
+    }
+    X.packed(bx_f, "Fdl");
+    return confined_dct() || Y.packed(by_p, "Fdl").op.kind == XOP_FOLD_IN;
+  }
+  void conv_dense() {
+    const int my = by_u.m;
+    const bool dct = confined_dct();
+    double* val = dct ? W2.p : A.p;
+    XGemm g[2] = {xgemm_of(X.packed(bx_u, "BS"), UX.p, val, my, 3, (long)FS, (long)FS),
+                  xgemm_of(X.packed(bx_u, "BDS"), UX.p, W1.p, my, 3, (long)FS, (long)FS)};
+    g[0].ldc = g[1].ldc = dct ? my : nx;
+    XGEMMS(g, 2, !dct);
+    conv_y(val, W1.p, dct);
+    const XGemm f = xgemm_of(X.packed(bx_f, "Fdl"), W2.p, CV.p, ny, 3, (long)FS, (long)FS);
+    XGEMMS(&f, 1, false);
   }
   // irfft of `batch` slots [2 mx, cols] -> [nx, cols], (i k)^times / sc first
   void IRFFT_B(const double* in, double* out, int cols, int times, double sc, int batch) {
@@ -1898,8 +1935,11 @@ class Navier {
   void update_batched() {  // navier.rs:737-765 with the three fields' work batched
     const int my = by_u.m;
     const size_t F = FS;
+    const bool dense = dense_sizes(), mixed = this->mixed && !dense;  // no FP32 kernels of those sizes
     if (mixed) {
       conv_mixed();
+    } else if (dense) {
+      conv_dense();
     } else {
       conv_fp64();
     }

@@ -360,6 +360,16 @@ LMat axis_operator(const Basis& b, const std::string& name, ld sc) {
   if (b.k == FO) {
     if (name == "BS") return dft_c2r(n);
     if (name == "FS") return dft_r2c(n);
+    if (name == "BDS") {  // of i k / sc times the spectrum
+      const LMat a = dft_c2r(n);
+      LMat d(a.r, a.c);
+      for (int j = 0; j < n; ++j)
+        for (int k = 0; k < b.m; ++k) {
+          d(j, k) = a(j, b.m + k) * (ld)k / sc;
+          d(j, b.m + k) = -a(j, k) * (ld)k / sc;
+        }
+      return d;
+    }
     if (name == "Fdl") {
       LMat a = dft_r2c(n);
       const int cut = b.m * 2 / 3;

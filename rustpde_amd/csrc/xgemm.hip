@@ -467,6 +467,7 @@ template <bool TR>
 void launch_kind(hipStream_t s, const XGemm* groups, int ng, int kind, int tile, int ch) {
   if (ng > 1) {
     if (kind == XOP_FOLD_OUT) launch_chunk<XOP_FOLD_OUT, XGEMM_GROUPS, TR>(s, groups, tile, ch);
+    else if (kind == XOP_DENSE) launch_chunk<XOP_DENSE, XGEMM_GROUPS, TR>(s, groups, tile, ch);
     else launch_chunk<XOP_BLOCKS, XGEMM_GROUPS, TR>(s, groups, tile, ch);
     return;
   }
@@ -544,8 +545,7 @@ static void xgemm_any(hipStream_t s, const XGemm* in, int ng, bool transposed) {
   }
   if (ng > 1) {
     for (int i = 0; i < ng; ++i)
-      if (in[i].op.kind == XOP_DENSE || in[i].op.kind == XOP_FOLD_IN ||
-          (!out && in[i].op.kind != XOP_BLOCKS))
+      if (in[i].op.kind == XOP_FOLD_IN || (in[i].op.kind == XOP_DENSE) != (in[0].op.kind == XOP_DENSE))
         throw std::invalid_argument("xgemm: these operators do not share a launch");
     for (int i = ng; i < XGEMM_GROUPS; ++i) {  // an empty group
       groups[i] = groups[0];
