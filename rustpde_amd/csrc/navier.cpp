@@ -1873,15 +1873,18 @@ class Navier {
     return nb == 1 && use_batch && periodic && vel_same && (fast || conv_dense_ok()) && use_bands &&
            fdma_rows_lds_supported(by_u.m, by_u.n) && tdma_rows_lds_supported(by_u.m) && by_phi.n == by_u.n;
   }
-  // A periodic grid without fast transforms along x, or along y on a short x axis: the convective terms
-  // by products with the dense x operators, the y stage as in the confined step.  160 x 129, 50
-  // steps and their output: 12.3 ms field by field (some 45 launches a step), 2.2 ms in seven.  (With fast x transforms and a longer
-  // x axis the dense products lose: 2 nx^2 operations per column against the transform's n log n.)
+  // The convective terms by products with the dense x operators, the y stage as in the confined step,
+  // where there are no fast transforms (160 x 129, 50 steps and their output: 12.3 ms field by field in
+  // some 45 launches a step, 2.2 ms in seven) and on small grids, whose transforms are bound by their
+  // launches and passes: us per step by transforms / products on MI355X, 64 x 65 50.5 / 32.7, 128 x 129
+  // 51.9 / 37.5, 256 x 129 55.7 / 44.7, 256 x 257 57.3 / 58.5, 512 x 257 72 / 90, 512 x 513 89 / 132.
   bool dense_sizes() const {
-    return periodic && (!fft_supported(nx) || (!cheb_y_supported(ny) && nx <= 256));
+    return periodic && (!fft_supported(nx) || (nx <= 256 && (ny <= 200 || !cheb_y_supported(ny))));
   }
+  // the mixed step keeps its FP32 transforms where they exist
+  bool dense_step() const { return dense_sizes() && !(mixed && fft_supported(nx) && cheb_y_supported(ny)); }
   bool conv_dense_ok() {
-    if (!dense_sizes() || !use_fuse || solid_on || !xg_ok() || by_u.k != CD) return false;
+    if (!dense_step() || !use_fuse || solid_on || !xg_ok() || by_u.k != CD) return false;
     for (const char* name : {"BS", "BDS"}) {
       X.packed(bx_u, name);
       if (!confined_dct() && Y.packed(by_u, name).op.kind != XOP_FOLD_OUT) return false;
@@ -1935,7 +1938,7 @@ class Navier {
   void update_batched() {  // navier.rs:737-765 with the three fields' work batched
     const int my = by_u.m;
     const size_t F = FS;
-    const bool dense = dense_sizes(), mixed = this->mixed && !dense;  // no FP32 kernels of those sizes
+    const bool dense = conv_dense_ok(), mixed = this->mixed && !dense;
     if (mixed) {
       conv_mixed();
     } else if (dense) {

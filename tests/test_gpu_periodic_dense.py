@@ -1,9 +1,9 @@
-"""Periodic steps on grids without fast transforms along one axis or both (the convective terms by
-products with the dense x operators): even and odd row lengths, the y stage as products and (from 201
+"""Periodic steps whose convective terms are products with the dense x operators (small grids, and those
+without fast transforms along one axis or both): even and odd row lengths, the y stage as products and (from 201
 points of a fast length) as transforms, a fast x axis with a row length that has none.
 
 Oracle tolerance 1e-12 after 5 steps, as the other periodic steps of these lengths; the single-precision
-option has no kernels for these grids and leaves the step's bits as they are."""
+option has no kernels for the grids without fast transforms and leaves the step's bits as they are."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ from helpers import compare, init_pair, rel_err
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(12, 9), (22, 20), (30, 33), (34, 66), (64, 50), (36, 257), (100, 65), (256, 40)]
+SHAPES = [(12, 9), (22, 20), (30, 33), (34, 66), (64, 50), (36, 257), (100, 65), (256, 40), (64, 65), (256, 129)]
 
 
 def _fields(g):
@@ -29,6 +29,9 @@ def test_dense_periodic(oracle, shape):
         g, o = make(), oracle.Navier2D.new_periodic(nx, ny, 1e4, 1.0, 2e-3, 2.0)
         init_pair(g, o, nx, ny, True, 1e-2, 3, "gaussian", velocity=(0.1, 2.0, 1.0))
         if option == "mixed":
+            if shape in ((64, 65), (256, 129)):  # FP32 transforms there
+                g.close()
+                continue
             g.set_option(g.OPT_MIXED, 1)
         if option == "batch":
             g.set_option(g.OPT_BATCH, 0)
@@ -43,7 +46,8 @@ def test_dense_periodic(oracle, shape):
             assert abs(g.eval_nu() - o.eval_nu()) < 1e-12 * abs(o.eval_nu())
         out.append(_fields(g))
         g.close()
-    assert all(np.array_equal(a, b) for a, b in zip(out[0], out[1]))
-    for other in out[2:]:
+    if len(out) == 4:
+        assert all(np.array_equal(a, b) for a, b in zip(out[0], out.pop(1)))
+    for other in out[1:]:
         for a, b in zip(out[0], other):
             assert rel_err(a, b) < 1e-12
