@@ -196,6 +196,89 @@ __global__ __launch_bounds__(NT) void proj_rows_kernel(ConfinedRows a, int per_n
   chains::unstage_row<MAXQ>(buf, const_cast<double*>(a.U) + f * a.field + o + (long)r * m, true, m, tid, NT, true);
 }
 
+// One block per row and field (blockIdx.y).  PER: rows are split planes of a Fourier x axis.  The row's
+// derivatives along y (the residual twice, for uy also pres once) run as suffix sums in LDS.
+template <int SLICE, bool PER>
+__global__ __launch_bounds__(NT) void adjoint_rows_kernel(AdjointRows a) {
+#pragma clang fp contract(off)
+  extern __shared__ double buf[];
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), p = tid / WAVE;
+  const int r = blockIdx.x, f = blockIdx.y, n = a.ny, m = a.my, nx = a.rows;
+  constexpr int MAXQ = (2 * SLICE * WAVE + 8 + NT - 1) / NT;
+  const double* sx = f == 2 ? a.sxt : a.sxu;
+  const double x0 = PER ? 1.0 : sx[r], x1 = PER ? 0.0 : sx[nx + r];
+  const double bx0 = PER ? 1.0 : a.sxu[r], bx1 = PER ? 0.0 : a.sxu[nx + r];  // uy's taps for the buoyancy
+  const bool im = PER && r >= a.mx;
+  const double kk = PER ? (double)(im ? r - a.mx : r) / a.kscale : 0.0;
+  // to_ortho of a spectral field at (r, i)
+  auto taps = [&](const double* q, int i, double c0, double c1, double cy0, double cy1) {
+    if constexpr (PER) {
+      const double* row = q + (long)r * m;
+      return (i < m ? row[min(i, m - 1)] * cy0 : 0.0) + (i >= 2 ? row[i - 2] * cy1 : 0.0);
+    } else {
+      return xy_taps(q, a.mx, m, r, i, c0, c1, cy0, cy1);
+    }
+  };
+  const double* F = a.F + f * a.field;
+  double s[MAXQ], gp[MAXQ];
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {  // the residual in ortho space
+    const int i = tid + q * NT;
+    s[q] = gp[q] = 0.0;
+    if (i < n) s[q] = taps(F, i, x0, x1, a.sy[i], a.sy[n + i]);
+  }
+  if (f == 1) {  // d/dy pres
+    chains::stage_row<MAXQ>(buf, a.P0 + (long)r * n, true, n, tid, NT);
+    __syncthreads();
+    rowdiff::derive<SLICE>(buf, n, a.per, lane, p);
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * NT;
+      if (i < n) gp[q] = buf[pad(i + 2)] * a.inv_scy;
+    }
+    __syncthreads();
+  } else if (f == 0) {
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * NT;
+      if (i >= n) continue;
+      if constexpr (PER) gp[q] = (im ? a.P0[(long)(r - a.mx) * n + i] : -a.P0[(long)(r + a.mx) * n + i]) * kk;
+      else gp[q] = a.GX[(long)r * n + i];
+    }
+  }
+  if (tid < 2) buf[pad(tid)] = 0.0;
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int j = tid + q * NT + 2;
+    if (j < n + 6) buf[pad(j)] = s[q];
+  }
+  __syncthreads();
+  rowdiff::derive<SLICE>(buf, n, a.per, lane, p);
+  rowdiff::derive<SLICE>(buf, n, a.per, lane, p);
+  const double k = f == 2 ? a.ka : a.nu;
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int i = tid + q * NT;
+    if (i >= n) continue;
+    const double cy0 = a.sy[i], cy1 = a.sy[n + i];
+    const long j = f * a.field + (long)r * n + i;
+    double lx;
+    if constexpr (PER) {
+      lx = -(kk * kk) * s[q];
+    } else {
+      const double* row = a.LX + f * a.field + (long)r * m;
+      lx = (i < m ? row[min(i, m - 1)] * cy0 : 0.0) + (i >= 2 ? row[i - 2] * cy1 : 0.0);
+    }
+    const double ly = (buf[pad(i + 2)] * a.inv_scy) * a.inv_scy;
+    double v = taps(a.U + f * a.field, i, x0, x1, cy0, cy1);
+    if (f < 2) v = v - gp[q] * a.dt;
+    v = v + a.CV[j] * a.dt;
+    if (f == 2) v = v + taps(a.F + a.field, i, bx0, bx1, cy0, cy1) * a.dt;
+    v = v + (lx * a.dt) * k;
+    a.RHS[j] = v + (ly * a.dt) * k;
+  }
+}
+
 }  // namespace
 
 bool confined_rows_supported(int nx, int ny) {
@@ -237,6 +320,26 @@ void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure) {
   if (blocks == 0) return;
   RBC_CONFINED(proj_rows_kernel, per_n, blocks, a, per_n, per);
   check("proj_rows");
+}
+
+void adjoint_rows(hipStream_t s, const AdjointRows& in) {
+  AdjointRows a = in;
+  const bool fourier = !a.LX;
+  if (!row_ops_supported(a.ny) || a.my != a.ny - 2 || a.mx < 1 || a.rows != (fourier ? 2 * a.mx : a.mx + 2))
+    throw std::invalid_argument("adjoint_rows: unsupported sizes");
+  a.per = fdma_rows_lds_per(a.ny);
+  const dim3 grid((unsigned)a.rows, 3), block(NT);
+  const size_t lds = buf_len(a.ny) * sizeof(double);
+#define RBC_ADJOINT(SL)                                                                        \
+  do {                                                                                         \
+    if (fourier) RBC_LAUNCH((adjoint_rows_kernel<SL, true>), grid, block, lds, s, a);          \
+    else RBC_LAUNCH((adjoint_rows_kernel<SL, false>), grid, block, lds, s, a);                 \
+  } while (0)
+  if (a.per <= 4) RBC_ADJOINT(4);
+  else if (a.per <= 8) RBC_ADJOINT(8);
+  else RBC_ADJOINT(16);
+#undef RBC_ADJOINT
+  check("adjoint_rows");
 }
 
 }  // namespace rbc

@@ -700,7 +700,9 @@ class Navier {
   static constexpr int GRAPH_STEPS = 8;
   int eager_steps = 0;     // eager steps since the captured step was last dropped
   bool graph_gpres = false;  // the captured step reads d/dy pres left by the step before it
+  unsigned long set_ups = 0;  // counts the set-up changes: graphs captured before one are stale
   void drop_graph() {
+    ++set_ups;
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (gexec_k) (void)hipGraphExecDestroy(gexec_k);
     gexec = nullptr;
@@ -1490,8 +1492,36 @@ class Navier {
       });
     }
   }
+  void divergence_confined(ConfinedRows a, double* out) {
+    const XGemm g = xgemm_of(X.packed(bx_u, "DS"), UX.p, W2.p, by_u.m, nb, dstr(), dstr());
+    XGEMMS(&g, 1, false);
+    a.TX = W2.p;
+    a.DIV = out;
+    a.f0 = 0;
+    a.f1 = 2;
+    timer.begin(st, 3, 8.0 * (double)nx * ny * nb * 3.0);
+    div_rows(st, a, nb);
+    timer.end(st);
+  }
+  // pseudo pressure of DIV: eigen-transform, row systems, back-transform with the projection's x parts;
+  // then the projection of ux and uy and the pressure update (of fields 0 and 1 of a)
+  void pressure_confined(const ConfinedRows& a) {
+    const Solver& sp = *solver[3];
+    const long po = pair_off(), d = dstr();
+    const XGemm f = xgemm_of(sp.pfp, DIV.p, A.p, ny, nb, d, d);
+    XGEMMS(&f, 1, false);
+    ROWSF(A.p, ny, W1.p, by_phi.m, sp.pf.rows, sp);
+    XGemm g[3] = {xgemm_of(sp.pbp, W1.p, P1.p, by_phi.m, nb, d, d),
+                  xgemm_of(*sp.leftp[0], W1.p, CV.p, by_phi.m, nb, d, d),
+                  xgemm_of(*sp.leftp[1], W1.p, CV.p + po, by_phi.m, nb, d, d)};
+    g[0].zero00 = 1;
+    XGEMMS(g, 3, false);
+    timer.begin(st, 3, 8.0 * (double)nx * ny * nb * 9.0);
+    proj_rows(st, a, nb, true);
+    timer.end(st);
+  }
   void update_confined() {
-    const Solver &s0 = *solver[0], &s2 = *solver[2], &sp = *solver[3];
+    const Solver &s0 = *solver[0], &s2 = *solver[2];
     const int mx_ = bx_u.m, my = by_u.m;
     const long po = pair_off(), d = dstr();
     const bool dct = confined_dct(), grp = nb > 1;
@@ -1546,20 +1576,7 @@ class Navier {
     timer.begin(st, 3, 8.0 * pts * 3.0);
     div_rows(st, a, nb);
     timer.end(st);
-    // pseudo pressure: eigen-transform, row systems, back-transform with the projection's x parts
-    {
-      const XGemm f = xgemm_of(sp.pfp, DIV.p, A.p, ny, nb, d, d);
-      XGEMMS(&f, 1, false);
-      ROWSF(A.p, ny, W1.p, by_phi.m, sp.pf.rows, sp);
-      XGemm g[3] = {xgemm_of(sp.pbp, W1.p, P1.p, by_phi.m, nb, d, d),
-                    xgemm_of(*sp.leftp[0], W1.p, CV.p, by_phi.m, nb, d, d),
-                    xgemm_of(*sp.leftp[1], W1.p, CV.p + po, by_phi.m, nb, d, d)};
-      g[0].zero00 = 1;
-      XGEMMS(g, 3, false);
-    }
-    timer.begin(st, 3, 8.0 * pts * 9.0);
-    proj_rows(st, a, nb, true);
-    timer.end(st);
+    pressure_confined(a);
     time += dt;
   }
 
@@ -2132,6 +2149,15 @@ class Navier {
     const double frows = conv3_ldf() ? (double)nx : 1.0;
     return bi * nx * 6.0 * by_u.m + bo * nx * 3.0 * ny + 8.0 * frows * ny * (bc_dx_zero ? 1.0 : 2.0);
   }
+  PressureArgs pressure_args(double visc) {
+    const Solver& sp = *solver[3];
+    PressureArgs pa{UX.p, UY.p, P0.p, P1.p, stencil_band(by_u).coef.p, stencil_band(by_phi).coef.p, sp.pybp.p,
+                    sp.diagp.p, tdma_tables(by_u).tabp.p, mx(), ny, by_u.m, 0, 0, scale[0], 1.0 / scale[1], visc,
+                    1.0 / dt};
+    pa.su_kind = by_u.k == CD ? 1 : by_u.k == CN ? 2 : 0;
+    pa.sp_kind = by_phi.k == CD ? 1 : by_phi.k == CN ? 2 : 0;
+    return pa;
+  }
   void solves_and_pressure() {
     const int my = by_u.m, R2 = 2 * mx();
     const size_t F = FS;
@@ -2151,12 +2177,7 @@ class Navier {
     timer.end(st);
     // projection (navier.rs:683-721)
     if (pressure_fused_ok()) {
-      const Solver& sp = *solver[3];
-      PressureArgs pa{UX.p, UY.p, P0.p, P1.p, stencil_band(by_u).coef.p, stencil_band(by_phi).coef.p, sp.pybp.p,
-                      sp.diagp.p, tdma_tables(by_u).tabp.p, mx(), ny, by_u.m, 0, 0, scale[0], 1.0 / scale[1], nu,
-                      1.0 / dt};
-      pa.su_kind = by_u.k == CD ? 1 : by_u.k == CN ? 2 : 0;
-      pa.sp_kind = by_phi.k == CD ? 1 : by_phi.k == CN ? 2 : 0;
+      PressureArgs pa = pressure_args(nu);
       pa.dP = G.p + FS;  // d/dy of the new pres for the next step
       if (fold_temp) {
         pa.rows_R = RHS.p + 2 * F;
@@ -2498,13 +2519,7 @@ class Navier {
     // one product and one row kernel in place of five launches (not an ensemble's instance, whose ux
     // and uy lie in slabs of their group)
     if (nb == 1 && UY.p == UX.p + pair_off() && confined_fused_ok()) {
-      XGemm g = xgemm_of(X.packed(bx_u, "DS"), UX.p, W2.p, by_u.m, 1, 0, 0);
-      XGEMM(&g, 1);
-      ConfinedRows a = confined_rows();
-      a.TX = W2.p;
-      a.DIV = G.p;
-      a.f1 = 2;
-      div_rows(st, a, 1);
+      divergence_confined(confined_rows(), G.p);
     } else {
       divergence(G.p);
     }
@@ -3086,7 +3101,8 @@ class Adjoint {
   std::unique_ptr<Navier> ad, ns;
   DBuf F1[3];        // smoothed residuals [1] of temp, ux, uy (spectral, the fields' layout)
   DBuf UNS[3];       // unsmoothed residuals (fields_unsmoothed: ux, uy, temp; ortho space)
-  DBuf U, V, TP;     // physical ux, uy, temp of the step start
+  DBuf U, V, TP;     // physical ux, uy, temp of the step start (transposed in the fused iteration)
+  DBuf F1B, UNSB, PV;  // the above, in the order ux, uy, temp (slots FS apart)
   DBuf B, LXX, LYY;  // buoyancy and the residuals' second derivatives (ortho space)
   double time = 0.0, dt = 0.0, res_tol = 1e-8;  // RES_TOL (:114)
 
@@ -3099,10 +3115,19 @@ class Adjoint {
     n.solver[0] = std::shared_ptr<Solver>(make_solver(HHOLTZ, n.bx_u, n.by_u, cs));
     n.solver[1] = std::shared_ptr<Solver>(make_solver(HHOLTZ, n.bx_u, n.by_u, cs));
     n.solver[2] = std::shared_ptr<Solver>(make_solver(HHOLTZ, n.bx_t, n.by_u, cs));
-    for (DBuf* b : {&F1[0], &F1[1], &F1[2], &UNS[0], &UNS[1], &UNS[2], &U, &V, &TP, &B, &LXX, &LYY}) b->alloc(n.FS);
+    for (DBuf* b : {&F1B, &UNSB, &PV}) b->alloc(3 * n.FS);
+    DBuf* views[3][3] = {{&F1[1], &F1[2], &F1[0]}, {&UNS[0], &UNS[1], &UNS[2]}, {&U, &V, &TP}};
+    for (int j = 0; j < 3; ++j) {
+      views[0][j]->view(F1B.p + j * n.FS, n.FS);
+      views[1][j]->view(UNSB.p + j * n.FS, n.FS);
+      views[2][j]->view(PV.p + j * n.FS, n.FS);
+    }
+    for (DBuf* b : {&B, &LXX, &LYY}) b->alloc(n.FS);
   }
   ~Adjoint() {
     if (ad) (void)hipStreamSynchronize(ad->st);
+    drop_graph();
+    if (norms_host) (void)hipHostFree(norms_host);
     ns.reset();  // shares ad's stream
   }
   long spec_len(const Basis& bx) const { return (long)ad->rows_spec(bx) * ad->by_u.m; }
@@ -3193,7 +3218,277 @@ class Adjoint {
     ew_adj_rhs(n.st, n.RHS.p, n.A.p, nullptr, n.CV.p, B.p, LXX.p, LYY.p, dt, n.ka, ortho_len());
     from_ortho_into(n.bx_t, n.T.p);
   }
-  void update() {  // Integrate::update (navier_adjoint.rs:760-790)
+  // ------------------------------------------------------------- fused iteration
+  // The three fields in one launch each: the residuals' smoothers, their x-transformed values and
+  // derivatives once (the terms above form them 14 times), the terms in one kernel, the right-hand
+  // sides by rows; then the step's own divergence, pressure and projection kernels.  Launches bound it: 96 x
+  // 97, ten iterations, their norms and fields take 1.46 ms as replays of a graph of some 33 launches an
+  // iteration, 7.33 ms with some 110 launches term by term.
+  DBuf SMF, SMB, BCT, LX;   // smoothers' packed products (pf of the three; pb negated), bc transposed
+  bool packed3[2] = {};     // the three operators share their classes: one launch
+  bool ready = false;
+  unsigned long made[2] = {};  // set-ups of ad and ns that the above and the graph belong to
+  hipGraphExec_t gexec = nullptr;
+  bool graph_gpres = false;  // the captured step reads d/dy pres left by the one before it
+  void drop_graph() {
+    if (gexec) (void)hipGraphExecDestroy(gexec);
+    gexec = nullptr;
+  }
+  static bool same3(const PackedOp& a, const PackedOp& b, const PackedOp& c) {
+    return Navier::same_classes(a.op, b.op) && Navier::same_classes(a.op, c.op) && a.buf.n == b.buf.n &&
+           a.buf.n == c.buf.n;
+  }
+  // dense x products and y products of one parity: beyond 512 Fourier points the transforms win
+  bool fused_ok() {
+    Navier& n = *ad;
+    if (!n.use_batch || !n.use_fuse || !n.use_bands || !n.xg_ok() || n.mixed || n.by_u.k != CD || n.by_phi.k != CN) return false;
+    if (!row_ops_supported(n.ny) || !tdma_rows_lds_supported(n.by_u.m)) return false;
+    for (int i = 0; i < 4; ++i)
+      if (!fdma_rows_lds_supported(n.solver[i]->m, n.ny) || n.solver[i]->pyb.mi != n.ny) return false;
+    for (const char* name : {"BS", "BDS"})
+      if (n.Y.packed(n.by_u, name).op.kind != XOP_FOLD_OUT) return false;
+    if (n.Y.packed(n.by_p, "Fdl").op.kind != XOP_FOLD_IN) return false;
+    if (n.periodic) {
+      if (n.nx > 512) return false;
+      for (int i = 0; i < 4; ++i)
+        if (n.solver[i]->has_fb || n.solver[i]->nsets != n.mx()) return false;
+      return true;
+    }
+    if (!confined_rows_supported(n.nx, n.ny) || n.bx_u.k != CD || n.bx_phi.k != CN || n.bx_t.m != n.bx_u.m ||
+        n.solver[3]->leftp.size() != 2)
+      return false;
+    for (int i = 0; i < 3; ++i)
+      if (!n.solver[i]->has_fb || n.solver[i]->nsets != n.solver[0]->nsets) return false;
+    for (const char* name : {"BS", "BDS", "DDS", "FO"})
+      if (!Navier::same_classes(n.X.packed(n.bx_u, name).op, n.X.packed(n.bx_t, name).op)) return false;
+    return n.X.packed(n.bx_u, "BS").op.kind == XOP_FOLD_OUT && n.X.packed(n.bx_u, "BDS").op.kind == XOP_FOLD_OUT;
+  }
+  void make_ready() {
+    Navier& n = *ad;
+    HIPCHECK(hipStreamSynchronize(n.st));
+    std::vector<double> bc = n.BCv.download((size_t)n.nx * n.ny), t(bc.size());
+    for (int i = 0; i < n.nx; ++i)
+      for (int j = 0; j < n.ny; ++j) t[(size_t)j * n.nx + i] = bc[(size_t)i * n.ny + j];
+    BCT.upload(t);
+    if (!n.periodic) {
+      if (LX.n < 3 * n.FS) LX.alloc(3 * n.FS);
+      for (int q = 0; q < 2; ++q) {
+        const PackedOp* p[3];
+        for (int i = 0; i < 3; ++i) p[i] = q ? &n.solver[i]->pbp : &n.solver[i]->pfp;
+        packed3[q] = same3(*p[0], *p[1], *p[2]);
+        DBuf& slab = q ? SMB : SMF;
+        if (slab.n != 3 * p[0]->buf.n) slab.alloc(3 * std::max({p[0]->buf.n, p[1]->buf.n, p[2]->buf.n}));
+        const size_t each = slab.n / 3;
+        for (int i = 0; i < 3; ++i) {
+          std::vector<double> v = p[i]->buf.download(p[i]->buf.n);
+          if (q)
+            for (double& x : v) x = -x;
+          HIPCHECK(hipMemcpy(slab.p + i * each, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice));
+        }
+      }
+    }
+    made[0] = ad->set_ups;
+    made[1] = ns->set_ups;
+    ready = true;
+  }
+  // the smoothers' products p_i (in `slab`) of the three fields
+  void smooth(int q, const double* in, int N, double* out) {
+    Navier& n = *ad;
+    const DBuf& slab = q ? SMB : SMF;
+    const size_t each = slab.n / 3;
+    const long F = (long)n.FS;
+    for (int i = 0; i < (packed3[q] ? 1 : 3); ++i) {
+      const PackedOp& p = q ? n.solver[i]->pbp : n.solver[i]->pfp;
+      XGemm g = xgemm_of(p, in + i * F, out + i * F, N, packed3[q] ? 3 : 1, F, F);
+      for (int c = 0; c < 2; ++c) {
+        g.op.a[c] = p.op.a[c] ? slab.p + i * each + (p.op.a[c] - p.op.a[0]) : nullptr;
+        g.a2[c] = g.op.a[c];
+        g.op.mnz[c] = g.op.M[c];
+      }
+      if (packed3[q]) {
+        g.sA = (long)each;
+        g.amod = 3;
+      }
+      n.XGEMMS(&g, 1, false);
+    }
+  }
+  void update_fused() {
+    Navier &n = *ad, &s = *ns;
+    const int my = n.by_u.m, ny = n.ny, nx = n.nx, ro = n.rows_ortho(n.bx_f);
+    const long F = (long)n.FS;
+    const bool per = n.periodic;
+    // residual of one Navier-Stokes step (:727-750)
+    HIPCHECK(hipMemcpyAsync(s.STATE.p, n.STATE.p, sizeof(double) * 3 * F, hipMemcpyDeviceToDevice, n.st));
+    s.update();
+    ew_residual(n.st, s.STATE.p, s.STATE.p, n.STATE.p, s.dt, 3 * F);
+    if (per || n.bx_t.k == n.bx_u.k) {
+      Navier::FieldPair ft(s, 3);
+      s.to_ortho(s.bx_u, s.by_u, s.UX.p, UNSB.p);
+    } else {
+      {
+        Navier::FieldPair ft(s, 2);
+        s.to_ortho(s.bx_u, s.by_u, s.UX.p, UNSB.p);
+      }
+      s.to_ortho(s.bx_t, s.by_u, s.T.p, UNSB.p + 2 * F);
+    }
+    const double *bands[3], *diags[3];
+    for (int i = 0; i < 3; ++i) {
+      bands[i] = n.solver[i]->pybp.p;
+      diags[i] = n.solver[i]->diagp.p;
+    }
+    const int nsets = n.solver[0]->nsets, rows = per ? ro : n.solver[0]->pf.rows;
+    if (!per) smooth(0, UNSB.p, ny, n.W1.p);
+    n.timer.begin(n.st, 1, 8.0 * 3.0 * ((double)rows * (ny + my) + 4.0 * (double)nsets * my));
+    fdma_rows_lds_multi(n.st, per ? UNSB.p : n.W1.p, ny, ny, per ? F1B.p : n.W2.p, my, rows, my, nsets, bands, diags, 3, F, F);
+    n.timer.end(n.st);
+    if (!per) smooth(1, n.W2.p, my, F1B.p);
+    else ew_scale(n.st, F1B.p, F1B.p, -1.0, 3 * F);
+    // x-transformed values and derivatives of the residuals, values of the fields (transposed)
+    const PackedOp &bs = n.X.packed(n.bx_u, "BS"), &bds = n.X.packed(n.bx_u, "BDS");
+    const PackedOp &bst = per ? bs : n.X.packed(n.bx_t, "BS"), &bdst = per ? bds : n.X.packed(n.bx_t, "BDS");
+    {
+      XGemm g[3] = {n.field_op(bs, bst, F1B.p, my, n.A.p, nx, 0, 3), n.field_op(bds, bdst, F1B.p, my, n.W1.p, nx, 0, 3),
+                    n.field_op(bs, bst, n.UX.p, my, n.W2.p, nx, 0, 3)};
+      n.XGEMMS(g, 3, true);
+    }
+    if (!per) {
+      XGemm g[2] = {n.field_op(n.X.packed(n.bx_u, "DDS"), n.X.packed(n.bx_t, "DDS"), F1B.p, my, LX.p, my, 0, 3),
+                    xgemm_of(n.X.packed(n.bx_p, "DS"), n.P0.p, n.G.p, ny, 1, F, F)};
+      n.XGEMMS(g, 2, false);
+    }
+    {
+      const XGemm g = xgemm_of(n.Y.packed(n.by_u, "BS"), n.W2.p, PV.p, nx, 3, F, F);
+      n.XGEMMS(&g, 1, false);
+    }
+    AdjointConvArgs c{};
+    c.bs = n.Y.packed(n.by_u, "BS").op;
+    c.bds = n.Y.packed(n.by_u, "BDS").op;
+    c.T = n.A.p;
+    c.D = n.W1.p;
+    c.V = PV.p;
+    c.bc = BCT.p;
+    c.C = n.CONV.p;
+    c.nx = nx;
+    c.stride = F;
+    n.timer.begin(n.st, 0, 2.0 * 10.0 * 0.5 * my * (double)nx * ny);
+    adjoint_products(n.st, c);
+    n.timer.end(n.st);
+    {
+      const XGemm fy = xgemm_of(n.Y.packed(n.by_p, "Fdl"), n.CONV.p, n.W2.p, nx, 3, F, F);
+      XGemm g = fy;
+      g.ldc = ny;
+      n.XGEMMS(&g, 1, true);
+      const XGemm fx = xgemm_of(n.X.packed(n.bx_f, "Fdl"), n.W2.p, n.CV.p, ny, 3, F, F);
+      n.XGEMMS(&fx, 1, false);
+    }
+    AdjointRows a{};
+    a.U = n.UX.p;
+    a.F = F1B.p;
+    a.LX = per ? nullptr : LX.p;
+    a.GX = per ? nullptr : n.G.p;
+    a.P0 = n.P0.p;
+    a.CV = n.CV.p;
+    a.RHS = n.RHS.p;
+    a.sxu = per ? nullptr : n.stencil_band(n.bx_u).coef.p;
+    a.sxt = per ? nullptr : n.stencil_band(n.bx_t).coef.p;
+    a.sy = n.stencil_band(n.by_u).coef.p;
+    a.rows = ro;
+    a.mx = per ? n.mx() : n.bx_u.m;
+    a.ny = ny;
+    a.my = my;
+    a.field = F;
+    a.dt = dt;
+    a.nu = n.nu;
+    a.ka = n.ka;
+    a.inv_scy = 1.0 / n.scale[1];
+    a.kscale = n.scale[0];
+    n.timer.begin(n.st, 3, 8.0 * 3.0 * (double)ro * (4.0 * my + 3.0 * ny));
+    adjoint_rows(n.st, a);
+    n.timer.end(n.st);
+    const int rs = n.rows_spec(n.bx_u);
+    if (!per) {
+      const XGemm g = n.field_op(n.X.packed(n.bx_u, "FO"), n.X.packed(n.bx_t, "FO"), n.RHS.p, ny, n.W1.p, ny, 0, 3);
+      n.XGEMMS(&g, 1, false);
+    }
+    n.timer.begin(n.st, 8, 8.0 * 3.0 * (double)rs * ((double)ny + my));
+    tdma_rows_lds(n.st, per ? n.RHS.p : n.W1.p, ny, n.UX.p, my, rs, my, n.tdma_tables(n.by_u).tabp.p, 3, F, F, false);
+    n.timer.end(n.st);
+    // projection and pressure update without the viscous term (:683-724)
+    if (!per) {
+      ConfinedRows q = n.confined_rows();
+      q.f1 = 2;
+      q.nu = 0.0;
+      q.inv_dt = 1.0 / dt;
+      n.divergence_confined(q, n.DIV.p);
+      n.pressure_confined(q);
+    } else if (n.pressure_fused_ok()) {
+      n.timer.begin(n.st, 10, 8.0 * ro * (2.0 * my + ny) + 8.0 * ro * (3.0 * my + ny) + 16.0 * ro * (double)n.by_phi.m);
+      pressure_rows(n.st, n.pressure_args(0.0));
+      n.timer.end(n.st);
+    } else {
+      pressure_unfused();
+    }
+    n.gpres_valid = false;
+    time += dt;
+  }
+  void pressure_unfused() {
+    Navier& n = *ad;
+    n.divergence(n.DIV.p);
+    n.solve_pres();
+    n.project_velocity();
+    // update_pres (:720-724): pres += to_ortho(pseu) / dt, no viscous term
+    n.to_ortho(n.bx_phi, n.by_phi, n.P1.p, n.W3.p);
+    ew_axpy(n.st, n.P0.p, n.P0.p, n.W3.p, 1.0 / dt, (long)n.rows_ortho(n.bx_p) * n.ny);
+  }
+  // The first iteration after a set-up change runs eagerly (and builds the operators it needs), the
+  // later ones replay its capture.
+  void update() {
+    Navier &n = *ad, &s = *ns;
+    if (ready && (made[0] != n.set_ups || made[1] != s.set_ups)) {
+      ready = false;
+      drop_graph();
+    }
+    if (!ready && !fused_ok()) {
+      update_terms();
+      return;
+    }
+    const bool graph = n.use_graph && !n.timer.on && !s.timer.on;
+    if (!ready || !graph || (gexec && graph_gpres && !s.gpres_valid)) {
+      if (!ready) make_ready();
+      update_fused();
+      return;
+    }
+    if (!gexec) {
+      hipGraph_t g = nullptr;
+      const double t0 = time, t1 = s.time;
+      const bool gp = graph_gpres = s.gpres_valid;
+      HIPCHECK(hipStreamBeginCapture(n.st, hipStreamCaptureModeThreadLocal));
+      try {
+        update_fused();
+      } catch (...) {
+        (void)hipStreamEndCapture(n.st, &g);
+        if (g) (void)hipGraphDestroy(g);
+        time = t0;
+        s.time = t1;
+        s.gpres_valid = gp;
+        throw;
+      }
+      time = t0;
+      s.time = t1;
+      HIPCHECK(hipStreamEndCapture(n.st, &g));
+      const hipError_t e = hipGraphInstantiate(&gexec, g, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(g);
+      if (e != hipSuccess) {
+        gexec = nullptr;
+        throw DeviceError(std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+      }
+    }
+    HIPCHECK(hipGraphLaunch(gexec, n.st));
+    s.time += s.dt;
+    n.gpres_valid = false;
+    time += dt;
+  }
+  void update_terms() {  // Integrate::update (navier_adjoint.rs:760-790)
     Navier& n = *ad;
     n.backward_vel(n.UX.p, U.p);
     n.backward_vel(n.UY.p, V.p);
@@ -3205,35 +3500,27 @@ class Adjoint {
     update_residual();
     solve_vel(0);
     solve_vel(1);
-    n.divergence(n.DIV.p);
-    n.solve_pres();
-    n.project_velocity();
-    // update_pres (:720-724): pres += to_ortho(pseu) / dt, no viscous term
-    n.to_ortho(n.bx_phi, n.by_phi, n.P1.p, n.W3.p);
-    ew_axpy(n.st, n.P0.p, n.P0.p, n.W3.p, 1.0 / dt, (long)n.rows_ortho(n.bx_p) * n.ny);
+    pressure_unfused();
     solve_temp();
     n.gpres_valid = false;
     time += dt;
   }
-  static double norm(const std::vector<double>& v) {  // norm_l2_f64 / norm_l2_c64 (:902-913)
-    double s = 0.0;
-    for (double x : v) s += x * x;
-    return std::sqrt(s);
-  }
-  // [|ux1|, |uy1|, |temp1|, |unsmoothed ux|, |uy|, |temp|] (callback / exit, :846-897)
+  // [|ux1|, |uy1|, |temp1|, |unsmoothed ux|, |uy|, |temp|] (callback / exit, :846-897): norm_l2_f64 /
+  // norm_l2_c64 (:902-913), formed into pinned memory
+  double* norms_host = nullptr;
   void norms(double* out) {
     Navier& n = *ad;
+    if (!norms_host) HIPCHECK(hipHostMalloc(&norms_host, 6 * sizeof(double)));
+    for (int j = 0; j < 6; ++j) {
+      const double* v = j < 3 ? F1B.p + j * n.FS : UNSB.p + (j - 3) * n.FS;
+      const long len = j >= 3 ? ortho_len() : spec_len(j == 2 ? n.bx_t : n.bx_u);
+      sum_squares(n.st, v, len, n.NRM.p, norms_host + j);
+    }
     HIPCHECK(hipStreamSynchronize(n.st));
-    out[0] = norm(F1[1].download(spec_len(n.bx_u)));
-    out[1] = norm(F1[2].download(spec_len(n.bx_u)));
-    out[2] = norm(F1[0].download(spec_len(n.bx_t)));
-    for (int j = 0; j < 3; ++j) out[3 + j] = norm(UNS[j].download(ortho_len()));
+    for (int j = 0; j < 6; ++j) out[j] = std::sqrt(norms_host[j]);
   }
   bool exit() {  // :882-897
-    Navier& n = *ad;
-    n.divergence(n.DIV.p);
-    HIPCHECK(hipStreamSynchronize(n.st));
-    if (std::isnan(norm(n.DIV.download(ortho_len())))) return true;
+    if (std::isnan(ad->div_norm())) return true;
     double r[6];
     norms(r);
     return r[0] + r[1] + r[2] < res_tol;

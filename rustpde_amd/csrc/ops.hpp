@@ -122,6 +122,19 @@ struct ConvArgs {
   long stride, sf;
 };
 void conv_products(hipStream_t s, const ConvArgs& a);
+// The adjoint convective terms (navier_adjoint.rs:581-648) in physical space, transposed as above:
+//   ux:   2 U dx u + V dy u + V dx v + (T + bc) dx t      temp: U dx t + V dy t
+//   uy:   U dx v + 2 V dy v + U dy u + (T + bc) dy t
+// of the residuals u, v, t (T their x-transformed values, D x-derivatives, [my, nx], `stride` apart)
+// and the fields' values V = (U, V, T) and bc [ny, nx].
+struct AdjointConvArgs {
+  XOp bs, bds;
+  const double *T, *D, *V, *bc;
+  double* C;
+  int nx;
+  long stride;
+};
+void adjoint_products(hipStream_t s, const AdjointConvArgs& a);
 
 // Banded 4-diagonal solves (offsets -2, 0, 2, 4; pre-swept as fdma.rs:73-82) of every
 // row r of X[nrows, m] with diagonal set (r % nsets); diag arrays are [nsets, m].
@@ -309,6 +322,21 @@ struct ConfinedRows {
   double dt, inv_dt, inv_scy, nu;
 };
 bool confined_rows_supported(int nx, int ny);
+
+// Right-hand sides of the adjoint step (navier_adjoint.rs:581-648), fields f = 0..2 (ux, uy, temp)
+// `field` apart: to_ortho(U_f) - dt grad pres + dt CV_f + dt buoyancy (temp: to_ortho of the residual
+// uy) + dt k_f laplacian(F_f), F the smoothed residuals.  Confined (rows = nx ortho rows along x, mx
+// composite): GX = d/dx pres and LX_f = d2/dx2 F_f (y-spectral, [nx, my]) come from the x products.
+// Periodic (rows = 2 mx split planes): both are formed from the wavenumber and kscale.
+struct AdjointRows {
+  const double *U, *F, *LX, *GX, *P0, *CV;
+  double* RHS;
+  const double *sxu, *sxt, *sy;
+  int rows, mx, ny, my, per;
+  long field;
+  double dt, nu, ka, inv_scy, kscale;
+};
+void adjoint_rows(hipStream_t s, const AdjointRows& a);
 void rhs_rows(hipStream_t s, const ConfinedRows& a, int nb);
 void div_rows(hipStream_t s, const ConfinedRows& a, int nb);
 void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure);

@@ -423,6 +423,109 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
   }
 }
 
+// adjoint_products: as conv_kernel with one of the three terms per block, the four products
+//   ux:   bs D_u, bds T_u, bs D_v, bs D_t      uy:   bs D_v, bds T_v, bds T_u, bds T_t
+//   temp: bs D_t, bds T_t (the other two repeat them: its blocks end with the others')
+// of the residuals' x-transformed values T and derivatives D, taken with the fields' values at the
+// point: one launch in place of 14 terms of four launches each.
+template <int CH>
+__global__ __launch_bounds__(256) void adjoint_kernel(AdjointConvArgs a, int tx, int ty) {
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lk = lane >> 4;
+  int t = fftlds::xcd_remap(blockIdx.x, gridDim.x);
+  const int n0 = (t % tx) * 16;
+  t /= tx;
+  const int m0 = (t % ty) * 16, f = t / ty, N = a.nx;
+  const int col = min(n0 + lr, N - 1), G = a.bs.groups;
+  // product p: operator 0 bs, 1 bds; its array
+  const int op[4] = {0, 1, f == 0 ? 0 : f == 1 ? 1 : 0, f == 0 ? 0 : 1};
+  const int field[4] = {f, f, f == 2 ? 2 : 1 - f, 2};
+  const double* opa[4][2];
+  const double* src[4][2];
+  int K[4][2];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const double* base = op[p] ? a.bds.a[c] : a.bs.a[c];
+      opa[p][c] = base + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
+      const int r0 = op[p] ? a.bds.r0[c] : a.bs.r0[c];
+      K[p][c] = op[p] ? a.bds.K[c] : a.bs.K[c];
+      src[p][c] = (op[p] ? a.T : a.D) + a.stride * field[p] + (long)r0 * N + col;
+    }
+  struct Chunk {
+    double2 o[4][2][CH], d[4][2][CH];
+  };
+  v4d acc[4][2];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[p][c] = v4d{0, 0, 0, 0};
+  auto load = [&](int g0, Chunk& x) {
+#pragma unroll
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const int k = (g0 + h) * 8 + 2 * lk;
+          x.o[p][c][h] = *reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128);
+          x.d[p][c][h] = double2{src[p][c][(long)2 * min(k, K[p][c] - 1) * N],
+                                 src[p][c][(long)2 * min(k + 1, K[p][c] - 1) * N]};
+        }
+  };
+  auto mac = [&](int g0, const Chunk& x) {
+#pragma unroll
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const int k = (g0 + h) * 8 + 2 * lk;
+          const double v0 = k < K[p][c] ? x.d[p][c][h].x : 0.0, v1 = k + 1 < K[p][c] ? x.d[p][c][h].y : 0.0;
+          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.o[p][c][h].x, v0, acc[p][c], 0, 0, 0);
+          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.o[p][c][h].y, v1, acc[p][c], 0, 0, 0);
+        }
+  };
+  Chunk x, y;
+  const int nch = G / (4 * CH), top = G - CH, g0 = wid * nch * CH;
+  load(g0, x);
+  int n = 0;
+  for (; n + 2 <= nch; n += 2) {
+    load(min(g0 + (n + 1) * CH, top), y);
+    mac(g0 + n * CH, x);
+    load(min(g0 + (n + 2) * CH, top), x);
+    mac(g0 + (n + 1) * CH, y);
+  }
+  if (n < nch) mac(g0 + n * CH, x);
+  const int ny = a.bs.rows;
+  double res[4][2];
+  __shared__ double part[8 * 16 * 64];
+  add_quarters<8>(part, wid, lane, [&](int e, int r) { return acc[e >> 1][e & 1][r]; },
+                  [&](int e, double v) { res[e >> 1][e & 1] = v; });
+  const int m = m0 + 4 * wid + lk, nn = n0 + lr;
+  if (m >= a.bs.M[0] || nn >= N) return;
+#pragma unroll
+  for (int side = 0; side < 2; ++side) {
+#pragma clang fp contract(off)
+    const int row = side ? ny - 1 - m : m;
+    if (side && row == m) continue;
+    double v[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) v[p] = side ? res[p][0] - res[p][1] : res[p][0] + res[p][1];
+    const size_t at = (size_t)row * N + nn;
+    const double U = a.V[at], V = a.V[a.stride + at];
+    double q = U * v[0] + V * v[1];
+    if (f < 2) {  // the terms in the order of navier_adjoint.rs:581-626
+      q = q + U * (f == 0 ? v[0] : v[2]);
+      q = q + V * (f == 0 ? v[2] : v[1]);
+      q = q + a.V[2 * a.stride + at] * v[3];
+      q = q + a.bc[at] * v[3];
+    }
+    a.C[a.stride * f + at] = q;
+  }
+}
+
 template <int FM, int FN, bool SPLIT, int CH, int KIND, int NG, bool TR>
 void launch(hipStream_t s, const XGemm* groups) {
   constexpr int BM = 16 * FM * (SPLIT ? 1 : 2), BN = 16 * FN * (SPLIT ? 1 : 2);
@@ -518,6 +621,18 @@ void conv_products(hipStream_t s, const ConvArgs& a) {
   else RBC_LAUNCH((conv_kernel<1, 1>), grid, block, 0, s, a, tx, ty);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw std::runtime_error(std::string("conv_products: ") + hipGetErrorString(e));
+}
+
+void adjoint_products(hipStream_t s, const AdjointConvArgs& a) {
+  if (a.bs.kind != XOP_FOLD_OUT || a.bds.kind != XOP_FOLD_OUT || a.bs.groups != a.bds.groups ||
+      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.bs.rstep != 2 || a.bds.rstep != 2 || a.nx < 1)
+    throw std::invalid_argument("adjoint_products: bad arguments");
+  const int tx = (a.nx + 15) / 16, ty = (a.bs.M[0] + 15) / 16;
+  const long total = 3L * tx * ty;
+  if (total > 0x7fffffffL) throw std::invalid_argument("adjoint_products: too many tiles");
+  RBC_LAUNCH((adjoint_kernel<1>), dim3((unsigned)total), dim3(256), 0, s, a, tx, ty);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) throw std::runtime_error(std::string("adjoint_products: ") + hipGetErrorString(e));
 }
 
 // The tile follows from the launch's size, 16 x 16 tiles times groups of 8 k values (twice when
