@@ -14,6 +14,7 @@
 #include <map>
 #include <tuple>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -610,6 +611,64 @@ class KernelTimer {
 };
 
 // ----------------------------------------------------------------------- Navier2D
+// Fields on their way to the caller's memory, through pinned chunks that the host copies on while the next
+// are written: by the copy engine, or for split planes by a kernel that interleaves them.  On MI355X, us
+// with the wait: 32 KB 8.6 (19.0 with a copy into pageable memory), 128 KB 12.5 (12.8), 512 KB 27.6 (27.7);
+// the coefficients of a 1024 x 1025 Fourier field 366 (922 with a host vector and a host loop between).
+class HostStage {
+ public:
+  ~HostStage() {
+    if (p_) (void)hipHostFree(p_);
+    for (hipEvent_t e : ev_)
+      if (e) (void)hipEventDestroy(e);
+  }
+  // n values a, or a and b interleaved, after the work queued on st
+  void read(hipStream_t st, const double* a, const double* b, size_t n, double* host) {
+    if (n == 0) return;
+    std::lock_guard<std::mutex> lock(mu_);
+    const size_t w = b ? 2 : 1, chunk = CHUNK / w, count = (n + chunk - 1) / chunk;
+    ensure(count == 1 ? n * w : CHUNK * std::min<size_t>(count, SLOTS));
+    if (count == 1) {
+      put(st, a, b, n, p_);
+      HIPCHECK(hipStreamSynchronize(st));
+      std::memcpy(host, p_, n * w * sizeof(double));
+      return;
+    }
+    auto drain = [&](size_t i) {
+      HIPCHECK(hipEventSynchronize(ev_[i % SLOTS]));
+      std::memcpy(host + i * chunk * w, p_ + (i % SLOTS) * CHUNK, std::min(chunk, n - i * chunk) * w * sizeof(double));
+    };
+    for (size_t i = 0; i < count; ++i) {
+      if (i >= SLOTS) drain(i - SLOTS);
+      const size_t at = i * chunk;
+      put(st, a + at, b ? b + at : nullptr, std::min(chunk, n - at), p_ + (i % SLOTS) * CHUNK);
+      HIPCHECK(hipEventRecord(ev_[i % SLOTS], st));
+    }
+    for (size_t i = count > SLOTS ? count - SLOTS : 0; i < count; ++i) drain(i);
+  }
+
+ private:
+  static constexpr size_t CHUNK = (size_t)1 << 16, SLOTS = 4;  // doubles (512 KiB)
+  std::mutex mu_;
+  double* p_ = nullptr;
+  size_t n_ = 0;
+  hipEvent_t ev_[SLOTS] = {};
+  static void put(hipStream_t st, const double* a, const double* b, size_t n, double* out) {
+    if (b) read_out(st, a, b, out, (long)n);
+    else HIPCHECK(hipMemcpyAsync(out, a, n * sizeof(double), hipMemcpyDeviceToHost, st));
+  }
+  void ensure(size_t n) {
+    for (hipEvent_t& e : ev_)
+      if (!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    if (n <= n_) return;
+    if (p_) HIPCHECK(hipHostFree(p_));
+    p_ = nullptr;
+    n_ = 0;
+    HIPCHECK(hipHostMalloc(&p_, n * sizeof(double)));
+    n_ = n;
+  }
+};
+
 class Navier {
  public:
   bool periodic;
@@ -632,7 +691,7 @@ class Navier {
   // rows of THAT_BC, GXX and GYY (spectral, [rows, ny]) before which every value is +0.0
   int bc_rows = 0;
   // workspaces
-  DBuf THAT, UXP, UYP, A, G, CONV, CV, RHS, DIV, W1, W2, W3, W4, W9, RED, NRM;
+  DBuf THAT, UXP, UYP, A, G, CONV, CV, RHS, DIV, W1, W2, W3, W4, W9, NRM;
   std::vector<double> wx_dx, wy_dx;  // cell widths of `field` (unscaled, field.rs:135-163)
   double len0 = 0, len1 = 0;
   DBuf DX0, DX1;
@@ -700,6 +759,7 @@ class Navier {
   static constexpr int GRAPH_STEPS = 8;
   int eager_steps = 0;     // eager steps since the captured step was last dropped
   bool graph_gpres = false;  // the captured step reads d/dy pres left by the step before it
+  std::shared_ptr<HostStage> stage = std::make_shared<HostStage>();  // an ensemble group's instances share one
   unsigned long set_ups = 0;  // counts the set-up changes: graphs captured before one are stale
   void drop_graph() {
     ++set_ups;
@@ -993,7 +1053,6 @@ class Navier {
       for (DBuf* b : {&BCXT, &BCYT}) b->alloc(full);
     BC.alloc((size_t)R * 2);
     BCv.alloc((size_t)nx * ny);
-    RED.alloc(std::max(ny, 8) + 300);
     NRM.alloc(SUM_SQUARES_PART);
     // solvers
     const double cv[2] = {dt * nu / std::pow(scale[0], 2.0), dt * nu / std::pow(scale[1], 2.0)};
@@ -2306,15 +2365,9 @@ class Navier {
     int n0, n1, c;
     shape(which, space, n0, n1, c);
     FieldRef f = field(which);
-    HIPCHECK(hipStreamSynchronize(st));
-    if (space == RBC_PHYS || !c) {
-      std::vector<double> v = (space == RBC_PHYS ? f.phys : f.spec)->download((size_t)n0 * n1);
-      std::memcpy(host, v.data(), v.size() * sizeof(double));
-      return;
-    }
-    std::vector<double> v = f.spec->download((size_t)2 * n0 * n1);
     const size_t pl = (size_t)n0 * n1;
-    for (size_t i = 0; i < pl; ++i) { host[2 * i] = v[i]; host[2 * i + 1] = v[pl + i]; }
+    const double* v = (space == RBC_PHYS ? f.phys : f.spec)->p;
+    stage->read(st, v, space == RBC_PHYS || !c ? nullptr : v + pl, pl, host);
   }
   void set(int which, int space, const double* host) {
     gpres_valid = false;
@@ -2370,8 +2423,9 @@ class Navier {
     ew_scale(st, G.p, G.p, -1.0, no);
     ew_scale(st, G.p, G.p, 1.0 / (scale[1] / 2.0), no);
     const double* v = field_backward(G.p);
-    col_weighted_sum(st, v, nx, ny, DX0.p, RED.p);
-    std::vector<double> avg = RED.download(ny);
+    col_weighted_sum(st, v, nx, ny, DX0.p, pinned());
+    HIPCHECK(hipStreamSynchronize(st));
+    const double* avg = norm_host;
     const double a0 = avg[0] / len0, a1 = avg[ny - 1] / len0;
     return (a1 + a0) / 2.0;
   }
@@ -2395,8 +2449,9 @@ class Navier {
     return weighted_average(CV.p);
   }
   double weighted_average(const double* v) {
-    col_weighted_sum(st, v, nx, ny, DX0.p, RED.p);
-    std::vector<double> s = RED.download(ny);
+    col_weighted_sum(st, v, nx, ny, DX0.p, pinned());
+    HIPCHECK(hipStreamSynchronize(st));
+    const double* s = norm_host;
     double tot = 0.0;
     for (int j = 0; j < ny; ++j) tot += (s[j] / len0) * wy_dx[j] / len1;
     return tot;
@@ -2526,10 +2581,13 @@ class Navier {
     return std::sqrt(read_norm(G.p, no));
   }
   // sum of squares of n device values, formed into pinned host memory: no copy follows the kernel
-  double* norm_host = nullptr;
+  double* norm_host = nullptr;  // max(ny, 8) doubles
+  double* pinned() {
+    if (!norm_host) HIPCHECK(hipHostMalloc(&norm_host, std::max(ny, 8) * sizeof(double)));
+    return norm_host;
+  }
   double read_norm(const double* v, long n) {
-    if (!norm_host) HIPCHECK(hipHostMalloc(&norm_host, 2 * sizeof(double)));
-    sum_squares(st, v, n, NRM.p, norm_host);
+    sum_squares(st, v, n, NRM.p, pinned());
     HIPCHECK(hipStreamSynchronize(st));
     return *norm_host;
   }
@@ -3038,6 +3096,7 @@ class Ensemble {
                                                    b > 0 ? g->navs[0].get() : nullptr));
         inst[mem[b]] = g->navs.back().get();
         inst[mem[b]]->leader = g->navs[0].get();
+        inst[mem[b]]->stage = g->navs[0]->stage;
         group_of[mem[b]] = (int)groups.size();
       }
       Navier& L = *g->navs[0];

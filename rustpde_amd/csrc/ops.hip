@@ -450,17 +450,31 @@ void ew_update_pres_group(hipStream_t s, double* p, const double* div, const dou
 }
 
 // ------------------------------------------------------------------------- reductions
-__global__ void col_weighted_sum_kernel(const double* __restrict__ v, int n0, int n1, const double* __restrict__ w,
-                                        double* __restrict__ out) {
+// sum_i v[i][j] w[i]: 16 columns per block, 32 threads a column, each every 32nd row; out may lie in
+// pinned host memory.  The chain of loads bounds it: 1024 x 1025 took 253 us with one thread a column.
+constexpr int CWS_COLS = 16, CWS_ROWS = 32;
+__global__ __launch_bounds__(CWS_COLS* CWS_ROWS) void col_weighted_sum_kernel(const double* __restrict__ v, int n0, int n1,
+                                                                              const double* __restrict__ w,
+                                                                              double* __restrict__ out) {
 #pragma clang fp contract(off)
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n1) return;
+  __shared__ double red[CWS_ROWS][CWS_COLS];
+  const int c = threadIdx.x % CWS_COLS, r = threadIdx.x / CWS_COLS, j = blockIdx.x * CWS_COLS + c;
   double s = 0.0;
-  for (int i = 0; i < n0; ++i) s = s + v[(size_t)i * n1 + j] * w[i];
-  out[j] = s;
+  if (j < n1) {
+#pragma unroll 8
+    for (int i = r; i < n0; i += CWS_ROWS) s = s + v[(size_t)i * n1 + j] * w[i];
+  }
+  red[r][c] = s;
+  __syncthreads();
+  for (int h = CWS_ROWS / 2; h > 0; h >>= 1) {
+    if (r < h) red[r][c] += red[r + h][c];
+    __syncthreads();
+  }
+  if (r == 0 && j < n1) out[j] = red[0][c];
 }
 void col_weighted_sum(hipStream_t s, const double* v, int n0, int n1, const double* w, double* out) {
-  RBC_LAUNCH(col_weighted_sum_kernel, dim3(blocks_for(n1, 64)), dim3(64), 0, s, v, n0, n1, w, out);
+  RBC_LAUNCH(col_weighted_sum_kernel, dim3((n1 + CWS_COLS - 1) / CWS_COLS), dim3(CWS_COLS * CWS_ROWS), 0, s, v, n0, n1, w,
+             out);
   check_launch("col_weighted_sum");
 }
 
@@ -508,6 +522,17 @@ void sum_squares(hipStream_t s, const double* b, long n, double* part, double* o
 }
 
 // --------------------------------------------------------------------- layout changes
+// values a and b, interleaved, into pinned host memory
+__global__ void read_out_kernel(const double* __restrict__ a, const double* __restrict__ b, double2* __restrict__ out,
+                                long n) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = double2{a[i], b[i]};
+}
+void read_out(hipStream_t s, const double* a, const double* b, double* out, long n) {
+  if (n <= 0) return;
+  RBC_LAUNCH(read_out_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, a, b, reinterpret_cast<double2*>(out), n);
+  check_launch("read_out");
+}
 // batch entries (blockIdx.y) are consecutive
 __global__ void i2s_kernel(const double* __restrict__ in, double* __restrict__ out, long n) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -243,6 +243,8 @@ void ew_update_pres_group(hipStream_t s, double* p, const double* div, const dou
 
 // Weighted column sums: out[j] = sum_i v[i, j] * w[i]  (i sequential, as average.rs:25-34)
 void col_weighted_sum(hipStream_t s, const double* v, int n0, int n1, const double* w, double* out);
+// out (16-byte aligned, pinned host memory): the n values a and b, interleaved
+void read_out(hipStream_t s, const double* a, const double* b, double* out, long n);
 // *out (device or pinned host memory) = sum of squares of b[0..n); part holds SUM_SQUARES_PART doubles,
 // zero before the first call and used by one call at a time
 constexpr int SUM_SQUARES_PART = 257;
