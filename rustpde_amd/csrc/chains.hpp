@@ -1,11 +1,13 @@
 // Recurrences along one parity chain of a row, held by one wavefront: lane l owns chain
 // positions t in [t0, t0 + cnt), t0 = l * per, in registers v[q] (q = t - t0).  Each pass is
 // a linear recurrence: the lane composes the affine map of its slice, the maps are scanned
-// across the wavefront with shuffles, and each lane replays its slice with the reference's
+// across the wavefront (wave.hpp), and each lane replays its slice with the reference's
 // arithmetic from its incoming state (divisions by a diagonal taken as products with its
 // tabulated reciprocal).  Used by the row kernels and the fused pressure stage.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include "wave.hpp"
 
 namespace rbc {
 namespace chains {
@@ -85,7 +87,7 @@ template <int SLICE>
 __device__ __forceinline__ void fdma_forward(double (&v)[SLICE], const double (&lo)[SLICE], int lane, int t0,
                                              int cnt) {
 #pragma clang fp contract(off)
-  static_assert(SLICE >= 4 && SLICE % 2 == 0, "two half slices of at least two entries");
+  static_assert(SLICE % 2 == 0, "two half slices");
   constexpr int H = SLICE / 2;
   double A1 = 1.0, B1 = 0.0, A2 = 1.0, B2 = 0.0;  // half maps y_out = A y_in + B
 #pragma unroll
@@ -105,16 +107,9 @@ __device__ __forceinline__ void fdma_forward(double (&v)[SLICE], const double (&
       B2 = v[q] - B2 * lo[q];
     }
   }
-  double pa = A2 * A1, pb = A2 * B1 + B2;  // lane map, then inclusive scan, lower lanes first
-  for (int off = 1; off < WAVE; off <<= 1) {
-    const double qa = __shfl_up(pa, off), qb = __shfl_up(pb, off);
-    if (lane >= off) {
-      pb = pa * qb + pb;
-      pa = pa * qa;
-    }
-  }
-  double y1 = __shfl_up(pb, 1);
-  if (lane == 0) y1 = 0.0;
+  double b[1] = {A2 * B1 + B2}, y[1];  // lane map
+  wave::scan_states<false>(A2 * A1, b, lane, y);
+  double y1 = y[0];
   double y2 = A1 * y1 + B1;
 #pragma unroll
   for (int j = 0; j < H; ++j) {
@@ -133,9 +128,7 @@ __device__ __forceinline__ void fdma_forward(double (&v)[SLICE], const double (&
 // Fdma back substitution: x_t = (y_t - x_{t+1} up1 - x_{t+2} up2) / dia over a chain of
 // length len (g1, g2 zero where t + 1, t + 2 leave the chain).  rd holds 1 / dia: the
 // division becomes a product with the tabulated reciprocal (one rounding apart).
-struct Map2 {  // s' = M s + w on the state s = (x_{t+1}, x_{t+2})
-  double m00 = 1.0, m01 = 0.0, m10 = 0.0, m11 = 1.0, w0 = 0.0, w1 = 0.0;
-};
+using wave::Map2;  // s' = M s + w on the state s = (x_{t+1}, x_{t+2})
 __device__ __forceinline__ void map2_step(Map2& a, double v, double r, double g1, double g2) {
 #pragma clang fp contract(off)
   const double c0 = v * r, c1 = -(g1 * r), c2 = -(g2 * r);
@@ -158,30 +151,8 @@ __device__ __forceinline__ void fdma_backward(double (&v)[SLICE], const double (
     if (j < cnt) map2_step(L, v[j], rd[j], g1[j], g2[j]);
     if (H + j < cnt) map2_step(U, v[H + j], rd[H + j], g1[H + j], g2[H + j]);
   }
-  // lane map M = M_L M_U, w = M_L w_U + w_L, then the suffix scan
-  double a00 = L.m00 * U.m00 + L.m01 * U.m10, a01 = L.m00 * U.m01 + L.m01 * U.m11;
-  double a10 = L.m10 * U.m00 + L.m11 * U.m10, a11 = L.m10 * U.m01 + L.m11 * U.m11;
-  double b0 = L.m00 * U.w0 + L.m01 * U.w1 + L.w0, b1 = L.m10 * U.w0 + L.m11 * U.w1 + L.w1;
-  for (int off = 1; off < WAVE; off <<= 1) {
-    const double q00 = __shfl_down(a00, off), q01 = __shfl_down(a01, off), q10 = __shfl_down(a10, off),
-                 q11 = __shfl_down(a11, off), r0 = __shfl_down(b0, off), r1 = __shfl_down(b1, off);
-    if (lane + off < WAVE) {
-      const double n00 = a00 * q00 + a01 * q10, n01 = a00 * q01 + a01 * q11;
-      const double n10 = a10 * q00 + a11 * q10, n11 = a10 * q01 + a11 * q11;
-      const double nb0 = a00 * r0 + a01 * r1 + b0, nb1 = a10 * r0 + a11 * r1 + b1;
-      a00 = n00;
-      a01 = n01;
-      a10 = n10;
-      a11 = n11;
-      b0 = nb0;
-      b1 = nb1;
-    }
-  }
-  double u0 = __shfl_down(b0, 1), u1 = __shfl_down(b1, 1);
-  if (lane == WAVE - 1) {
-    u0 = 0.0;
-    u1 = 0.0;
-  }
+  double u0, u1;
+  wave::scan_states2(wave::compose(L, U), lane, u0, u1);
   double l0 = U.m00 * u0 + U.m01 * u1 + U.w0, l1 = U.m10 * u0 + U.m11 * u1 + U.w1;
 #pragma unroll
   for (int j = H - 1; j >= 0; --j) {
@@ -235,16 +206,9 @@ __device__ __forceinline__ void tdma_forward(double (&v)[SLICE], const double (&
       B2 = (v[q] - B2 * of[q]) * rn[q];
     }
   }
-  double pa = A2 * A1, pb = A2 * B1 + B2;
-  for (int o2 = 1; o2 < WAVE; o2 <<= 1) {
-    const double qa = __shfl_up(pa, o2), qb = __shfl_up(pb, o2);
-    if (lane >= o2) {
-      pb = pa * qb + pb;
-      pa = pa * qa;
-    }
-  }
-  double g1v = __shfl_up(pb, 1);
-  if (lane == 0) g1v = 0.0;
+  double b[1] = {A2 * B1 + B2}, y[1];
+  wave::scan_states<false>(A2 * A1, b, lane, y);
+  double g1v = y[0];
   double g2v = A1 * g1v + B1;
 #pragma unroll
   for (int j = 0; j < H; ++j) {
@@ -289,16 +253,9 @@ __device__ __forceinline__ void tdma_backward(double (&v)[SLICE], const double (
       }
     }
   }
-  double pa = A1 * A2, pb = A1 * B2 + B1;
-  for (int o2 = 1; o2 < WAVE; o2 <<= 1) {
-    const double qa = __shfl_down(pa, o2), qb = __shfl_down(pb, o2);
-    if (lane + o2 < WAVE) {
-      pb = pa * qb + pb;
-      pa = pa * qa;
-    }
-  }
-  double x2 = __shfl_down(pb, 1);
-  if (lane == WAVE - 1) x2 = 0.0;
+  double b[1] = {A1 * B2 + B1}, y[1];
+  wave::scan_states<true>(A1 * A2, b, lane, y);
+  double x2 = y[0];
   double x1 = A2 * x2 + B2;
 #pragma unroll
   for (int j = H - 1; j >= 0; --j) {
@@ -344,20 +301,9 @@ __device__ __forceinline__ void tdma_forward2(double (&v)[SLICE], double (&u)[SL
       C2 = (u[q] - C2 * of[q]) * rn[q];
     }
   }
-  double pa = A2 * A1, pb = A2 * B1 + B2, pc = A2 * C1 + C2;
-  for (int o2 = 1; o2 < WAVE; o2 <<= 1) {
-    const double qa = __shfl_up(pa, o2), qb = __shfl_up(pb, o2), qc = __shfl_up(pc, o2);
-    if (lane >= o2) {
-      pb = pa * qb + pb;
-      pc = pa * qc + pc;
-      pa = pa * qa;
-    }
-  }
-  double g1v = __shfl_up(pb, 1), h1v = __shfl_up(pc, 1);
-  if (lane == 0) {
-    g1v = 0.0;
-    h1v = 0.0;
-  }
+  double b[2] = {A2 * B1 + B2, A2 * C1 + C2}, y[2];
+  wave::scan_states<false>(A2 * A1, b, lane, y);
+  double g1v = y[0], h1v = y[1];
   double g2v = A1 * g1v + B1, h2v = A1 * h1v + C1;
 #pragma unroll
   for (int j = 0; j < H; ++j) {
@@ -409,20 +355,9 @@ __device__ __forceinline__ void tdma_backward2(double (&v)[SLICE], double (&u)[S
       }
     }
   }
-  double pa = A1 * A2, pb = A1 * B2 + B1, pc = A1 * C2 + C1;
-  for (int o2 = 1; o2 < WAVE; o2 <<= 1) {
-    const double qa = __shfl_down(pa, o2), qb = __shfl_down(pb, o2), qc = __shfl_down(pc, o2);
-    if (lane + o2 < WAVE) {
-      pb = pa * qb + pb;
-      pc = pa * qc + pc;
-      pa = pa * qa;
-    }
-  }
-  double x2 = __shfl_down(pb, 1), y2 = __shfl_down(pc, 1);
-  if (lane == WAVE - 1) {
-    x2 = 0.0;
-    y2 = 0.0;
-  }
+  double b[2] = {A1 * B2 + B1, A1 * C2 + C1}, y[2];
+  wave::scan_states<true>(A1 * A2, b, lane, y);
+  double x2 = y[0], y2 = y[1];
   double x1 = A2 * x2 + B2, y1 = A2 * y2 + C2;
 #pragma unroll
   for (int j = H - 1; j >= 0; --j) {
@@ -456,13 +391,8 @@ __device__ __forceinline__ void suffix_sum(double (&v)[SLICE], int lane, int cnt
     if (j < cnt) t1 = v[j] + t1;
     if (H + j < cnt) t2 = v[H + j] + t2;
   }
-  double inc = t1 + t2;  // inclusive suffix sum over lanes
-  for (int off = 1; off < WAVE; off <<= 1) {
-    const double o = __shfl_down(inc, off);
-    if (lane + off < WAVE) inc = inc + o;
-  }
-  double a2 = __shfl_down(inc, 1);
-  if (lane == WAVE - 1) a2 = 0.0;
+  double a2;
+  wave::suffix_sum(t1 + t2, lane, a2);
   double a1 = t2 + a2;
 #pragma unroll
   for (int j = H - 1; j >= 0; --j) {

@@ -295,7 +295,8 @@ static void check_args(const ConfinedRows& a, int nb) {
   do {                                                                                       \
     const dim3 grid((unsigned)(blocks), nb), block(NT);                                      \
     const size_t lds = buf_len(a.ny) * sizeof(double);                                       \
-    if ((per) <= 4) RBC_LAUNCH(KERNEL<4>, grid, block, lds, s, __VA_ARGS__);                 \
+    if ((per) <= 2) RBC_LAUNCH(KERNEL<2>, grid, block, lds, s, __VA_ARGS__);                 \
+    else if ((per) <= 4) RBC_LAUNCH(KERNEL<4>, grid, block, lds, s, __VA_ARGS__);                 \
     else if ((per) <= 8) RBC_LAUNCH(KERNEL<8>, grid, block, lds, s, __VA_ARGS__);            \
     else RBC_LAUNCH(KERNEL<16>, grid, block, lds, s, __VA_ARGS__);                           \
   } while (0)
@@ -335,7 +336,8 @@ void adjoint_rows(hipStream_t s, const AdjointRows& in) {
     if (fourier) RBC_LAUNCH((adjoint_rows_kernel<SL, true>), grid, block, lds, s, a);          \
     else RBC_LAUNCH((adjoint_rows_kernel<SL, false>), grid, block, lds, s, a);                 \
   } while (0)
-  if (a.per <= 4) RBC_ADJOINT(4);
+  if (a.per <= 2) RBC_ADJOINT(2);
+  else if (a.per <= 4) RBC_ADJOINT(4);
   else if (a.per <= 8) RBC_ADJOINT(8);
   else RBC_ADJOINT(16);
 #undef RBC_ADJOINT

@@ -432,17 +432,21 @@ void pressure_rows(hipStream_t s, const PressureArgs& args) {
   const int perd = ((a.ny - 1) / 2 + WAVE - 1) / WAVE, sl = a.per > perd ? a.per : perd;
   const size_t lds = (size_t)6 * a.bl * sizeof(double);
   const bool rbc = a.su_kind == 1 && a.sp_kind == 2 && a.isc != 0.0;
+  const int slice = sl <= 2 ? 2 : sl <= 4 ? 4 : 8;
   if (a.rows_nsets > 0) {  // the further rows: slices within the stage's SLICE, buffers within its LDS
     a.rows_per = fdma_rows_lds_per(a.rows_m);
     a.rows_bl = buf_len(a.rows_nr);
-    if (!fdma_rows_lds_supported(a.rows_m, a.rows_nr) || (a.rows_per <= 4 ? 4 : 8) > (sl <= 4 ? 4 : 8) ||
+    if (!fdma_rows_lds_supported(a.rows_m, a.rows_nr) || a.rows_per > slice || fdma_rows_lds_per(a.rows_nr - 2) > slice ||
         (size_t)(rowsolve::WAVES / 2) * a.rows_bl * sizeof(double) > lds || !a.rows_R || !a.rows_X || !a.rows_diag)
       throw std::invalid_argument("pressure_rows: unsupported further rows");
   } else {
     a.rows_nsets = 0;
   }
   const dim3 grid((unsigned)(a.mx + a.rows_nsets));
-  if (sl <= 4) {
+  if (slice == 2) {
+    if (rbc) RBC_LAUNCH((pressure_rows_kernel<2, true>), grid, dim3(256), lds, s, a);
+    else RBC_LAUNCH((pressure_rows_kernel<2, false>), grid, dim3(256), lds, s, a);
+  } else if (slice == 4) {
     if (rbc) RBC_LAUNCH((pressure_rows_kernel<4, true>), grid, dim3(256), lds, s, a);
     else RBC_LAUNCH((pressure_rows_kernel<4, false>), grid, dim3(256), lds, s, a);
   } else {

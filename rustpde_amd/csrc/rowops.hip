@@ -184,7 +184,8 @@ bool row_ops_supported(int n) { return n >= 6 && fdma_rows_lds_per(n) <= 16; }
 #define RBC_ROW_OP(KERNEL, CPLX, per, ...)                                                                   \
   do {                                                                                                       \
     const dim3 grid((unsigned)((CPLX) ? rows : (rows + 1) / 2)), block(WAVE * WAVES);                         \
-    if ((per) <= 4) RBC_LAUNCH((KERNEL<4, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
+    if ((per) <= 2) RBC_LAUNCH((KERNEL<2, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
+    else if ((per) <= 4) RBC_LAUNCH((KERNEL<4, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
     else if ((per) <= 8) RBC_LAUNCH((KERNEL<8, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__); \
     else RBC_LAUNCH((KERNEL<16, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);                \
   } while (0)

@@ -150,6 +150,12 @@ bool fdma_rows_lds_supported(int m, int nr) {
          (size_t)(WAVES / 2) * buf_len(nr) * sizeof(double) <= 65536;
 }
 
+// entries per lane and chain that hold the row's solution and stage its right-hand side
+static int slice_of(int m, int nr) {
+  const int a = fdma_rows_lds_per(m), b = fdma_rows_lds_per(nr - 2);
+  return a > b ? a : b;
+}
+
 static void launch_rows(hipStream_t s, const double* R, int ldr, int nr, double* X, int ld, int nrows, int m,
                         int nsets, const RowTables& tb, int batch, long sr, long sx) {
   if (!fdma_rows_lds_supported(m, nr)) throw std::invalid_argument("fdma_rows_lds: unsupported row length");
@@ -157,7 +163,7 @@ static void launch_rows(hipStream_t s, const double* R, int ldr, int nr, double*
   if (!tb.shared && batch > 4) throw std::invalid_argument("fdma_rows_lds: at most 4 entries with own tables");
   for (int k = 0; k < (tb.shared ? 1 : batch); ++k)
     if (!tb.band[k] && nr != m) throw std::invalid_argument("fdma_rows_lds: rhs length must equal m without a band");
-  const int per = fdma_rows_lds_per(m), bl = buf_len(nr);
+  const int per = fdma_rows_lds_per(m), bl = buf_len(nr), sl = slice_of(m, nr);
   const unsigned blocks = nrows == 2 * nsets ? (unsigned)nsets : (unsigned)((nrows + 1) / 2);
   const size_t lds = (size_t)(WAVES / 2) * bl * sizeof(double);
   // entries 0 and 1 on the same tables, one block per set: interleaved 1-D grid
@@ -166,10 +172,13 @@ static void launch_rows(hipStream_t s, const double* R, int ldr, int nr, double*
   const int pairg = paired ? (nsets + 7) / 8 : 0;
   const dim3 grid = paired ? dim3((unsigned)(16 * pairg + (batch - 2) * nsets), 1) : dim3(blocks, batch),
              block(WAVE * WAVES);
-  if (per <= 4)
+  if (sl <= 2)
+    RBC_LAUNCH(fdma_rows_lds_kernel<2>, grid, block, lds, s, R, ldr, nr, X, ld, nrows, m, nsets, per, bl, tb,
+                       sr, sx, pairg);
+  else if (sl <= 4)
     RBC_LAUNCH(fdma_rows_lds_kernel<4>, grid, block, lds, s, R, ldr, nr, X, ld, nrows, m, nsets, per, bl, tb,
                        sr, sx, pairg);
-  else if (per <= 8)
+  else if (sl <= 8)
     RBC_LAUNCH(fdma_rows_lds_kernel<8>, grid, block, lds, s, R, ldr, nr, X, ld, nrows, m, nsets, per, bl, tb,
                        sr, sx, pairg);
   else
@@ -204,15 +213,17 @@ void fdma_rows_lds_complex(hipStream_t s, const double* R, int ldr, int nr, doub
                            const double* bandp, const double* diagp, int batch) {
   if (!fdma_rows_lds_supported(m, nr)) throw std::invalid_argument("fdma_rows_lds_complex: unsupported row length");
   if (nsets < 1 || batch < 1 || !bandp || !diagp) throw std::invalid_argument("fdma_rows_lds_complex: bad arguments");
-  const int per = fdma_rows_lds_per(m), bl = buf_len(nr);
+  const int per = fdma_rows_lds_per(m), bl = buf_len(nr), sl = slice_of(m, nr);
   const size_t lds = (size_t)(WAVES / 2) * bl * sizeof(double);
   for (int b = 0; b < batch; b += 65535) {
     const dim3 grid(nsets, batch - b < 65535 ? batch - b : 65535), block(WAVE * WAVES);
     const double* Rb = R + 2 * (size_t)nsets * ldr * b;
     double* Xb = X + 2 * (size_t)nsets * ld * b;
-    if (per <= 4)
+    if (sl <= 2)
+      RBC_LAUNCH(fdma_rows_complex_kernel<2>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
+    else if (sl <= 4)
       RBC_LAUNCH(fdma_rows_complex_kernel<4>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
-    else if (per <= 8)
+    else if (sl <= 8)
       RBC_LAUNCH(fdma_rows_complex_kernel<8>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
     else
       RBC_LAUNCH(fdma_rows_complex_kernel<16>, grid, block, lds, s, Rb, ldr, nr, Xb, ld, m, nsets, per, bl, bandp, diagp);
@@ -231,7 +242,9 @@ void tdma_rows_lds(hipStream_t s, const double* R, int ldr, double* X, int ld, i
   const int per = fdma_rows_lds_per(m), bl = buf_len(m + 2), pj = project ? 1 : 0;
   const dim3 grid((unsigned)((rows + 1) / 2), batch), block(WAVE * WAVES);
   const size_t lds = (size_t)(WAVES / 2) * bl * sizeof(double);
-  if (per <= 4)
+  if (per <= 2)
+    RBC_LAUNCH(tdma_rows_lds_kernel<2>, grid, block, lds, s, R, ldr, X, ld, rows, m, per, bl, tabp, sr, sx, pj);
+  else if (per <= 4)
     RBC_LAUNCH(tdma_rows_lds_kernel<4>, grid, block, lds, s, R, ldr, X, ld, rows, m, per, bl, tabp, sr, sx, pj);
   else if (per <= 8)
     RBC_LAUNCH(tdma_rows_lds_kernel<8>, grid, block, lds, s, R, ldr, X, ld, rows, m, per, bl, tabp, sr, sx, pj);
