@@ -54,6 +54,20 @@ constexpr int classes_of() {
   return KIND == XOP_DENSE ? 1 : KIND == XOP_BLOCKS ? (TR ? 2 : 1) : 2;
 }
 
+// The values from element off on of an array whose valid part ends at element `end`, as a buffer: loads
+// beyond it give zero.  Base and bound stay in scalar registers, so a load of row k of an operand costs no
+// vector instruction but itself; 64-bit addresses, clamped rows and selects per value cost a tenth of the
+// kernels' time (510^2 x 64 200 -> 186 us, the convective products of 257^2 15.3 -> 13.5).
+using Buffer = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ Buffer rows_from(const double* base, long off, long end) {
+  const long left = (end - off) * 8;
+  const int n = left <= 0 ? 0 : left > 0x7ffffff8L ? 0x7ffffff8 : (int)left;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(base + off), 0, n, 0x00020000);
+}
+__device__ __forceinline__ double value_at(Buffer b, unsigned byte) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, byte, 0, 0));
+}
+
 // (q0 + q1) + (q2 + q3) of the four wavefronts' partial tiles e < NE, in LDS: get(e, r) gives the
 // calling wavefront's register r of tile e, put(e, v) takes the sum of register wid.
 template <int NE, class Get, class Put>
@@ -77,7 +91,7 @@ __device__ __forceinline__ void add_quarters(double* part, int wid, int lane, Ge
 // quarters in turn.  KIND: the groups' operators' (folding out, a group may hold block
 // operators too).  CH: groups of 8 k values per chunk of loads.
 template <int FM, int FN, bool SPLIT, int CH, int KIND, int NG, bool TR>
-__global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
+__global__ __launch_bounds__(256, 2) void xgemm_kernel(XArgs<NG> ar) {
   constexpr bool IN2 = KIND == XOP_FOLD_IN;
   constexpr int NC = classes_of<KIND, TR>(), ND = IN2 ? 1 : NC;  // ND: distinct sets of data loads
   constexpr int BM = 16 * FM * (SPLIT ? 1 : 2), BN = 16 * FN * (SPLIT ? 1 : 2);
@@ -124,6 +138,8 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
   // class c of the block (both, or its own)
   const double* Ac[NC];
   int Kc[NC], r0[NC];
+  const double* Bc[NC];  // the class's first input row, and its extent
+  long end[NC];
   bool any = false;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
@@ -131,11 +147,19 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
     any = any || m0 < pick(one, g.op.mnz[0], g.op.mnz[1]);  // else past a cut: zero rows
     Kc[c] = pick(one, g.op.K[0], g.op.K[1]);
     r0[c] = pick(one, g.op.r0[0], g.op.r0[1]);
-    Ac[c] = pick(one, a0, a1) + aoff + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
+    Ac[c] = pick(one, a0, a1) + aoff + (size_t)(m0 >> 4) * G * 128;
+    Bc[c] = B + (long)r0[c] * ldb;
+    end[c] = (long)(Kc[c] - 1) * rs * ldb + N;
   }
   const double* Bn[FN];  // this lane's columns (past N: a column inside, never stored)
+  unsigned at[FN][2];    // and its two k values of a group there
 #pragma unroll
-  for (int j = 0; j < FN; ++j) Bn[j] = B + min(n0 + 16 * j + lr, N - 1);
+  for (int j = 0; j < FN; ++j) {
+    const int col = min(n0 + 16 * j + lr, N - 1);
+    Bn[j] = B + col;
+    at[j][0] = 8u * (unsigned)(2 * lk * rs * ldb + col);
+    at[j][1] = at[j][0] + 8u * (unsigned)(rs * ldb);
+  }
   const long kst = ldb;  // from one input row of the operator to the next
 
   struct Chunk {
@@ -148,18 +172,22 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
       for (int h = 0; h < CH; ++h) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
-          x.a[c][h][i] = *reinterpret_cast<const double2*>(Ac[c] + ((size_t)i * G + g0 + h) * 128);
+          x.a[c][h][i] = reinterpret_cast<const double2*>(Ac[c] + ((size_t)i * G + g0 + h) * 128)[lane];
         if (c >= ND) continue;
-        const int k = (g0 + h) * 8 + 2 * lk;
-        const int q0 = r0[c] + rs * min(k, Kc[c] - 1), q1 = r0[c] + rs * min(k + 1, Kc[c] - 1);
+        if constexpr (IN2) {  // clamped rows: the mirrored ones run down, past no bound that a buffer has
+          const int k = (g0 + h) * 8 + 2 * lk;
+          const int q0 = r0[c] + rs * min(k, Kc[c] - 1), q1 = r0[c] + rs * min(k + 1, Kc[c] - 1);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
-          x.b[c][h][j].x = Bn[j][q0 * kst];
-          x.b[c][h][j].y = Bn[j][q1 * kst];
-          if constexpr (IN2) {
+          for (int j = 0; j < FN; ++j) {
+            x.b[c][h][j].x = Bn[j][q0 * kst];
+            x.b[c][h][j].y = Bn[j][q1 * kst];
             x.m[h][j].x = Bn[j][(last - q0) * kst];
             x.m[h][j].y = Bn[j][(last - q1) * kst];
           }
+        } else {
+          const Buffer w = rows_from(Bc[c], (long)(g0 + h) * 8 * rs * ldb, end[c]);
+#pragma unroll
+          for (int j = 0; j < FN; ++j) x.b[c][h][j] = double2{value_at(w, at[j][0]), value_at(w, at[j][1])};
         }
       }
   };
@@ -178,16 +206,16 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         const int k = (g0 + h) * 8 + 2 * lk;
-        const bool ok0 = k < Kc[c], ok1 = k + 1 < Kc[c];  // the packed rows end in zeros, B does not
+        const bool ok0 = k < Kc[c], ok1 = k + 1 < Kc[c];
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
           double2 b = x.b[c < ND ? c : 0][h][j];
           if constexpr (IN2) {
             b.x = c ? b.x - x.m[h][j].x : b.x + x.m[h][j].x;
             b.y = c ? b.y - x.m[h][j].y : b.y + x.m[h][j].y;
+            b.x = ok0 ? b.x : 0.0;  // the packed rows end in zeros, the clamped rows do not
+            b.y = ok1 ? b.y : 0.0;
           }
-          b.x = ok0 ? b.x : 0.0;
-          b.y = ok1 ? b.y : 0.0;
 #pragma unroll
           for (int i = 0; i < FM; ++i) {
             const double2 a = x.a[c][h][i];
@@ -235,7 +263,8 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
     add_quarters<NC * FM * FN>(part, wid, lane, [&](int e, int r) { return acc[e / (FM * FN)][e / FN % FM][e % FN][r]; },
                                [&](int e, double v) { res[e / (FM * FN)][e / FN % FM][e % FN][0] = v; });
   } else {
-    v4d sum[NC][FM][FN], pair[NC][FM][FN];
+    v4d pair[NC][FM][FN];
+    __shared__ v4d sum[NC][FM][FN][256];
     if (any) {
       load(0, x);
 #pragma unroll
@@ -247,10 +276,10 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
           for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
-              if (q == 0) sum[c][i][j] = acc[c][i][j];
+              if (q == 0) sum[c][i][j][tid] = acc[c][i][j];
               else if (q == 2) pair[c][i][j] = acc[c][i][j];
-              else if (q == 1) sum[c][i][j] += acc[c][i][j];
-              else acc[c][i][j] = sum[c][i][j] + (pair[c][i][j] + acc[c][i][j]);
+              else if (q == 1) sum[c][i][j][tid] += acc[c][i][j];
+              else acc[c][i][j] = sum[c][i][j][tid] + (pair[c][i][j] + acc[c][i][j]);
             }
       }
     } else {
@@ -303,10 +332,10 @@ __global__ __launch_bounds__(256) void xgemm_kernel(XArgs<NG> ar) {
 //   u = bs T_ux, v = bs T_uy, and per field d/dx q = bs D_q, d/dy q = bds T_q,
 // of two parity classes each, combined point by point.  NF = 1: one field per block, u and v formed
 // again for each; NF = 3: the three fields in one block (8 products in place of 12, on 16 tiles of
-// accumulators per wavefront, so one block per CU).  One launch in place of four (the velocity, two
+// accumulators per wavefront).  One launch in place of four (the velocity, two
 // products with an epilogue, the boundary field's gradient).
-template <int CH, int NF>
-__global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
+template <int CH, int NF, int W>
+__global__ __launch_bounds__(256, W) void conv_kernel(ConvArgs a, int tx, int ty) {
   constexpr int ND = NF == 3 ? 6 : 4, NP = NF == 3 ? 8 : 4;  // data arrays, products
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
@@ -321,17 +350,18 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
   for (int i = 0; i < ND; ++i) {
     const int ff = NF == 3 ? i % 3 : i < 2 ? i : f;
     src[i] = (NF == 3 ? i < 3 : i != 2) ? a.T : a.D;
-    src[i] += a.stride * (ff * a.nb + b) + col;
+    src[i] += a.stride * (ff * a.nb + b);
   }
+  const unsigned at0 = 8u * (unsigned)(4 * lk * N + col), at1 = at0 + 16u * (unsigned)N;
   const double* opa[2][2];  // [bs, bds][class]
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    opa[0][c] = a.bs.a[c] + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
-    opa[1][c] = a.bds.a[c] + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
+    opa[0][c] = a.bs.a[c] + (size_t)(m0 >> 4) * G * 128;
+    opa[1][c] = a.bds.a[c] + (size_t)(m0 >> 4) * G * 128;
   }
   // rows of row parity p: 2 k + p below cols; class c of bs takes parity rb[c], of bds rd[c]
   const int Kp[2] = {a.bs.r0[0] == 0 ? a.bs.K[0] : a.bs.K[1], a.bs.r0[0] == 0 ? a.bs.K[1] : a.bs.K[0]};
-  const int b0 = a.bs.r0[0], d0 = a.bds.r0[0];  // parity of class 0
+  const int pb = a.bs.r0[0], pd = a.bds.r0[0];  // parity of class 0
   struct Chunk {
     double2 o[2][2][CH], d[ND][2][CH];  // [operator][class], [array][row parity]
   };
@@ -345,34 +375,30 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
     for (int h = 0; h < CH; ++h)
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        const int k = (g0 + h) * 8 + 2 * lk;
 #pragma unroll
-        for (int p = 0; p < 2; ++p) x.o[p][c][h] = *reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128);
-        const long q0 = (long)(c + 2 * min(k, Kp[c] - 1)) * N, q1 = (long)(c + 2 * min(k + 1, Kp[c] - 1)) * N;
+        for (int p = 0; p < 2; ++p)
+          x.o[p][c][h] = reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128)[lane];
 #pragma unroll
-        for (int i = 0; i < ND; ++i) x.d[i][c][h] = double2{src[i][q0], src[i][q1]};
+        for (int i = 0; i < ND; ++i) {
+          const Buffer w = rows_from(src[i] + c * N, (long)(g0 + h) * 16 * N, (long)(2 * Kp[c] - 1) * N);
+          x.d[i][c][h] = double2{value_at(w, at0), value_at(w, at1)};
+        }
       }
   };
   // operator and data array of product p
   auto op_of = [](int p) { return NF == 3 ? p >= 5 : p == 3; };
   auto data_of = [](int p) { return NF == 3 ? (p < 2 ? p : p < 5 ? p + 1 : p - 5) : p; };
-  auto mac = [&](int g0, const Chunk& x) {
+  auto mac = [&](const Chunk& x) {
 #pragma unroll
     for (int h = 0; h < CH; ++h) {
-      const int k = (g0 + h) * 8 + 2 * lk;
-      double2 d[ND][2];
-#pragma unroll
-      for (int i = 0; i < ND; ++i)
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-          d[i][c] = double2{k < Kp[c] ? x.d[i][c][h].x : 0.0, k + 1 < Kp[c] ? x.d[i][c][h].y : 0.0};
 #pragma unroll
       for (int p = 0; p < NP; ++p)
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           const double2 o = x.o[op_of(p) ? 1 : 0][c][h];
-          const bool odd = (c ^ (op_of(p) ? d0 : b0)) != 0;
-          const double v0 = odd ? d[data_of(p)][1].x : d[data_of(p)][0].x, v1 = odd ? d[data_of(p)][1].y : d[data_of(p)][0].y;
+          const bool odd = (c ^ (op_of(p) ? pd : pb)) != 0;
+          const double2 &d0 = x.d[data_of(p)][0][h], &d1 = x.d[data_of(p)][1][h];
+          const double v0 = odd ? d1.x : d0.x, v1 = odd ? d1.y : d0.y;
           acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.x, v0, acc[p][c], 0, 0, 0);
           acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.y, v1, acc[p][c], 0, 0, 0);
         }
@@ -384,11 +410,11 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
   int n = 0;
   for (; n + 2 <= nch; n += 2) {
     load(min(g0 + (n + 1) * CH, top), y);
-    mac(g0 + n * CH, x);
+    mac(x);
     load(min(g0 + (n + 2) * CH, top), x);
-    mac(g0 + (n + 1) * CH, y);
+    mac(y);
   }
-  if (n < nch) mac(g0 + n * CH, x);
+  if (n < nch) mac(x);
   const int ny = a.bs.rows;
   double res[NP][2];
   __shared__ double part[8 * 16 * 64];
@@ -429,7 +455,7 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a, int tx, int ty) {
 // of the residuals' x-transformed values T and derivatives D, taken with the fields' values at the
 // point: one launch in place of 14 terms of four launches each.
 template <int CH>
-__global__ __launch_bounds__(256) void adjoint_kernel(AdjointConvArgs a, int tx, int ty) {
+__global__ __launch_bounds__(256, 2) void adjoint_kernel(AdjointConvArgs a, int tx, int ty) {
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   int t = fftlds::xcd_remap(blockIdx.x, gridDim.x);
@@ -448,11 +474,12 @@ __global__ __launch_bounds__(256) void adjoint_kernel(AdjointConvArgs a, int tx,
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const double* base = op[p] ? a.bds.a[c] : a.bs.a[c];
-      opa[p][c] = base + ((size_t)(m0 >> 4) * G * 64 + lane) * 2;
+      opa[p][c] = base + (size_t)(m0 >> 4) * G * 128;
       const int r0 = op[p] ? a.bds.r0[c] : a.bs.r0[c];
       K[p][c] = op[p] ? a.bds.K[c] : a.bs.K[c];
-      src[p][c] = (op[p] ? a.T : a.D) + a.stride * field[p] + (long)r0 * N + col;
+      src[p][c] = (op[p] ? a.T : a.D) + a.stride * field[p] + (long)r0 * N;
     }
+  const unsigned at0 = 8u * (unsigned)(4 * lk * N + col), at1 = at0 + 16u * (unsigned)N;
   struct Chunk {
     double2 o[4][2][CH], d[4][2][CH];
   };
@@ -468,23 +495,20 @@ __global__ __launch_bounds__(256) void adjoint_kernel(AdjointConvArgs a, int tx,
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-          const int k = (g0 + h) * 8 + 2 * lk;
-          x.o[p][c][h] = *reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128);
-          x.d[p][c][h] = double2{src[p][c][(long)2 * min(k, K[p][c] - 1) * N],
-                                 src[p][c][(long)2 * min(k + 1, K[p][c] - 1) * N]};
+          x.o[p][c][h] = reinterpret_cast<const double2*>(opa[p][c] + (size_t)(g0 + h) * 128)[lane];
+          const Buffer w = rows_from(src[p][c], (long)(g0 + h) * 16 * N, (long)(2 * K[p][c] - 1) * N);
+          x.d[p][c][h] = double2{value_at(w, at0), value_at(w, at1)};
         }
   };
-  auto mac = [&](int g0, const Chunk& x) {
+  auto mac = [&](const Chunk& x) {
 #pragma unroll
     for (int h = 0; h < CH; ++h)
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-          const int k = (g0 + h) * 8 + 2 * lk;
-          const double v0 = k < K[p][c] ? x.d[p][c][h].x : 0.0, v1 = k + 1 < K[p][c] ? x.d[p][c][h].y : 0.0;
-          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.o[p][c][h].x, v0, acc[p][c], 0, 0, 0);
-          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.o[p][c][h].y, v1, acc[p][c], 0, 0, 0);
+          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.o[p][c][h].x, x.d[p][c][h].x, acc[p][c], 0, 0, 0);
+          acc[p][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(x.o[p][c][h].y, x.d[p][c][h].y, acc[p][c], 0, 0, 0);
         }
   };
   Chunk x, y;
@@ -493,11 +517,11 @@ __global__ __launch_bounds__(256) void adjoint_kernel(AdjointConvArgs a, int tx,
   int n = 0;
   for (; n + 2 <= nch; n += 2) {
     load(min(g0 + (n + 1) * CH, top), y);
-    mac(g0 + n * CH, x);
+    mac(x);
     load(min(g0 + (n + 2) * CH, top), x);
-    mac(g0 + (n + 1) * CH, y);
+    mac(y);
   }
-  if (n < nch) mac(g0 + n * CH, x);
+  if (n < nch) mac(x);
   const int ny = a.bs.rows;
   double res[4][2];
   __shared__ double part[8 * 16 * 64];
@@ -552,7 +576,7 @@ void launch_tile(hipStream_t s, const XGemm* groups, int tile) {
   switch (tile) {
     case TILE_16: launch<1, 1, true, CH, KIND, NG, TR>(s, groups); break;
     case TILE_32: launch<2, 1, true, CS, KIND, NG, TR>(s, groups); break;
-    default: launch<2, 2, false, CS, KIND, NG, TR>(s, groups); break;
+    default: launch<2, 2, false, 1, KIND, NG, TR>(s, groups); break;
   }
 }
 
@@ -602,30 +626,34 @@ int xop_groups(int K) {
 
 void conv_products(hipStream_t s, const ConvArgs& a) {
   if (a.bs.kind != XOP_FOLD_OUT || a.bds.kind != XOP_FOLD_OUT || a.bs.groups != a.bds.groups ||
-      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.f0 < 0 || a.f1 > 3 || a.f0 >= a.f1 || a.nx < 1 || a.nb < 1)
+      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.f0 < 0 || a.f1 > 3 || a.f0 >= a.f1 || a.nx < 1 || a.nx > (1 << 24) || a.nb < 1)
     throw std::invalid_argument("conv_products: bad arguments");
   if (a.bs.rstep != 2 || a.bds.rstep != 2) throw std::invalid_argument("conv_products: bad operators");
   const int tx = (a.nx + 15) / 16, ty = (a.bs.M[0] + 15) / 16;
   const long tiles = (long)tx * ty * a.nb;
-  // the three fields in one block where their tiles, times groups of 8 k values, fill the chip anyway
-  // (one / three fields per block: 128^2, 1 instance (256): 5.7 / 8.9 us, 3 (768): 10.0 / 9.4; 192^2,
-  // 1 (864): 7.6 / 10.8; 64^2, 36 (1,152): 10.6 / 11.0; 96^2, 12 (1,728): 14.8 / 9.1; 257^2, 1 (2,448):
-  // 17.7 / 15.3; 128^2, 36 (9,216): 61 / 40).  A wavefront per tile with the whole k range is no faster
-  // (192^2, 36: 85 us against 100, but 32 against 38 at 12 and 11 against 30 at 3).
-  const bool three = a.f0 == 0 && a.f1 == 3 && tiles * a.bs.groups >= 1200;
+  // one field per block while these are at most two per CU, else the three in one (us, one / three: 64^2,
+  // 12 instances (288 blocks of one field) 5.3 / 6.1, 36 (864) 9.6 / 7.6; 96^2, 6 (324) 7.1 / 8.9, 12 (648)
+  // 10.6 / 8.8; 128^2, 6 (576) 10.6 / 9.6; 192^2, 2 (432) 9.2 / 11.0, 3 (648) 12.9 / 11.0; 257^2, 1 (459)
+  // 13.2 / 13.5, 3 (1,377) 30.5 / 23.2, 12 98.6 / 71.3).  A wavefront per tile with the whole k range is no
+  // faster (192^2, 36: 85 us against 67, 3: 30 against 11).
+  const bool three = a.f0 == 0 && a.f1 == 3 && 3 * tiles > 512;
   const long total = tiles * (three ? 1 : a.f1 - a.f0);
   if (total > 0x7fffffffL) throw std::invalid_argument("conv_products: too many tiles");
   const dim3 grid((unsigned)total), block(256);
-  if (three) RBC_LAUNCH((conv_kernel<1, 3>), grid, block, 0, s, a, tx, ty);
-  else if (a.bs.groups / 4 % 2 == 0) RBC_LAUNCH((conv_kernel<2, 1>), grid, block, 0, s, a, tx, ty);
-  else RBC_LAUNCH((conv_kernel<1, 1>), grid, block, 0, s, a, tx, ty);
+  // W blocks per CU: two hide each other's loads and sums (257^2, 12 instances: 87 us with one, 71 with
+  // two; 128^2, 12: 16.0 / 14.2); where there is one per CU at most it takes all registers (153 blocks, 257^2:
+  // 13.5 with one, 15.3 with two)
+  if (three && tiles <= 256) RBC_LAUNCH((conv_kernel<1, 3, 1>), grid, block, 0, s, a, tx, ty);
+  else if (three) RBC_LAUNCH((conv_kernel<1, 3, 2>), grid, block, 0, s, a, tx, ty);
+  else if (a.bs.groups / 4 % 2 == 0) RBC_LAUNCH((conv_kernel<2, 1, 2>), grid, block, 0, s, a, tx, ty);
+  else RBC_LAUNCH((conv_kernel<1, 1, 2>), grid, block, 0, s, a, tx, ty);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw std::runtime_error(std::string("conv_products: ") + hipGetErrorString(e));
 }
 
 void adjoint_products(hipStream_t s, const AdjointConvArgs& a) {
   if (a.bs.kind != XOP_FOLD_OUT || a.bds.kind != XOP_FOLD_OUT || a.bs.groups != a.bds.groups ||
-      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.bs.rstep != 2 || a.bds.rstep != 2 || a.nx < 1)
+      a.bs.rows != a.bds.rows || a.bs.cols != a.bds.cols || a.bs.rstep != 2 || a.bds.rstep != 2 || a.nx < 1 || a.nx > (1 << 24))
     throw std::invalid_argument("adjoint_products: bad arguments");
   const int tx = (a.nx + 15) / 16, ty = (a.bs.M[0] + 15) / 16;
   const long total = 3L * tx * ty;
@@ -642,21 +670,28 @@ void adjoint_products(hipStream_t s, const AdjointConvArgs& a) {
 //   128^2 x 36 (18,432):                  5.76 / 5.34  (9.04)     257^2 x 3 (22,032): 6.50 / 5.81  (10.3)
 //   192^2 x 36 (62,208):                  12.3 / 10.2  (19.0)     257^2 x 36 (264,384): 36.8 / 28.8  (45.6)
 //   64^2 x 3 (384): 2.47 / 2.79 (4.00), of which 1.66 is an empty launch.
-// Beyond a million the wavefronts of a block take a tile of their own each, 64 x 64 together, which
-// halves the loads per product: 510^2 x 64 (2.1 million) 179 us, 47 TFLOP/s, against 195 us.
+// Beyond 400,000 the wavefronts of a block take a tile of their own each, 64 x 64 together, which halves
+// the loads per product, unless the larger tiles are more than a tenth of padding (32 x 16 / 64 x 64:
+// 510^2 x 64 (2.1 million) 216 / 168, 50.5 TFLOP/s, 510^2 x 16 (524,288) 51 / 40, 510^2 x 4 (131,072) 14.5 /
+// 14.5, folding in 512^2 x 8 (262,144) 29.4 / 31.7; 300^2 x 36, a quarter of padding, 33 / 44).  The sum of
+// their first two quarters waits in LDS and the registers are bounded for two blocks per CU: 510^2 x 64
+// takes 186 us with the sum in registers, 182 without the bound.
 static void xgemm_any(hipStream_t s, const XGemm* in, int ng, bool transposed) {
   if (ng < 1 || ng > XGEMM_GROUPS) throw std::invalid_argument("xgemm: bad group count");
   XGemm groups[XGEMM_GROUPS];
   bool out = false;
-  long size = 0;
+  long size = 0, size64 = 0;  // the latter with the padding of 64 x 64 tiles
   for (int i = 0; i < ng; ++i) {
     const XGemm& g = groups[i] = in[i];
     out = out || g.op.kind == XOP_FOLD_OUT;
     if (g.entries < 1 || g.N < 1 || g.op.M[0] < 1 || !g.B || !g.C || g.op.M[1] > g.op.M[0])
       throw std::invalid_argument("xgemm: bad sizes");
+    if (g.ldb > (1 << 24) || g.ldb < g.N) throw std::invalid_argument("xgemm: rows too long");
     if (g.op.groups != in[0].op.groups) throw std::invalid_argument("xgemm: the groups' operators differ in length");
     const int ncls = g.op.kind == XOP_DENSE ? 1 : 2;
-    size += (long)((g.N + 15) / 16) * ((g.op.M[0] + 15) / 16) * ncls * g.entries * g.op.groups;
+    const long per = (long)ncls * g.entries * g.op.groups;
+    size += (long)((g.N + 15) / 16) * ((g.op.M[0] + 15) / 16) * per;
+    size64 += 16L * ((g.N + 63) / 64) * ((g.op.M[0] + 63) / 64) * per;
   }
   if (ng > 1) {
     for (int i = 0; i < ng; ++i)
@@ -668,7 +703,7 @@ static void xgemm_any(hipStream_t s, const XGemm* in, int ng, bool transposed) {
     }
   }
   const int kind = out ? (int)XOP_FOLD_OUT : groups[0].op.kind, ch = xop_chunk(groups[0].op.groups);
-  const int tile = size < 18000 ? TILE_16 : size < 1000000 ? TILE_32 : TILE_64;
+  const int tile = size < 18000 ? TILE_16 : size < 400000 || 10 * size64 > 11 * size ? TILE_32 : TILE_64;
   if (transposed) launch_kind<true>(s, groups, ng, kind, tile, ch);
   else launch_kind<false>(s, groups, ng, kind, tile, ch);
   hipError_t e = hipGetLastError();
