@@ -47,37 +47,52 @@ __device__ __forceinline__ double xy_taps(const double* __restrict__ q, int mx, 
   return (i < my ? v0 * cy0 : 0.0) + (i >= 2 ? v2 * cy1 : 0.0);
 }
 
+// one block per row and field: 128 x 129 3.5 us, 257 x 257 6.5 (5.7 and 8.6 with the three fields of a row
+// in one block, two wavefronts a CU)
 template <int SLICE>
 __global__ __launch_bounds__(NT) void rhs_rows_kernel(ConfinedRows a, int per) {
 #pragma clang fp contract(off)
   extern __shared__ double buf[];
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), p = tid / WAVE;
-  const int r = blockIdx.x, n = a.ny;
-  const long o = a.stride * blockIdx.y, at = (long)r * n;
+  const int r = blockIdx.x, n = a.ny, f = a.f0 + blockIdx.z;
+  const long o = a.stride * blockIdx.y, at = o + (long)r * n;
   constexpr int MAXQ = (2 * SLICE * WAVE + 8 + NT - 1) / NT;
-  if (a.f0 <= 1 && a.f1 > 1) {  // uy: d/dy pres
-    chains::stage_row<MAXQ>(buf, a.P0 + o + at, true, n, tid, NT);
+  const double* U = a.U + f * a.field + o;
+  double* out = a.RHS + f * a.field + at;
+  const double* cv = a.CV + f * a.field + at;
+  const double x0 = f == 2 ? a.sxt[r] : a.sxu[r], x1 = f == 2 ? a.sxt[a.nx + r] : a.sxu[a.nx + r];
+  if (f == 1) {  // d/dy pres, buoyancy
+    chains::stage_row<MAXQ>(buf, a.P0 + at, true, n, tid, NT);
+    const double xt0 = a.sxt[r], xt1 = a.sxt[a.nx + r];
+    double v[MAXQ], t[MAXQ];
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * NT;
+      v[q] = t[q] = 0.0;
+      if (i >= n) continue;
+      const double cy0 = a.sy[i], cy1 = a.sy[n + i];
+      v[q] = xy_taps(U, a.mx, a.my, r, i, x0, x1, cy0, cy1);
+      t[q] = xy_taps(a.U + 2 * a.field + o, a.mx, a.my, r, i, xt0, xt1, cy0, cy1) + a.that_bc[at + i];
+    }
     __syncthreads();
     rowdiff::derive<SLICE>(buf, n, per, lane, p);
+#pragma unroll
+    for (int q = 0; q < MAXQ; ++q) {
+      const int i = tid + q * NT;
+      if (i >= n) continue;
+      double w = v[q] - (buf[pad(i + 2)] * a.inv_scy) * a.dt;
+      w = w + t[q] * a.dt;
+      out[i] = w - cv[i] * a.dt;
+    }
+    return;
   }
-  const double xu0 = a.sxu[r], xu1 = a.sxu[a.nx + r], xt0 = a.sxt[r], xt1 = a.sxt[a.nx + r];
-  for (int i = tid; i < n; i += NT) {
-    const double cy0 = a.sy[i], cy1 = a.sy[n + i];
-    const long j = o + at + i;
-    const double t = a.f1 > 1 ? xy_taps(a.U + 2 * a.field + o, a.mx, a.my, r, i, xt0, xt1, cy0, cy1) : 0.0;
-    if (a.f0 <= 0 && a.f1 > 0) {
-      const double u = xy_taps(a.U + o, a.mx, a.my, r, i, xu0, xu1, cy0, cy1);
-      const double v = u - a.G[j] * a.dt;
-      a.RHS[j] = v - a.CV[j] * a.dt;
-    }
-    if (a.f0 <= 1 && a.f1 > 1) {
-      const double u = xy_taps(a.U + a.field + o, a.mx, a.my, r, i, xu0, xu1, cy0, cy1);
-      double v = u - (buf[pad(i + 2)] * a.inv_scy) * a.dt;
-      v = v + (t + a.that_bc[j]) * a.dt;
-      a.RHS[a.field + j] = v - a.CV[a.field + j] * a.dt;
-    }
-    if (a.f0 <= 2 && a.f1 > 2)
-      a.RHS[2 * a.field + j] = ((t + a.gxx[j]) + a.gyy[j]) - a.CV[2 * a.field + j] * a.dt;
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int i = tid + q * NT;
+    if (i >= n) continue;
+    const double u = xy_taps(U, a.mx, a.my, r, i, x0, x1, a.sy[i], a.sy[n + i]);
+    const double w = f == 0 ? u - a.G[at + i] * a.dt : (u + a.gxx[at + i]) + a.gyy[at + i];
+    out[i] = w - cv[i] * a.dt;
   }
 }
 
@@ -112,10 +127,43 @@ __global__ __launch_bounds__(NT) void div_rows_kernel(ConfinedRows a, int per) {
   __syncthreads();
   rowdiff::derive<SLICE>(buf, n, per, lane, p);
   double* out = a.DIV + o + (long)r * n;
+  double sum = 0.0;
 #pragma unroll
   for (int q = 0; q < MAXQ; ++q) {
     const int i = tid + q * NT;
-    if (i < n) out[i] = buf[pad(i + 2)] * a.inv_scy + w[q];
+    if (i >= n) continue;
+    const double d = buf[pad(i + 2)] * a.inv_scy + w[q];
+    if (a.norm) sum += d * d;
+    else out[i] = d;
+  }
+  if (!a.norm) return;
+  // the sum of squares instead: the rows' sums are added by the last block to arrive, which leaves the
+  // counter at zero
+  __shared__ double red[NT];
+  __shared__ bool last;
+  auto add = [&](double v) {
+    red[tid] = v;
+    __syncthreads();
+    for (int h = NT / 2; h > 0; h >>= 1) {
+      if (tid < h) red[tid] += red[tid + h];
+      __syncthreads();
+    }
+  };
+  add(sum);
+  unsigned* count = reinterpret_cast<unsigned*>(a.part);
+  if (tid == 0) {
+    __hip_atomic_store(a.part + 1 + r, red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  sum = 0.0;
+  for (int i = tid; i < (int)gridDim.x; i += NT)
+    sum += __hip_atomic_load(a.part + 1 + i, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+  add(sum);
+  if (tid == 0) {
+    *a.norm = red[0];
+    __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -291,9 +339,9 @@ static void check_args(const ConfinedRows& a, int nb) {
   if (nb < 1 || nb > 65535 || a.f0 < 0 || a.f1 > 3 || a.f0 > a.f1) throw std::invalid_argument("confined rows: bad batch");
 }
 
-#define RBC_CONFINED(KERNEL, per, blocks, ...)                                               \
+#define RBC_CONFINED(KERNEL, per, blocks, fields, ...)                                       \
   do {                                                                                       \
-    const dim3 grid((unsigned)(blocks), nb), block(NT);                                      \
+    const dim3 grid((unsigned)(blocks), nb, fields), block(NT);                              \
     const size_t lds = buf_len(a.ny) * sizeof(double);                                       \
     if ((per) <= 2) RBC_LAUNCH(KERNEL<2>, grid, block, lds, s, __VA_ARGS__);                 \
     else if ((per) <= 4) RBC_LAUNCH(KERNEL<4>, grid, block, lds, s, __VA_ARGS__);                 \
@@ -304,13 +352,15 @@ static void check_args(const ConfinedRows& a, int nb) {
 void rhs_rows(hipStream_t s, const ConfinedRows& a, int nb) {
   check_args(a, nb);
   const int per = fdma_rows_lds_per(a.ny);
-  RBC_CONFINED(rhs_rows_kernel, per, a.nx, a, per);
+  if (a.f0 == a.f1) return;
+  RBC_CONFINED(rhs_rows_kernel, per, a.nx, a.f1 - a.f0, a, per);
   check("rhs_rows");
 }
 void div_rows(hipStream_t s, const ConfinedRows& a, int nb) {
   check_args(a, nb);
   const int per = fdma_rows_lds_per(a.ny);
-  RBC_CONFINED(div_rows_kernel, per, a.nx, a, per);
+  if (a.norm && (nb != 1 || !a.part)) throw std::invalid_argument("div_rows: the norm of one instance");
+  RBC_CONFINED(div_rows_kernel, per, a.nx, 1, a, per);
   check("div_rows");
 }
 void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure) {
@@ -319,7 +369,7 @@ void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure) {
   const int per_n = fdma_rows_lds_per(a.ny), per = fdma_rows_lds_per(a.my);
   const int blocks = (a.f1 - a.f0) * a.mx + (pressure ? a.nx : 0);
   if (blocks == 0) return;
-  RBC_CONFINED(proj_rows_kernel, per_n, blocks, a, per_n, per);
+  RBC_CONFINED(proj_rows_kernel, per_n, blocks, 1, a, per_n, per);
   check("proj_rows");
 }
 

@@ -691,7 +691,7 @@ class Navier {
   // rows of THAT_BC, GXX and GYY (spectral, [rows, ny]) before which every value is +0.0
   int bc_rows = 0;
   // workspaces
-  DBuf THAT, UXP, UYP, A, G, CONV, CV, RHS, DIV, W1, W2, W3, W4, W9, NRM;
+  DBuf THAT, UXP, UYP, A, G, CONV, CV, RHS, DIV, W1, W2, W3, W4, W9, NRM, DVN;
   std::vector<double> wx_dx, wy_dx;  // cell widths of `field` (unscaled, field.rs:135-163)
   double len0 = 0, len1 = 0;
   DBuf DX0, DX1;
@@ -2571,13 +2571,19 @@ class Navier {
   }
   double div_norm() {
     const long no = (long)rows_ortho(bx_u) * ny;
-    // one product and one row kernel in place of five launches (not an ensemble's instance, whose ux
-    // and uy lie in slabs of their group)
+    // one product and one row kernel, which forms the sum, in place of eight operations (not an ensemble's
+    // instance, whose ux and uy lie in slabs of their group).  Launches bound it: a 64 x 64 run under
+    // integrate(), which tests exit() after each step, takes 66 us per step, 101 with the eight.
     if (nb == 1 && UY.p == UX.p + pair_off() && confined_fused_ok()) {
-      divergence_confined(confined_rows(), G.p);
-    } else {
-      divergence(G.p);
+      ConfinedRows a = confined_rows();
+      if (DVN.n < (size_t)nx + 1) DVN.alloc(nx + 1);
+      a.norm = pinned();
+      a.part = DVN.p;
+      divergence_confined(a, nullptr);
+      HIPCHECK(hipStreamSynchronize(st));
+      return std::sqrt(*norm_host);
     }
+    divergence(G.p);
     return std::sqrt(read_norm(G.p, no));
   }
   // sum of squares of n device values, formed into pinned host memory: no copy follows the kernel

@@ -479,10 +479,8 @@ void col_weighted_sum(hipStream_t s, const double* v, int n0, int n1, const doub
 }
 
 // The partial sums are added by the last block to arrive, and the result may lie in pinned host memory:
-// one launch in place of three operations (two launches and a copy to pageable memory).  Launches bound
-// it: a confined 64^2 run under integrate(), which tests exit() after each step, takes 73 us per step
-// (101 before, with the divergence in five launches).  The counter, at part[NSUM], returns to zero for
-// the next call.
+// one launch in place of three operations (two launches and a copy to pageable memory).  The counter, at
+// part[NSUM], returns to zero for the next call.
 constexpr int NSUM = SUM_SQUARES_PART - 1;
 __global__ __launch_bounds__(256) void sum_squares_kernel(const double* __restrict__ b, long n, double* __restrict__ part,
                                                           double* __restrict__ out) {

@@ -322,6 +322,9 @@ struct ConfinedRows {
   int nx, ny, mx, my, f0, f1;
   long field, stride;
   double dt, inv_dt, inv_scy, nu;
+  // div_rows: when set, *norm (device or pinned host memory) = the sum of squares of the divergence, which
+  // is not written; part holds 1 + nx doubles, the first of them zero before the first call
+  double *norm, *part;
 };
 bool confined_rows_supported(int nx, int ny);
 

@@ -11,6 +11,7 @@
 // (15 us a launch; the rest is each call's wait).
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <stdexcept>
 #include <string>
 
@@ -39,7 +40,7 @@ template <int SLICE, bool CPLX>
 __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* __restrict__ in, double* __restrict__ out,
                                                                  long rows, int mi, int n, int per, int bl,
                                                                  const double* __restrict__ coef, int d1, int d0, int m0,
-                                                                 double sc) {
+                                                                 double sc, double isc) {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
@@ -97,7 +98,10 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
     const double ns = sc * sc + 0.0 * 0.0;
     for (int i = threadIdx.x; i < n; i += WAVE * WAVES) {
       double a = lds[pad(i + 2)], b = lds[bl + pad(i + 2)];
-      if (sc != 1.0) {  // num-complex division by (sc, 0)
+      if (isc != 0.0) {  // sc a power of two: the same value (and sign of a zero) without the division
+        a = (a * sc + b * 0.0) * isc * isc;
+        b = (b * sc - a * 0.0) * isc * isc;
+      } else if (sc != 1.0) {  // num-complex division by (sc, 0)
         const double na = (a * sc + b * 0.0) / ns, nb = (b * sc - a * 0.0) / ns;
         a = na;
         b = nb;
@@ -186,6 +190,7 @@ bool row_ops_supported(int n) { return n >= 6 && fdma_rows_lds_per(n) <= 16; }
     const dim3 grid((unsigned)((CPLX) ? rows : (rows + 1) / 2)), block(WAVE * WAVES);                         \
     if ((per) <= 2) RBC_LAUNCH((KERNEL<2, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
     else if ((per) <= 4) RBC_LAUNCH((KERNEL<4, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
+    else if ((per) <= 6) RBC_LAUNCH((KERNEL<6, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__); \
     else if ((per) <= 8) RBC_LAUNCH((KERNEL<8, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__); \
     else RBC_LAUNCH((KERNEL<16, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);                \
   } while (0)
@@ -196,8 +201,10 @@ void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cp
     throw std::invalid_argument("ortho_rows: bad arguments");
   if (rows < 1 || rows > 0x3fffffff) throw std::invalid_argument("ortho_rows: bad rows");
   const int per = fdma_rows_lds_per(n), bl = buf_len(n);
-  if (cplx) RBC_ROW_OP(ortho_rows_kernel, true, per, in, out, rows, mi, n, per, bl, coef, d1, d0, m0, sc);
-  else RBC_ROW_OP(ortho_rows_kernel, false, per, in, out, rows, mi, n, per, bl, coef, d1, 0, 1, sc);
+  int ex = 0;
+  const double isc = sc > 0.0 && sc != 1.0 && std::frexp(sc, &ex) == 0.5 ? 1.0 / sc : 0.0;
+  if (cplx) RBC_ROW_OP(ortho_rows_kernel, true, per, in, out, rows, mi, n, per, bl, coef, d1, d0, m0, sc, isc);
+  else RBC_ROW_OP(ortho_rows_kernel, false, per, in, out, rows, mi, n, per, bl, coef, d1, 0, 1, sc, 0.0);
   check("ortho_rows");
 }
 
