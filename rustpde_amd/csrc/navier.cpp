@@ -2661,6 +2661,10 @@ class Space {
     xgemm(st, &g, 1);
     return out;
   }
+  // the transform along y (op 0 forward, 1 backward) by fast transforms: yop's first branch
+  bool y_fast(int op) const {
+    return (b1.k == CHEB || b1.k == CD || b1.k == CN) && cheb_y_supported(b1.n) && (op == 1 || b1.k == CHEB || rows_ok());
+  }
   // y-operator on `rows` consecutive real rows
   const double* yop(const char* name, const double* in, long rows, double* out) {
     const std::string op_name = name;
@@ -2755,6 +2759,17 @@ class Space {
       }
       irfft_cols_interleaved(st, src, W1.p, b0.n, b1.m, nb);
       return yop("BS", W1.p, (long)nb * b0.n, dst);
+    }
+    if (!cplx && op < 2 && !y_fast(op)) {  // both products with transposed results, parity classes along both axes
+      const char* name = op == 0 ? "FS" : "BS";
+      const PackedOp &px = X.packed(b0, name), &py = Y.packed(b1, name);
+      XGemm g = xgemm_of(px, src, W1.p, py.op.cols, nb, (long)px.op.cols * py.op.cols, (long)px.op.rows * py.op.cols);
+      g.ldc = px.op.rows;
+      xgemm_t(st, &g, 1);
+      g = xgemm_of(py, W1.p, dst, px.op.rows, nb, (long)px.op.rows * py.op.cols, (long)px.op.rows * py.op.rows);
+      g.ldc = py.op.rows;
+      xgemm_t(st, &g, 1);
+      return dst;
     }
     const bool in_c = cplx && op != 0, out_c = cplx && op != 1;
     const double* x = src;
