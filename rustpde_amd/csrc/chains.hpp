@@ -82,45 +82,48 @@ __device__ __forceinline__ void unstage_row(const double* buf, double* __restric
 // state, so both halves are replayed side by side: two independent dependency chains per
 // lane instead of one.
 
-// Fdma forward elimination (fdma.rs:101-118): y_t = x_t - y_{t-1} lo_t (lo_t = low[i - 2])
-template <int SLICE>
-__device__ __forceinline__ void fdma_forward(double (&v)[SLICE], const double (&lo)[SLICE], int lane, int t0,
+// Fdma forward elimination (fdma.rs:101-118): y_t = x_t - y_{t-1} lo_t (lo_t = low[i - 2]), of NR
+// right-hand sides with the same multipliers
+template <int SLICE, int NR>
+__device__ __forceinline__ void fdma_forward(double (&v)[NR][SLICE], const double (&lo)[SLICE], int lane, int t0,
                                              int cnt) {
 #pragma clang fp contract(off)
   static_assert(SLICE % 2 == 0, "two half slices");
   constexpr int H = SLICE / 2;
-  double A1 = 1.0, B1 = 0.0, A2 = 1.0, B2 = 0.0;  // half maps y_out = A y_in + B
+  double A1 = 1.0, A2 = 1.0, B1[NR] = {}, B2[NR] = {};  // half maps y_out = A y_in + B
 #pragma unroll
   for (int j = 0; j < H; ++j) {
     if (j < cnt) {
-      if (t0 + j == 0) {
-        A1 = 0.0;
-        B1 = v[j];
-      } else {
-        A1 = -A1 * lo[j];
-        B1 = v[j] - B1 * lo[j];
-      }
+      const bool start = t0 + j == 0;
+      A1 = start ? 0.0 : -A1 * lo[j];
+#pragma unroll
+      for (int k = 0; k < NR; ++k) B1[k] = start ? v[k][j] : v[k][j] - B1[k] * lo[j];
     }
     const int q = H + j;
     if (q < cnt) {
       A2 = -A2 * lo[q];
-      B2 = v[q] - B2 * lo[q];
+#pragma unroll
+      for (int k = 0; k < NR; ++k) B2[k] = v[k][q] - B2[k] * lo[q];
     }
   }
-  double b[1] = {A2 * B1 + B2}, y[1];  // lane map
-  wave::scan_states<false>(A2 * A1, b, lane, y);
-  double y1 = y[0];
-  double y2 = A1 * y1 + B1;
+  double b[NR], y[NR];  // lane map
 #pragma unroll
-  for (int j = 0; j < H; ++j) {
-    if (j < cnt) {
-      y1 = (t0 + j == 0) ? v[j] : v[j] - y1 * lo[j];
-      v[j] = y1;
-    }
-    const int q = H + j;
-    if (q < cnt) {
-      y2 = v[q] - y2 * lo[q];
-      v[q] = y2;
+  for (int k = 0; k < NR; ++k) b[k] = A2 * B1[k] + B2[k];
+  wave::scan_states<false>(A2 * A1, b, lane, y);
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    double y1 = y[k], y2 = A1 * y1 + B1[k];
+#pragma unroll
+    for (int j = 0; j < H; ++j) {
+      if (j < cnt) {
+        y1 = (t0 + j == 0) ? v[k][j] : v[k][j] - y1 * lo[j];
+        v[k][j] = y1;
+      }
+      const int q = H + j;
+      if (q < cnt) {
+        y2 = v[k][q] - y2 * lo[q];
+        v[k][q] = y2;
+      }
     }
   }
 }
@@ -129,55 +132,80 @@ __device__ __forceinline__ void fdma_forward(double (&v)[SLICE], const double (&
 // length len (g1, g2 zero where t + 1, t + 2 leave the chain).  rd holds 1 / dia: the
 // division becomes a product with the tabulated reciprocal (one rounding apart).
 using wave::Map2;  // s' = M s + w on the state s = (x_{t+1}, x_{t+2})
-__device__ __forceinline__ void map2_step(Map2& a, double v, double r, double g1, double g2) {
+template <int SLICE, int NR>
+__device__ __forceinline__ void fdma_backward(double (&v)[NR][SLICE], const double (&rd)[SLICE], const double (&g1)[SLICE],
+                                              const double (&g2)[SLICE], int lane, int t0, int cnt, int len) {
 #pragma clang fp contract(off)
-  const double c0 = v * r, c1 = -(g1 * r), c2 = -(g2 * r);
-  const double n00 = c1 * a.m00 + c2 * a.m10, n01 = c1 * a.m01 + c2 * a.m11, nw0 = c1 * a.w0 + c2 * a.w1 + c0;
-  a.m10 = a.m00;
-  a.m11 = a.m01;
-  a.w1 = a.w0;
-  a.m00 = n00;
-  a.m01 = n01;
-  a.w0 = nw0;
+  constexpr int H = SLICE / 2;
+  Map2 h[2];  // lower and upper half, top-down: the upper first; their offsets per right-hand side
+  double w[2][NR][2] = {};
+  auto step = [&](int s, int q) {
+    Map2& a = h[s];
+    const double r = rd[q], c1 = -(g1[q] * r), c2 = -(g2[q] * r);
+    const double n00 = c1 * a.m00 + c2 * a.m10, n01 = c1 * a.m01 + c2 * a.m11;
+    a.m10 = a.m00;
+    a.m11 = a.m01;
+    a.m00 = n00;
+    a.m01 = n01;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const double n = c1 * w[s][k][0] + c2 * w[s][k][1] + v[k][q] * r;
+      w[s][k][1] = w[s][k][0];
+      w[s][k][0] = n;
+    }
+  };
+#pragma unroll
+  for (int j = H - 1; j >= 0; --j) {
+    if (j < cnt) step(0, j);
+    if (H + j < cnt) step(1, H + j);
+  }
+  const Map2 &L = h[0], &U = h[1];
+  double b[NR][2], u[NR][2];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    b[k][0] = __builtin_fma(L.m00, w[1][k][0], __builtin_fma(L.m01, w[1][k][1], w[0][k][0]));
+    b[k][1] = __builtin_fma(L.m10, w[1][k][0], __builtin_fma(L.m11, w[1][k][1], w[0][k][1]));
+  }
+  wave::scan_states2(wave::compose(L, U), b, lane, u);
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    double u0 = u[k][0], u1 = u[k][1];
+    double l0 = U.m00 * u0 + U.m01 * u1 + w[1][k][0], l1 = U.m10 * u0 + U.m11 * u1 + w[1][k][1];
+#pragma unroll
+    for (int j = H - 1; j >= 0; --j) {
+      if (j < cnt) {
+        const int t = t0 + j;
+        double val = v[k][j];
+        if (t + 1 < len) val = val - l0 * g1[j];
+        if (t + 2 < len) val = val - l1 * g2[j];
+        val = val * rd[j];
+        l1 = l0;
+        l0 = val;
+        v[k][j] = val;
+      }
+      const int q = H + j;
+      if (q < cnt) {
+        const int t = t0 + q;
+        double val = v[k][q];
+        if (t + 1 < len) val = val - u0 * g1[q];
+        if (t + 2 < len) val = val - u1 * g2[q];
+        val = val * rd[q];
+        u1 = u0;
+        u0 = val;
+        v[k][q] = val;
+      }
+    }
+  }
+}
+// one right-hand side
+template <int SLICE>
+__device__ __forceinline__ void fdma_forward(double (&v)[SLICE], const double (&lo)[SLICE], int lane, int t0, int cnt) {
+  fdma_forward(reinterpret_cast<double(&)[1][SLICE]>(v), lo, lane, t0, cnt);
 }
 template <int SLICE>
 __device__ __forceinline__ void fdma_backward(double (&v)[SLICE], const double (&rd)[SLICE], const double (&g1)[SLICE],
                                               const double (&g2)[SLICE], int lane, int t0, int cnt, int len) {
-#pragma clang fp contract(off)
-  constexpr int H = SLICE / 2;
-  Map2 L, U;  // top-down: U first, then L
-#pragma unroll
-  for (int j = H - 1; j >= 0; --j) {
-    if (j < cnt) map2_step(L, v[j], rd[j], g1[j], g2[j]);
-    if (H + j < cnt) map2_step(U, v[H + j], rd[H + j], g1[H + j], g2[H + j]);
-  }
-  double u0, u1;
-  wave::scan_states2(wave::compose(L, U), lane, u0, u1);
-  double l0 = U.m00 * u0 + U.m01 * u1 + U.w0, l1 = U.m10 * u0 + U.m11 * u1 + U.w1;
-#pragma unroll
-  for (int j = H - 1; j >= 0; --j) {
-    if (j < cnt) {
-      const int t = t0 + j;
-      double val = v[j];
-      if (t + 1 < len) val = val - l0 * g1[j];
-      if (t + 2 < len) val = val - l1 * g2[j];
-      val = val * rd[j];
-      l1 = l0;
-      l0 = val;
-      v[j] = val;
-    }
-    const int q = H + j;
-    if (q < cnt) {
-      const int t = t0 + q;
-      double val = v[q];
-      if (t + 1 < len) val = val - u0 * g1[q];
-      if (t + 2 < len) val = val - u1 * g2[q];
-      val = val * rd[q];
-      u1 = u0;
-      u0 = val;
-      v[q] = val;
-    }
-  }
+  fdma_backward(reinterpret_cast<double(&)[1][SLICE]>(v), rd, g1, g2, lane, t0, cnt, len);
 }
 
 // tdma normal equations (linalg.rs:14-57), forward: g_i = (d_i - g_{i-2} off_{i-2}) / den_i,

@@ -72,6 +72,89 @@ __global__ __launch_bounds__(WAVE* WAVES, SLICE <= 8 ? 4 : 2) void fdma_rows_com
   rowsolve::fdma_block<SLICE, true>(lds, R, ldr, nr, X, ld, 2 * nsets, m, nsets, per, bl, bandp, diagp, blockIdx.x);
 }
 
+// The rows of NR batch entries (from NR blockIdx.y on) with the same tables by one wavefront per (set,
+// parity chain): the tables are read and the maps' matrices composed and scanned once for the NR right-hand
+// sides.  One row per set and entry (nrows = nsets); a block holds two sets.  512 x 512, 64 right-hand sides:
+// 89 us against 122 us with a wavefront per row; its 267 MB would take 54 us, the rest is the scans.
+template <int SLICE, int NR>
+__global__ __launch_bounds__(WAVE* WAVES, 2) void fdma_rows_batch_kernel(const double* __restrict__ R, int ldr, int nr,
+                                                                         double* __restrict__ X, int ld, int m,
+                                                                         int nsets, int per, int bl,
+                                                                         const double* __restrict__ bandp,
+                                                                         const double* __restrict__ diagp, int batch,
+                                                                         long sr, long sx) {
+#pragma clang fp contract(off)
+  extern __shared__ double lds[];
+  const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
+  const int slot = w >> 1, p = w & 1, tid = p * WAVE + lane;
+  double* buf = lds + slot * NR * bl;
+  const int set = blockIdx.x * (WAVES / 2) + slot, b0 = blockIdx.y * NR, s0 = min(set, nsets - 1);
+  constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
+  auto valid = [&](int k) { return set < nsets && b0 + k < batch; };
+#pragma unroll
+  for (int k = 0; k < NR; ++k)
+    chains::stage_row<MAXQ>(buf + k * bl, R + sr * (b0 + k) + (size_t)set * ldr, valid(k), nr, tid, 2 * WAVE);
+  __syncthreads();
+  const int len = p == 0 ? (m + 1) / 2 : m / 2, t0 = lane * per, cnt = max(0, min(per, len - t0));
+  double v[NR][SLICE];
+  if (bandp) {  // taps at offsets 0, -2, +2, +4, summed in that order
+    const size_t tp = (size_t)2 * per * WAVE;
+    double c[4][SLICE];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int q = 0; q < SLICE; ++q) c[t][q] = bandp[t * tp + ((size_t)p * per + q) * WAVE + lane];
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+#pragma unroll
+      for (int q = 0; q < SLICE; ++q) {
+        double val = 0.0;
+        if (q < cnt) {
+          const int j = p + 2 * (t0 + q) + 2;
+          const double* row = buf + k * bl;
+          val = c[0][q] * row[pad(j)];
+          val = val + c[1][q] * row[pad(j - 2)];
+          val = val + c[2][q] * row[pad(j + 2)];
+          val = val + c[3][q] * row[pad(j + 4)];
+        }
+        v[k][q] = val;
+      }
+  } else {
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+#pragma unroll
+      for (int q = 0; q < SLICE; ++q) v[k][q] = q < cnt ? buf[k * bl + pad(p + 2 * (t0 + q) + 2)] : 0.0;
+  }
+  const double* dg = diagp + (size_t)s0 * (8 * (size_t)per * WAVE);
+  auto table = [&](int a, int q) { return dg[((size_t)(a * 2 + p) * per + q) * WAVE + lane]; };
+  {
+    double lo[SLICE];
+#pragma unroll
+    for (int q = 0; q < SLICE; ++q) lo[q] = table(0, q);
+    chains::fdma_forward(v, lo, lane, t0, cnt);
+  }
+  {
+    double rd[SLICE], g1[SLICE], g2[SLICE];  // 1 / dia, up1, up2
+#pragma unroll
+    for (int q = 0; q < SLICE; ++q) {
+      rd[q] = table(1, q);
+      g1[q] = table(2, q);
+      g2[q] = table(3, q);
+    }
+    chains::fdma_backward(v, rd, g1, g2, lane, t0, cnt, len);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NR; ++k)
+#pragma unroll
+    for (int q = 0; q < SLICE; ++q)
+      if (q < cnt) buf[k * bl + pad(p + 2 * (t0 + q) + 2)] = v[k][q];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NR; ++k)
+    chains::unstage_row<MAXQ>(buf + k * bl, X + sx * (b0 + k) + (size_t)set * ld, valid(k), m, tid, 2 * WAVE, false);
+}
+
 // from_ortho of a composite basis per row (composite_stencil.rs:250-276, linalg.rs:14-57):
 // d_i = p_i diag_i + p_{i+2} low2_i, then g_i = (d_i - g_{i-2} off_{i-2}) / den_i and
 // x_i = g_i - x_{i+2} w_i (x_i = g_i for the last two i), arithmetic as tdma_y.  One
@@ -172,6 +255,24 @@ static void launch_rows(hipStream_t s, const double* R, int ldr, int nr, double*
   const int pairg = paired ? (nsets + 7) / 8 : 0;
   const dim3 grid = paired ? dim3((unsigned)(16 * pairg + (batch - 2) * nsets), 1) : dim3(blocks, batch),
              block(WAVE * WAVES);
+  // four right-hand sides per wavefront from two blocks per CU on (a whole solve, a row / four rows per
+  // wavefront: 510 rows x 8 (510 blocks) 90.0 / 86.6 us, 126 x 64 (1,008) 48.8 / 43.9, 510 x 4 (255) 56.6 /
+  // 57.2, 94 x 8 (94) 23.5 / 25.9)
+  constexpr int NR = 4;
+  if (tb.shared && nrows == nsets && batch >= NR && sl <= 8 && (size_t)NR * lds <= 65536 &&
+      (long)blocks * (batch / NR) >= 500) {
+    const dim3 g2(blocks, (batch + NR - 1) / NR);
+    const size_t l2 = NR * lds;
+#define RBC_BATCH(SL)                                                                                                \
+  RBC_LAUNCH((fdma_rows_batch_kernel<SL, NR>), g2, block, l2, s, R, ldr, nr, X, ld, m, nsets, per, bl, tb.band[0], \
+             tb.diag[0], batch, sr, sx)
+    if (sl <= 2) RBC_BATCH(2);
+    else if (sl <= 4) RBC_BATCH(4);
+    else RBC_BATCH(8);
+#undef RBC_BATCH
+    check("fdma_rows_batch");
+    return;
+  }
   if (sl <= 2)
     RBC_LAUNCH(fdma_rows_lds_kernel<2>, grid, block, lds, s, R, ldr, nr, X, ld, nrows, m, nsets, per, bl, tb,
                        sr, sx, pairg);
@@ -193,6 +294,12 @@ void fdma_rows_lds(hipStream_t s, const double* R, int ldr, int nr, double* X, i
   tb.band[0] = bandp;
   tb.diag[0] = diagp;
   tb.shared = 1;
+  if (batch == 1 && nrows >= 4L * nsets && nrows % nsets == 0 && nrows / nsets <= 65535) {  // entries of one row per set
+    batch = nrows / nsets;
+    nrows = nsets;
+    sr = (long)nsets * ldr;
+    sx = (long)nsets * ld;
+  }
   launch_rows(s, R, ldr, nr, X, ld, nrows, m, nsets, tb, batch, sr, sx);
 }
 

@@ -110,32 +110,59 @@ __device__ __forceinline__ Map2 compose(const Map2& a, const Map2& b) {
   c.w1 = __builtin_fma(a.m10, b.w0, __builtin_fma(a.m11, b.w1, a.w1));
   return c;
 }
-template <int CTRL>
-__device__ __forceinline__ Map2 dpp_map(const Map2& x) {
-  return Map2{dpp_or<CTRL>(x.m00, 1.0), dpp_or<CTRL>(x.m01, 0.0), dpp_or<CTRL>(x.m10, 0.0),
-              dpp_or<CTRL>(x.m11, 1.0), dpp_or<CTRL>(x.w0, 0.0),  dpp_or<CTRL>(x.w1, 0.0)};
+// The scan for NB right-hand sides with the same matrices (a's own w is not used): w_j the lane's offsets,
+// u_j its entry states
+template <int CTRL, int NB>
+__device__ __forceinline__ void scan_step2(Map2& a, double (&w)[NB][2]) {
+  Map2 q = a;
+  q.m00 = dpp_or<CTRL>(a.m00, 1.0);
+  q.m01 = dpp_or<CTRL>(a.m01, 0.0);
+  q.m10 = dpp_or<CTRL>(a.m10, 0.0);
+  q.m11 = dpp_or<CTRL>(a.m11, 1.0);
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const double q0 = dpp_or<CTRL>(w[j][0], 0.0), q1 = dpp_or<CTRL>(w[j][1], 0.0);
+    w[j][0] = __builtin_fma(a.m00, q0, __builtin_fma(a.m01, q1, w[j][0]));
+    w[j][1] = __builtin_fma(a.m10, q0, __builtin_fma(a.m11, q1, w[j][1]));
+  }
+  const Map2 c = compose(a, q);
+  a.m00 = c.m00;
+  a.m01 = c.m01;
+  a.m10 = c.m10;
+  a.m11 = c.m11;
+}
+template <int NB>
+__device__ __forceinline__ void scan_states2(Map2 a, double (&w)[NB][2], int lane, double (&u)[NB][2]) {
+  scan_step2<ROW_SHL + 1>(a, w);
+  scan_step2<ROW_SHL + 2>(a, w);
+  scan_step2<ROW_SHL + 4>(a, w);
+  scan_step2<ROW_SHL + 8>(a, w);
+  const int row = 3 - (lane >> 4);
+  const double x00 = dpp_or<ROW_SHL + 1>(a.m00, 1.0), x01 = dpp_or<ROW_SHL + 1>(a.m01, 0.0);
+  const double x10 = dpp_or<ROW_SHL + 1>(a.m10, 0.0), x11 = dpp_or<ROW_SHL + 1>(a.m11, 1.0);
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    double s0[4], s1[4];  // entry states of rows 3, 2, 1, 0
+    s0[0] = s1[0] = 0.0;
+    s0[1] = lane_value(w[j][0], 48);
+    s1[1] = lane_value(w[j][1], 48);
+#pragma unroll
+    for (int r = 2; r < 4; ++r) {
+      const int l = 64 - 16 * r;
+      s0[r] = __builtin_fma(lane_value(a.m00, l), s0[r - 1], __builtin_fma(lane_value(a.m01, l), s1[r - 1], lane_value(w[j][0], l)));
+      s1[r] = __builtin_fma(lane_value(a.m10, l), s0[r - 1], __builtin_fma(lane_value(a.m11, l), s1[r - 1], lane_value(w[j][1], l)));
+    }
+    const double e0 = row == 0 ? 0.0 : row == 1 ? s0[1] : row == 2 ? s0[2] : s0[3];
+    const double e1 = row == 0 ? 0.0 : row == 1 ? s1[1] : row == 2 ? s1[2] : s1[3];
+    u[j][0] = __builtin_fma(x00, e0, __builtin_fma(x01, e1, dpp_or<ROW_SHL + 1>(w[j][0], 0.0)));
+    u[j][1] = __builtin_fma(x10, e0, __builtin_fma(x11, e1, dpp_or<ROW_SHL + 1>(w[j][1], 0.0)));
+  }
 }
 __device__ __forceinline__ void scan_states2(Map2 a, int lane, double& u0, double& u1) {
-  a = compose(a, dpp_map<ROW_SHL + 1>(a));
-  a = compose(a, dpp_map<ROW_SHL + 2>(a));
-  a = compose(a, dpp_map<ROW_SHL + 4>(a));
-  a = compose(a, dpp_map<ROW_SHL + 8>(a));
-  double s0[4], s1[4];  // entry states of rows 3, 2, 1, 0
-  s0[0] = s1[0] = 0.0;
-  s0[1] = lane_value(a.w0, 48);
-  s1[1] = lane_value(a.w1, 48);
-#pragma unroll
-  for (int r = 2; r < 4; ++r) {
-    const int l = 64 - 16 * r;
-    s0[r] = __builtin_fma(lane_value(a.m00, l), s0[r - 1], __builtin_fma(lane_value(a.m01, l), s1[r - 1], lane_value(a.w0, l)));
-    s1[r] = __builtin_fma(lane_value(a.m10, l), s0[r - 1], __builtin_fma(lane_value(a.m11, l), s1[r - 1], lane_value(a.w1, l)));
-  }
-  const int row = 3 - (lane >> 4);
-  const double e0 = row == 0 ? 0.0 : row == 1 ? s0[1] : row == 2 ? s0[2] : s0[3];
-  const double e1 = row == 0 ? 0.0 : row == 1 ? s1[1] : row == 2 ? s1[2] : s1[3];
-  const Map2 x = dpp_map<ROW_SHL + 1>(a);
-  u0 = __builtin_fma(x.m00, e0, __builtin_fma(x.m01, e1, x.w0));
-  u1 = __builtin_fma(x.m10, e0, __builtin_fma(x.m11, e1, x.w1));
+  double w[1][2] = {{a.w0, a.w1}}, u[1][2];
+  scan_states2(a, w, lane, u);
+  u0 = u[0][0];
+  u1 = u[0][1];
 }
 
 }  // namespace wave
