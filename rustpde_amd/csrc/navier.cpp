@@ -2999,9 +2999,13 @@ class SolverDev {
     if (cplx) y = w.out;
     Solver& sv = *s;
     if (sv.kind == ADI) {
-      const XGemm g = xgemm_of(sv.hxp, x, w.w1, o1, batch, (long)in_sz, (long)sv.hx.rows * o1);
-      xgemm(st, &g, 1);
-      gemm_mfma(st, batch * sv.hx.rows, m1, sv.hy.rows, w.w1, sv.hy.rows, sv.hy.b.p, sv.hy.cols, y, m1, 1.0, 0.0);
+      const long mid = (long)sv.hxp.op.rows * o1;  // [o1, m0]: results transposed, so both are x products
+      XGemm g = xgemm_of(sv.hxp, x, w.w1, o1, batch, (long)in_sz, mid);
+      g.ldc = sv.hxp.op.rows;
+      xgemm_t(st, &g, 1);
+      g = xgemm_of(sv.hyp, w.w1, y, sv.hxp.op.rows, batch, mid, (long)out_sz);
+      g.ldc = m1;
+      xgemm_t(st, &g, 1);
     } else if (!sv.has_fb) {
       rows_launch(x, o1, y, m1, batch * ro, sv);
     } else {
