@@ -1951,11 +1951,14 @@ class Navier {
   }
   // The convective terms by products with the dense x operators, the y stage as in the confined step,
   // where there are no fast transforms (160 x 129, 50 steps and their output: 12.3 ms field by field in
-  // some 45 launches a step, 2.2 ms in seven) and on small grids, whose transforms are bound by their
-  // launches and passes: us per step by transforms / products on MI355X, 64 x 65 50.5 / 32.7, 128 x 129
-  // 51.9 / 37.5, 256 x 129 55.7 / 44.7, 256 x 257 57.3 / 58.5, 512 x 257 72 / 90, 512 x 513 89 / 132.
+  // some 45 launches a step, 1.9 ms in seven) and on small grids, whose transforms are bound by their
+  // launches and passes: us per step by transforms / products on MI355X, 64 x 65 50.5 / 32.7 (before the
+  // row kernels' lane scans), 512 x 129 60.1 / 52.6, 128 x 257 46.0 / 42.0, 256 x 257
+  // 51.5 / 51.6, 512 x 257 65 / 78, 256 x 513 68 / 75.
   bool dense_sizes() const {
-    return periodic && (!fft_supported(nx) || (nx <= 256 && (ny <= 200 || !cheb_y_supported(ny))));
+    if (!periodic) return false;
+    if (!fft_supported(nx) || (!cheb_y_supported(ny) && nx <= 256)) return true;
+    return ny <= 200 ? nx <= 512 : nx <= 128 && ny <= 257;
   }
   // the mixed step keeps its FP32 transforms where they exist
   bool dense_step() const { return dense_sizes() && !(mixed && fft_supported(nx) && cheb_y_supported(ny)); }
