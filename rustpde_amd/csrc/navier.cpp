@@ -2028,11 +2028,40 @@ class Navier {
     // d/dy pres, then the right-hand sides (navier.rs:622-674) with to_ortho of ux, uy, temp,
     // the buoyancy temp + fieldbc (navier.rs:740-742) and d/dx pres formed in the same kernel
     if (!gpres_valid || !pressure_fused_ok()) yop(by_p, "DS", P0.p, rows_ortho(bx_p), G.p + F);
+    const int cutx = bx_f.m * 2 / 3, cuty = ny * 2 / 3;
+    if (rows_form_rhs()) {  // the right-hand sides in the solves' own launches
+      StepRhs r;
+      r.U = UX.p;
+      r.stencil = stencil_band(by_u).coef.p;
+      r.P0 = P0.p;
+      r.g1 = G.p + F;
+      r.thbc = THAT_BC.p;
+      r.gxx = GXX.p;
+      r.gyy = GYY.p;
+      r.cv = mixed ? (const void*)MIX.p : CV.p;
+      r.cv32 = mixed ? 1 : 0;
+      r.my = my;
+      r.mx = mx();
+      r.ny = ny;
+      r.bcr = bc_rows;
+      r.cutx = cutx;
+      r.cuty = cuty;
+      r.F = (long)F;
+      r.kscale = scale[0];
+      int ex = 0;
+      r.isc = scale[0] > 0.0 && std::frexp(scale[0], &ex) == 0.5 ? 1.0 / scale[0] : 0.0;
+      r.dt = dt;
+      const Solver& sv = *solver[0];
+      timer.begin(st, 1, 8.0 * 2.0 * mx() * (2.0 * my + 2.0 * (my + ny) + 4.0 * my) + (mixed ? 4.0 : 8.0) * 4.0 * cutx * cuty);
+      step_rows(st, r, UX.p, sv.pybp.p, sv.diagp.p);
+      timer.end(st);
+      solves_and_pressure(&r);
+      return;
+    }
     // bytes: ux, uy, temp coefficients, pres, d/dy pres read, three right-hand sides
     // written; fieldbc, gxx, gyy in their bc_rows nonzero rows; the three convective terms
     // inside the dealiasing cuts (bx_f.m 2/3 wavenumbers, ny 2/3 y-modes: zero beyond)
     const double bcb = 8.0 * 3.0 * bc_rows * ny;
-    const int cutx = bx_f.m * 2 / 3, cuty = ny * 2 / 3;
     const double cvn = 3.0 * 2.0 * cutx * cuty;
     if (mixed) {  // FP32 convective terms (conv_mixed)
       timer.begin(st, 3, 8.0 * 2.0 * mx() * (3.0 * my + 5.0 * ny) + 4.0 * cvn + bcb);
@@ -2220,7 +2249,13 @@ class Navier {
     pa.sp_kind = by_phi.k == CD ? 1 : by_phi.k == CN ? 2 : 0;
     return pa;
   }
-  void solves_and_pressure() {
+  // the periodic step's right-hand sides are formed by its row solves
+  bool rows_form_rhs() {
+    return step_rows_supported(ny) && pressure_fused_ok() && vel_same && solver[0]->nsets == mx() && solver[2]->nsets == mx() && !solver[2]->has_fb &&
+           !solver[0]->has_fb && by_u.n == ny && by_u.m == ny - 2;
+  }
+  // rhs: ux and uy are solved already, temp's right-hand side comes from it
+  void solves_and_pressure(const StepRhs* rhs = nullptr) {
     const int my = by_u.m, R2 = 2 * mx();
     const size_t F = FS;
     // implicit solves of ux, uy (one solver for both) and temp in one launch; with the fused
@@ -2233,10 +2268,12 @@ class Navier {
     const double* diags[3] = {sv.diagp.p, sv.diagp.p, stt.diagp.p};
     // bytes: right-hand sides read and results written per row, the diagonal sets once per solver
     const double temp_bytes = 8.0 * ((double)R2 * (ny + my) + 4.0 * (double)stt.nsets * my);
-    timer.begin(st, 1, 8.0 * (2.0 * (double)R2 * (ny + my) + 4.0 * (double)sv.nsets * my) +
-                           (fold_temp ? 0.0 : temp_bytes));
-    fdma_rows_lds_multi(st, RHS.p, ny, ny, UX.p, my, R2, my, sv.nsets, bands, diags, nsolve, (long)F, (long)F);
-    timer.end(st);
+    if (!rhs) {
+      timer.begin(st, 1, 8.0 * (2.0 * (double)R2 * (ny + my) + 4.0 * (double)sv.nsets * my) +
+                             (fold_temp ? 0.0 : temp_bytes));
+      fdma_rows_lds_multi(st, RHS.p, ny, ny, UX.p, my, R2, my, sv.nsets, bands, diags, nsolve, (long)F, (long)F);
+      timer.end(st);
+    }
     // projection (navier.rs:683-721)
     if (pressure_fused_ok()) {
       PressureArgs pa = pressure_args(nu);
@@ -2251,6 +2288,7 @@ class Navier {
         pa.rows_ld = my;
         pa.rows_m = my;
         pa.rows_nsets = stt.nsets;
+        if (rhs) pa.rows_rhs = *rhs;
       }
       const double rows = 2.0 * mx();
       // bytes, distinct arrays once per row: ux, uy, pres read; ux, uy, pseu, pres and d/dy

@@ -352,6 +352,23 @@ void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure);
 // [2 mx, mu]; su / sp are the stencil taps [2][ny] of the velocity / pseudo-pressure y
 // bases; pybp / pdiag the Poisson solver's P_y taps and diagonal sets and ttab the tdma
 // tables of the velocity y basis, all in slice order.  per and bl are set by the call.
+// Right-hand sides of the periodic step formed by the row solves themselves: rhs3_fused's values with its
+// arguments (U: ux, uy, temp, F apart; stencil [2][ny]; cv FP32 when cv32).
+struct StepRhs {
+  const double *U = nullptr, *stencil, *P0, *g1, *thbc, *gxx, *gyy;
+  const void* cv;
+  int cv32, my, mx, ny, bcr, cutx, cuty;
+  long F;
+  double kscale, isc, dt;  // isc = 1 / kscale when kscale is a power of two, else 0
+};
+// ux and uy (fields 0 and 1) solved in place, both with the tables bandp, diagp (mx sets)
+// rows of up to four entries a lane (514 points): a step with / without, 64 x 65 25.0 / 27.3 us, 512 x 257
+// 62.8 / 65.1, 1024 x 513 109 / 116; with eight entries the values in flight cost the kernels their
+// occupancy (1024 x 1025 mixed: 82.6 us in two launches against 72.3 in three)
+constexpr int STEP_SLICE = 4;
+bool step_rows_supported(int ny);
+void step_rows(hipStream_t s, const StepRhs& a, double* X, const double* bandp, const double* diagp);
+
 struct PressureArgs {
   double *UX, *UY, *P0, *P1;
   const double *su, *sp, *pybp, *pdiag, *ttab;
@@ -373,6 +390,7 @@ struct PressureArgs {
   const double *rows_band = nullptr, *rows_diag = nullptr;
   int rows_ldr = 0, rows_nr = 0, rows_ld = 0, rows_m = 0, rows_nsets = 0;
   int rows_per = 0, rows_bl = 0;  // set by pressure_rows
+  StepRhs rows_rhs;  // with U set: the further rows are temp's, their right-hand sides formed from it (rows_R unused)
 };
 bool pressure_rows_supported(int ny, int mu);
 void pressure_rows(hipStream_t s, const PressureArgs& a);

@@ -68,6 +68,13 @@ __global__ __launch_bounds__(256, 3) void pressure_rows_kernel(PressureArgs a) {
   const int su_kind = RBC ? 1 : a.su_kind, sp_kind = RBC ? 2 : a.sp_kind;
   extern __shared__ double lds[];
   if ((int)blockIdx.x >= a.mx) {  // the whole block
+    if constexpr (SLICE <= STEP_SLICE) {
+      if (a.rows_rhs.U) {
+        rowsolve::step_block<SLICE>(lds, a.rows_rhs, 2, a.rows_X, a.rows_per, a.rows_bl, a.rows_band, a.rows_diag,
+                                    (int)blockIdx.x - a.mx);
+        return;
+      }
+    }
     rowsolve::fdma_block<SLICE>(lds, a.rows_R, a.rows_ldr, a.rows_nr, a.rows_X, a.rows_ld, 2 * a.rows_nsets,
                                 a.rows_m, a.rows_nsets, a.rows_per, a.rows_bl, a.rows_band,
                                 a.rows_diag, (int)blockIdx.x - a.mx);
@@ -437,7 +444,10 @@ void pressure_rows(hipStream_t s, const PressureArgs& args) {
     a.rows_per = fdma_rows_lds_per(a.rows_m);
     a.rows_bl = buf_len(a.rows_nr);
     if (!fdma_rows_lds_supported(a.rows_m, a.rows_nr) || a.rows_per > slice || fdma_rows_lds_per(a.rows_nr - 2) > slice ||
-        (size_t)(rowsolve::WAVES / 2) * a.rows_bl * sizeof(double) > lds || !a.rows_R || !a.rows_X || !a.rows_diag)
+        (size_t)(rowsolve::WAVES / 2) * a.rows_bl * sizeof(double) > lds ||
+        (!a.rows_R && !a.rows_rhs.U) || !a.rows_X || !a.rows_diag ||
+        (a.rows_rhs.U && (slice > STEP_SLICE || a.rows_m != a.rows_rhs.my || a.rows_nr != a.rows_rhs.ny || a.rows_nsets != a.rows_rhs.mx ||
+                          a.rows_ld != a.rows_m)))
       throw std::invalid_argument("pressure_rows: unsupported further rows");
   } else {
     a.rows_nsets = 0;

@@ -58,6 +58,19 @@ __global__ __launch_bounds__(WAVE* WAVES, SLICE <= 8 ? 4 : 2) void fdma_rows_lds
                               tb.diag[ti], bx);
 }
 
+// ux and uy of the periodic step, a set's rows of both fields 8 blocks apart (as above), with the right-hand
+// sides formed in place of a launch that writes and a pass that reads them: 256 x 257, 6.8 us where these
+// took 4.0 and 4.9
+template <int SLICE>
+__global__ __launch_bounds__(WAVE* WAVES, 4) void step_rows_kernel(StepRhs a, double* X, int per, int bl,
+                                                                   const double* __restrict__ bandp,
+                                                                   const double* __restrict__ diagp) {
+  extern __shared__ double lds[];
+  const int bx = blockIdx.x, f = (bx >> 3) & 1, set = (bx >> 4) * 8 + (bx & 7);
+  if (set >= a.mx) return;  // the whole block: no barrier reached
+  rowsolve::step_block<SLICE>(lds, a, f, X + f * a.F, per, bl, bandp, diagp, set);
+}
+
 // The rows of blockIdx.y-th interleaved complex array [nsets, nr] -> [nsets, m], one block per
 // set.  The caller's arrays are read and written once: at fourier_r2c(256) x cheb_neumann(257),
 // 4 right-hand sides, 19 us a call with the wait for it, against 59 us with a split and a merge
@@ -314,6 +327,20 @@ void fdma_rows_lds_multi(hipStream_t s, const double* R, int ldr, int nr, double
   }
   tb.shared = 0;
   launch_rows(s, R, ldr, nr, X, ld, nrows, m, nsets, tb, batch, sr, sx);
+}
+
+bool step_rows_supported(int ny) {
+  return ny >= 9 && fdma_rows_lds_supported(ny - 2, ny) && fdma_rows_lds_per(ny - 2) <= STEP_SLICE;
+}
+void step_rows(hipStream_t s, const StepRhs& a, double* X, const double* bandp, const double* diagp) {
+  if (!step_rows_supported(a.ny) || a.my != a.ny - 2 || a.mx < 1 || !a.U || !bandp || !diagp)
+    throw std::invalid_argument("step_rows: unsupported sizes");
+  const int per = fdma_rows_lds_per(a.my), bl = buf_len(a.ny), sl = slice_of(a.my, a.ny);
+  const dim3 grid(16 * ((a.mx + 7) / 8)), block(WAVE * WAVES);
+  const size_t lds = (size_t)(WAVES / 2) * bl * sizeof(double);
+  if (sl <= 2) RBC_LAUNCH(step_rows_kernel<2>, grid, block, lds, s, a, X, per, bl, bandp, diagp);
+  else RBC_LAUNCH(step_rows_kernel<4>, grid, block, lds, s, a, X, per, bl, bandp, diagp);
+  check("step_rows");
 }
 
 void fdma_rows_lds_complex(hipStream_t s, const double* R, int ldr, int nr, double* X, int ld, int m, int nsets,

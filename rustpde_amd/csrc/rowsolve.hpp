@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include "chains.hpp"
+#include "ops.hpp"
 
 namespace rbc {
 namespace rowsolve {
@@ -30,9 +31,9 @@ constexpr int WAVES = 4;  // wavefronts per block: two row slots of two parity c
 // bx, else the rows 2 bx and 2 bx + 1.  Every thread of the block must call it.
 // CPLX: the block holds the real and the imaginary part of complex row bx of set bx, rows ldr
 // and ld interleaved values apart.
-template <int SLICE, bool CPLX = false>
-__device__ __forceinline__ void fdma_block(double* lds, const double* __restrict__ R, int ldr, int nr,
-                                           double* __restrict__ X, int ld, int nrows, int m, int nsets, int per,
+// stage(buf, r, valid, slot, tid): row r's right-hand side into buf by threads tid < 2 WAVE, as stage_row.
+template <int SLICE, bool CPLX = false, class Stage>
+__device__ __forceinline__ void fdma_block(double* lds, Stage stage, int nr, double* __restrict__ X, int ld, int nrows, int m, int nsets, int per,
                                            int bl, const double* __restrict__ bandp,
                                            const double* __restrict__ diagp, int bx) {
 #pragma clang fp contract(off)
@@ -53,10 +54,7 @@ __device__ __forceinline__ void fdma_block(double* lds, const double* __restrict
   }
   // (1) row -> LDS: element i at pad(i + 2); i in [-2, 0) and [nr, nr + 4) read as zero
   constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
-  if constexpr (CPLX)
-    chains::stage_row<MAXQ, 2>(buf, R + 2 * (size_t)bx * ldr + slot, valid, nr, p * WAVE + lane, 2 * WAVE);
-  else
-    chains::stage_row<MAXQ>(buf, R + (size_t)r * ldr, valid, nr, p * WAVE + lane, 2 * WAVE);
+  stage(buf, r, valid, slot, p * WAVE + lane);
   __syncthreads();
   const int len = p == 0 ? (m + 1) / 2 : m / 2;
   const int t0 = lane * per;
@@ -117,6 +115,92 @@ __device__ __forceinline__ void fdma_block(double* lds, const double* __restrict
     chains::unstage_row<MAXQ, 2>(buf, X + 2 * (size_t)bx * ld + slot, valid, m, p * WAVE + lane, 2 * WAVE, false);
   else
     chains::unstage_row<MAXQ>(buf, X + (size_t)r * ld, valid, m, p * WAVE + lane, 2 * WAVE, false);
+}
+
+// rows R (stride ldr) as right-hand sides
+template <int SLICE, bool CPLX = false>
+__device__ __forceinline__ void fdma_block(double* lds, const double* __restrict__ R, int ldr, int nr,
+                                           double* __restrict__ X, int ld, int nrows, int m, int nsets, int per, int bl,
+                                           const double* __restrict__ bandp, const double* __restrict__ diagp, int bx) {
+  constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
+  fdma_block<SLICE, CPLX>(
+      lds,
+      [&](double* buf, int r, bool valid, int slot, int tid) {
+        if constexpr (CPLX) chains::stage_row<MAXQ, 2>(buf, R + 2 * (size_t)bx * ldr + slot, valid, nr, tid, 2 * WAVE);
+        else chains::stage_row<MAXQ>(buf, R + (size_t)r * ldr, valid, nr, tid, 2 * WAVE);
+      },
+      nr, X, ld, nrows, m, nsets, per, bl, bandp, diagp, bx);
+}
+
+// Row r of the right-hand side of field f into buf (rhs3_fused_kernel's values): the solves read the fields
+// instead of an array that a launch of its own wrote.
+template <int MAXQ, typename CV>
+__device__ __forceinline__ void stage_rhs(double* buf, const StepRhs& a, int f, int r, int tid) {
+#pragma clang fp contract(off)
+  const int n = a.ny, my = a.my;
+  const bool imag = r >= a.mx, bc = r < a.bcr;
+  const int k = imag ? r - a.mx : r;
+  const double kk = (double)k, dt = a.dt;
+  const double *u = a.U + f * a.F + (size_t)r * my, *t = a.U + 2 * a.F + (size_t)r * my;
+  const double *c0 = a.stencil, *c1 = a.stencil + n;
+  const double *pa = a.P0 + (size_t)k * n, *pb = a.P0 + (size_t)(a.mx + k) * n;
+  const long row = (long)r * n;
+  const CV* cv = static_cast<const CV*>(a.cv) + f * a.F + row;
+  auto taps = [&](const double* q, int i) {
+    const double x0 = i < my ? q[min(i, my - 1)] : 0.0, x2 = i >= 2 && i - 2 < my ? q[i - 2] : 0.0;
+    return x0 * c0[i] + x2 * c1[i];
+  };
+  auto conv = [&](int i) { return k >= a.cutx || i >= a.cuty ? 0.0 : (double)cv[i]; };
+  double v[MAXQ];
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int i = tid + q * 2 * WAVE - 2;
+    v[q] = 0.0;
+    if (i < 0 || i >= n) continue;
+    const double x = taps(u, i), c = conv(i);
+    if (f == 0) {
+      double na = pa[i] * 0.0 - pb[i] * kk, nb = pa[i] * kk + pb[i] * 0.0;
+      if (a.kscale != 1.0) {
+        if (a.isc != 0.0) {
+          na = na * a.isc;
+          nb = nb * a.isc;
+        } else {
+          const double ns = a.kscale * a.kscale + 0.0 * 0.0;
+          const double qa = (na * a.kscale + nb * 0.0) / ns, qb = (nb * a.kscale - na * 0.0) / ns;
+          na = qa;
+          nb = qb;
+        }
+      }
+      const double w = x - (imag ? nb : na) * dt;
+      v[q] = w - c * dt;
+    } else if (f == 1) {
+      double w = x - a.g1[row + i] * dt;
+      const double buoy = taps(t, i) + (bc ? a.thbc[row + i] : 0.0);
+      w = w + buoy * dt;
+      v[q] = w - c * dt;
+    } else {
+      const double gx2 = bc ? a.gxx[row + i] : 0.0, gy2 = bc ? a.gyy[row + i] : 0.0;
+      v[q] = ((x + gx2) + gy2) - c * dt;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int j = tid + q * 2 * WAVE;
+    if (j < n + 6) buf[pad(j)] = v[q];
+  }
+}
+// the rows of set bx of field f, solved in place
+template <int SLICE>
+__device__ __forceinline__ void step_block(double* lds, const StepRhs& a, int f, double* __restrict__ X, int per, int bl,
+                                           const double* __restrict__ bandp, const double* __restrict__ diagp, int bx) {
+  constexpr int MAXQ = (2 * SLICE * WAVE + 8 + 2 * WAVE - 1) / (2 * WAVE);
+  fdma_block<SLICE>(
+      lds,
+      [&](double* buf, int r, bool, int, int tid) {
+        if (a.cv32) stage_rhs<MAXQ, float>(buf, a, f, r, tid);
+        else stage_rhs<MAXQ, double>(buf, a, f, r, tid);
+      },
+      a.ny, X, a.my, 2 * a.mx, a.my, a.mx, per, bl, bandp, diagp, bx);
 }
 
 }  // namespace rowsolve
