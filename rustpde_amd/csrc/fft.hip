@@ -32,11 +32,14 @@ using fftlds::lp_size;
 using fftlds::xcd_remap;
 
 // geometry for length L and LDS value size VB: PP column pairs per block, E = PP L complex
-// values, T = E / 8.  Blocks of L >= 512 take 8 columns (row segments of 64 bytes in FP64,
-// 32 in FP32); shorter lengths take 2048 / L column pairs.
+// values, T = E / 8.  Blocks of L = 512 and 1024 take 8 columns (row segments of 64 bytes in FP64,
+// 32 in FP32), of L = 256 four, shorter lengths 2048 / L column pairs.  At 512 and 256 points few
+// columns are there (a step's three fields of 255 are 96 blocks of 16): with 16 columns a block, a step
+// of 512 x 257 takes 62.4 us against 59.4 with 8, of 256 x 257 48.6 against 46.9 with 4 (8: 47.5); 64
+// fields of 256 x 257 transform in 68 us either way.
 template <int L, int VB = 8>
 struct CGeo {
-  static constexpr int PP = L >= 2048 ? 1 : (L >= 512 ? 4096 : 2048) / L;
+  static constexpr int PP = L >= 2048 ? 1 : L == 256 ? 2 : (L >= 1024 ? 4096 : 2048) / L;
   static constexpr int E = PP * L;
   static constexpr int T = E / 8;
   static constexpr int C = 2 * PP;  // columns per block
