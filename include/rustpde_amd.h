@@ -188,9 +188,10 @@ int rbc_set_option(rbc_navier* h, int option, int value);
  * the external criterion bench benches/benchmark_navier.rs:23-40).  When enabled, HIP
  * events are recorded on the handle's stream around each launch of a kernel class;
  * rbc_timing_read returns the launches, their summed duration and summed algorithmic
- * work (flops for GEMMs, bytes for the memory-bound classes) since enabling.  Each class
- * but RBC_K_ELEMENTWISE is one kernel:
- *   RBC_K_GEMM gemm_mfma_kernel (dense transforms), RBC_K_ROWSOLVE fdma_rows_lds_kernel
+ * work (flops for products, bytes for the memory-bound classes) since enabling.  Each class
+ * but the first two and RBC_K_ELEMENTWISE is one kernel:
+ *   RBC_K_GEMM the FP64 products of the dense operators (xgemm_kernel, conv_kernel,
+ *   gemm_mfma_kernel), RBC_K_ROWSOLVE fdma_rows_lds_kernel and step_rows_kernel
  *   (Hholtz/Poisson rows), RBC_K_FFT irfft_cols_kernel, RBC_K_RFFT rfft_cols_kernel,
  *   RBC_K_DCT cheb_y_bwd_kernel, RBC_K_DCT_FWD cheb_y_fwd_kernel, RBC_K_DIFF_Y
  *   cheb_y_diff_kernel, RBC_K_TDMA tdma_rows_lds_kernel, RBC_K_BAND band_y_kernel;
@@ -198,7 +199,8 @@ int rbc_set_option(rbc_navier* h, int option, int value);
  *   cheb_y_conv_kernel (the convective term's y transforms and products, one launch);
  *   RBC_K_GEMM32 gemm_mfma_kernel in FP32 (the confined mixed step's convective terms);
  *   RBC_K_CONV3 cheb_y_conv3_kernel (the whole y-stage of the convective terms, one launch);
- *   RBC_K_ELEMENTWISE the remaining timed kernels (Fourier derivative, fallbacks). */
+ *   RBC_K_ELEMENTWISE the remaining timed kernels (row kernels of the confined step and
+ *   the adjoint, Fourier derivative, fallbacks). */
 #define RBC_K_GEMM 0
 #define RBC_K_ROWSOLVE 1
 #define RBC_K_FFT 2
