@@ -1411,7 +1411,7 @@ class Navier {
   // The dense operators as parity-class products along x or, on transposed arrays, along y
   // (xgemm.hip), and what lies between them as row kernels (confined.hip): 12 launches, 13 with the
   // y transforms by DCT, where stencils, derivatives, sums and products of their own took 29.  A
-  // step takes 47 us at 64^2 (105 before), 53 us at 128 x 129 (173), 101 us at 257^2 (205).
+  // step takes 38 us at 64^2 (105 before), 44 us at 128 x 129 (173), 91 us at 257^2 (205).
   // RBC_OPT_BATCH 0 runs every launch field by field with the same arithmetic.
   bool confined_fused_ok() {
     if (periodic || mixed || solid_on || !use_bands || !xg_ok() || !vel_same || !confined_rows_supported(nx, ny)) return false;
@@ -1430,9 +1430,9 @@ class Navier {
     return s0.hxp.op.kind == XOP_BLOCKS && s0.hyp.op.kind == XOP_BLOCKS && same_classes(s0.hxp.op, s2.hxp.op) &&
            same_classes(s0.hyp.op, s2.hyp.op);
   }
-  // the y transforms of the convective terms by DCT: above 200 points the O(n log n) kernels are
-  // ahead of the dense products (257^2, one step: 101 us by DCT, 113 us dense; 128 x 129: 62 and
-  // 53 us; 64 x 65: 58 and 47 us)
+  // the y transforms of the convective terms by DCT: the dense products are ahead below 200 points (a
+  // step of 128 x 129 53 us against 62 by DCT, periodic 32 against 41) and even at the next fast length
+  // (257^2 91.6 against 91.2, periodic 128 x 257 40.9 against 42.0), whose operations grow faster
   bool confined_dct() const { return use_dct && nb == 1 && ny > 200 && cheb_y_supported(ny); }
   // the products `op` (temp: `opt`) of fields f0 <= f < f1: in [op.cols, N] -> out at row stride ldc
   XGemm field_op(const PackedOp& op, const PackedOp& opt, const double* in, int N, double* out, int ldc, int f0, int f1) {
@@ -1951,7 +1951,7 @@ class Navier {
   }
   // The convective terms by products with the dense x operators, the y stage as in the confined step,
   // where there are no fast transforms (160 x 129, 50 steps and their output: 12.3 ms field by field in
-  // some 45 launches a step, 1.9 ms in seven) and on small grids, whose transforms are bound by their
+  // some 45 launches a step, 1.8 ms in seven) and on small grids, whose transforms are bound by their
   // launches and passes: us per step by transforms / products on MI355X, 64 x 65 50.5 / 32.7 (before the
   // row kernels' lane scans), 512 x 129 60.1 / 52.6, 128 x 257 46.0 / 42.0, 256 x 257
   // 51.5 / 51.6, 512 x 257 65 / 78, 256 x 513 68 / 75.
