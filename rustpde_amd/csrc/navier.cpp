@@ -3402,8 +3402,9 @@ class Adjoint {
         for (int i = 0; i < 3; ++i) p[i] = q ? &n.solver[i]->pbp : &n.solver[i]->pfp;
         packed3[q] = same3(*p[0], *p[1], *p[2]);
         DBuf& slab = q ? SMB : SMF;
-        if (slab.n != 3 * p[0]->buf.n) slab.alloc(3 * std::max({p[0]->buf.n, p[1]->buf.n, p[2]->buf.n}));
-        const size_t each = slab.n / 3;
+        // equal places for the largest of the three: a tensor set from outside may pack to another size
+        const size_t each = std::max({p[0]->buf.n, p[1]->buf.n, p[2]->buf.n});
+        if (slab.n != 3 * each) slab.alloc(3 * each);
         for (int i = 0; i < 3; ++i) {
           std::vector<double> v = p[i]->buf.download(p[i]->buf.n);
           if (q)
