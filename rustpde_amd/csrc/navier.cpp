@@ -29,6 +29,9 @@ namespace rbc {
 struct DeviceError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
+struct OutOfMemory : DeviceError {
+  using DeviceError::DeviceError;
+};
 struct NumericError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
@@ -62,7 +65,13 @@ struct DBuf {
   void alloc(size_t count) {
     release();
     if (count == 0) count = 1;
-    HIPCHECK(hipMalloc(&p, count * sizeof(double)));
+    const hipError_t e = hipMalloc(&p, count * sizeof(double));
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();  // the next launch's check does not find it
+      p = nullptr;
+      throw OutOfMemory("hipMalloc of " + std::to_string(count * sizeof(double)) + " bytes: " + hipGetErrorString(e));
+    }
+    HIPCHECK(e);
     n = count;
     HIPCHECK(hipMemset(p, 0, count * sizeof(double)));
   }
@@ -2648,6 +2657,7 @@ class Space {
   hipStream_t st = nullptr;
   OpCache X, Y;
   DBuf W1, W2, W3, W4;
+  size_t work_size = 0;  // doubles that the current chunk's work arrays hold
   Space(int k0, int n0, int k1, int n1) : b0((Kind)k0, n0), b1((Kind)k1, n1), cplx(k0 == FO), X(false, 1.0), Y(true, 1.0) {
     if (k1 == FO) throw std::invalid_argument("axis 1 must be a Chebyshev basis");
     if (n0 < 6 || n1 < 6) throw std::invalid_argument("sizes must be >= 6");
@@ -2664,17 +2674,25 @@ class Space {
   const double* stencil_coef() {
     if (b1.k == CHEB) return nullptr;
     if (!band) {
-      band = std::make_unique<DBand>();
-      make_stencil_band(b1, *band);
+      auto t = std::make_unique<DBand>();
+      make_stencil_band(b1, *t);
+      band = std::move(t);
     }
     return band->coef.p;
   }
   const double* tdma_tab() {
     if (!tdma) {
-      tdma = std::make_unique<DTdma>();
-      make_tdma(b1, *tdma);
+      auto t = std::make_unique<DTdma>();
+      make_tdma(b1, *t);
+      tdma = std::move(t);
     }
     return tdma->tabp.p;
+  }
+  // a work array of the current chunk, made when an operator first needs it: the row operators on
+  // interleaved arrays take none, most transforms one
+  double* work(DBuf& w) {
+    if (w.n < work_size) w.alloc(work_size);
+    return w.p;
   }
   // axis-1 bases and lengths of the row kernels (rowops.hip)
   bool rows_ok() const { return (b1.k == CHEB || b1.k == CD || b1.k == CN) && row_ops_supported(b1.n); }
@@ -2718,7 +2736,7 @@ class Space {
         return out;
       }
       if (op_name == "FS" && (b1.k == CHEB || rows_ok())) {
-        double* to = b1.k == CHEB ? out : W3.p;
+        double* to = b1.k == CHEB ? out : work(W3);
         cheb_y_forward(st, in, b1.n, to, b1.n, (int)rows, b1.n, b1.n);
         if (b1.k != CHEB) composite_rows(st, to, out, rows, false, b1.m, tdma_tab());
         return out;
@@ -2764,16 +2782,26 @@ class Space {
     const bool inplace = overlap(in, in_sz * batch, out, out_sz * batch);
     const size_t rows = (size_t)std::max(r_ortho(), b0.n);
     const size_t most = std::max<size_t>(1, std::min(CHUNK_DOUBLES / big, CHUNK_ROWS / rows));
-    const int chunk = inplace ? 1 : (int)std::min<size_t>((size_t)std::min(batch, 65535), most);
-    if (inplace && W4.n < big) W4.alloc(big);
-    for (DBuf* w : {&W1, &W2, &W3})
-      if (w->n < big * chunk) w->alloc(big * chunk);
+    int chunk = inplace ? 1 : (int)std::min<size_t>((size_t)std::min(batch, 65535), most);
     GemmNoTune no_tune;  // a call's first use of a shape is not spent on timing tiles
-    for (int b = 0; b < batch; b += chunk) {
+    bool fresh = false;  // one field at a time, with no work arrays left from before
+    for (int b = 0; b < batch;) {
       const int nb = std::min(chunk, batch - b);
       double* dst = out + b * out_sz;
-      const double* r = apply(op, in + b * in_sz, inplace ? W4.p : dst, nb, in_r, in_c1, out_r, out_c1, d0, d1, s0, s1);
-      if (r != dst) HIPCHECK(hipMemcpyAsync(dst, r, sizeof(double) * out_sz * nb, hipMemcpyDeviceToDevice, st));
+      try {
+        work_size = big * nb;
+        const double* r =
+            apply(op, in + b * in_sz, inplace ? work(W4) : dst, nb, in_r, in_c1, out_r, out_c1, d0, d1, s0, s1);
+        if (r != dst) HIPCHECK(hipMemcpyAsync(dst, r, sizeof(double) * out_sz * nb, hipMemcpyDeviceToDevice, st));
+      } catch (const OutOfMemory&) {  // a nearly full card: smaller chunks, down to a field's work arrays
+        HIPCHECK(hipStreamSynchronize(st));
+        for (DBuf* w : {&W1, &W2, &W3, &W4}) w->release();
+        if (nb == 1 && fresh) throw;
+        fresh = nb == 1;
+        chunk = std::max(1, nb / 2);
+        continue;
+      }
+      b += nb;
     }
     HIPCHECK(hipStreamSynchronize(st));
   }
@@ -2795,19 +2823,19 @@ class Space {
     }
     if (pairs && fft_supported(b0.n) && op < 2) {
       if (op == 0) {
-        rfft_cols_interleaved(st, yop("FS", src, (long)nb * b0.n, W1.p), dst, b0.n, b1.m, nb);
+        rfft_cols_interleaved(st, yop("FS", src, (long)nb * b0.n, work(W1)), dst, b0.n, b1.m, nb);
         return dst;
       }
-      irfft_cols_interleaved(st, src, W1.p, b0.n, b1.m, nb);
-      return yop("BS", W1.p, (long)nb * b0.n, dst);
+      irfft_cols_interleaved(st, src, work(W1), b0.n, b1.m, nb);
+      return yop("BS", work(W1), (long)nb * b0.n, dst);
     }
     if (!cplx && op < 2 && !y_fast(op)) {  // both products with transposed results, parity classes along both axes
       const char* name = op == 0 ? "FS" : "BS";
       const PackedOp &px = X.packed(b0, name), &py = Y.packed(b1, name);
-      XGemm g = xgemm_of(px, src, W1.p, py.op.cols, nb, (long)px.op.cols * py.op.cols, (long)px.op.rows * py.op.cols);
+      XGemm g = xgemm_of(px, src, work(W1), py.op.cols, nb, (long)px.op.cols * py.op.cols, (long)px.op.rows * py.op.cols);
       g.ldc = px.op.rows;
       xgemm_t(st, &g, 1);
-      g = xgemm_of(py, W1.p, dst, px.op.rows, nb, (long)px.op.rows * py.op.cols, (long)px.op.rows * py.op.rows);
+      g = xgemm_of(py, work(W1), dst, px.op.rows, nb, (long)px.op.rows * py.op.cols, (long)px.op.rows * py.op.rows);
       g.ldc = py.op.rows;
       xgemm_t(st, &g, 1);
       return dst;
@@ -2815,21 +2843,21 @@ class Space {
     const bool in_c = cplx && op != 0, out_c = cplx && op != 1;
     const double* x = src;
     if (in_c) {
-      interleaved_to_split(st, src, W3.p, in_r / 2, in_c1, nb);
-      x = W3.p;
+      interleaved_to_split(st, src, work(W3), in_r / 2, in_c1, nb);
+      x = work(W3);
     }
-    double* last = out_c ? W2.p : dst;  // where the second operator writes
+    double* last = out_c ? work(W2) : dst;  // where the second operator writes
     const double* r;
     if (op == 0) {  // forward: axis 1 then axis 0
-      r = xop("FS", yop("FS", x, (long)nb * b0.n, W1.p), b1.m, last, nb);
+      r = xop("FS", yop("FS", x, (long)nb * b0.n, work(W1)), b1.m, last, nb);
     } else if (op == 1) {  // backward: axis 0 then axis 1
-      r = yop("BS", xop("BS", x, b1.m, W1.p, nb), (long)nb * b0.n, last);
+      r = yop("BS", xop("BS", x, b1.m, work(W1), nb), (long)nb * b0.n, last);
     } else if (op == 2) {
-      r = yop("S", xop("S", x, b1.m, W1.p, nb), (long)nb * r_ortho(), last);
+      r = yop("S", xop("S", x, b1.m, work(W1), nb), (long)nb * r_ortho(), last);
     } else if (op == 3) {
-      r = yop("FO", xop("FO", x, b1.n, W1.p, nb), (long)nb * r_spec(), last);
+      r = yop("FO", xop("FO", x, b1.n, work(W1), nb), (long)nb * r_spec(), last);
     } else {
-      r = yop(dn[d1], xop(dn[d0], x, b1.m, W1.p, nb), (long)nb * r_ortho(), last);
+      r = yop(dn[d1], xop(dn[d0], x, b1.m, work(W1), nb), (long)nb * r_ortho(), last);
       if (sc != 1.0) {
         const size_t e = (size_t)r_ortho() * b1.n;
         if (b0.k == FO) {  // complex division by (sc, 0): (a sc) / sc^2 per component
