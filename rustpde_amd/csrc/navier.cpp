@@ -2792,6 +2792,10 @@ class Space {
         work_size = big * nb;
         const double* r =
             apply(op, in + b * in_sz, inplace ? work(W4) : dst, nb, in_r, in_c1, out_r, out_c1, d0, d1, s0, s1);
+        if (inplace && r != dst && r != W4.p) {  // an identity's input: no copy between ranges that may overlap
+          HIPCHECK(hipMemcpyAsync(W4.p, r, sizeof(double) * out_sz, hipMemcpyDeviceToDevice, st));
+          r = W4.p;
+        }
         if (r != dst) HIPCHECK(hipMemcpyAsync(dst, r, sizeof(double) * out_sz * nb, hipMemcpyDeviceToDevice, st));
       } catch (const OutOfMemory&) {  // a nearly full card: smaller chunks, down to a field's work arrays
         HIPCHECK(hipStreamSynchronize(st));
