@@ -3056,6 +3056,8 @@ class SolverDev {
            !Space::overlap(rhs, in_size() * batch, out, out_size() * batch);
   }
   void solve_ws(const double* rhs, double* out, int batch, const Work& w) {
+    // the entry point's limit, that of a grid axis in the products of the mixed form
+    if (!cplx && batch > 65535) throw std::invalid_argument("solver: batch exceeds 65535");
     const int o1 = b1.ortho(), m1 = b1.m, m0 = b0.m, ro = rows_out();
     const size_t in_sz = in_size(), out_sz = out_size();
     const double* x = rhs;
