@@ -212,6 +212,28 @@ static void make_tdma(const Basis& b, DTdma& t) {
   }));
 }
 
+// the tables of composite_rows
+struct DComposite {
+  DBuf tab;
+  Composite c;
+};
+static void make_composite(const Basis& b, DComposite& d) {
+  const int n = b.n;
+  std::vector<ld> w(n, 1.0L);
+  for (int i = n - 3; i >= 0; --i) w[i] = -(ld)b.low2[i] * w[i + 2];
+  for (int p = 0; p < 2; ++p) {
+    ld s = 0.0L;
+    for (int i = p; i < n; i += 2) s += w[i] * w[i];
+    d.c.iw[p] = (double)(1.0L / s);
+  }
+  d.c.m = b.m;
+  if (b.k == CD) return;
+  d.tab.upload(slice_order(1, n, 2, [&](int, int a, int i, int t, int) -> double {
+    return a == 0 ? (double)w[i] : t >= 1 ? b.low2[i - 2] : 0.0;
+  }));
+  d.c.tab = d.tab.p;
+}
+
 static ld ipow(ld x, int e) {
   ld r = 1.0L;
   for (int i = 0; i < e; ++i) r *= x;
@@ -2670,7 +2692,7 @@ class Space {
   int r_spec() const { return cplx ? 2 * b0.m : b0.m; }
   int r_ortho() const { return cplx ? 2 * b0.m : b0.n; }
   std::unique_ptr<DBand> band;  // stencil taps of a composite axis-1 basis
-  std::unique_ptr<DTdma> tdma;  // its from_ortho tables
+  std::unique_ptr<DComposite> comp;  // its from_ortho tables
   const double* stencil_coef() {
     if (b1.k == CHEB) return nullptr;
     if (!band) {
@@ -2680,13 +2702,13 @@ class Space {
     }
     return band->coef.p;
   }
-  const double* tdma_tab() {
-    if (!tdma) {
-      auto t = std::make_unique<DTdma>();
-      make_tdma(b1, *t);
-      tdma = std::move(t);
+  const Composite& composite() {
+    if (!comp) {
+      auto t = std::make_unique<DComposite>();
+      make_composite(b1, *t);
+      comp = std::move(t);
     }
-    return tdma->tabp.p;
+    return comp->c;
   }
   // a work array of the current chunk, made when an operator first needs it: the row operators on
   // interleaved arrays take none, most transforms one
@@ -2738,7 +2760,7 @@ class Space {
       if (op_name == "FS" && (b1.k == CHEB || rows_ok())) {
         double* to = b1.k == CHEB ? out : work(W3);
         cheb_y_forward(st, in, b1.n, to, b1.n, (int)rows, b1.n, b1.n);
-        if (b1.k != CHEB) composite_rows(st, to, out, rows, false, b1.m, tdma_tab());
+        if (b1.k != CHEB) composite_rows(st, to, out, rows, false, composite());
         return out;
       }
     }
@@ -2749,7 +2771,7 @@ class Space {
         return out;
       }
       if (op_name == "FO") {
-        composite_rows(st, in, out, rows, false, b1.m, tdma_tab());
+        composite_rows(st, in, out, rows, false, composite());
         return out;
       }
     }
@@ -2821,7 +2843,7 @@ class Space {
     if (pairs && rows_ok() && op >= 2) {
       const long rows = (long)nb * b0.m;
       if (op == 3 && b1.k == CHEB) return src;
-      if (op == 3) composite_rows(st, src, dst, rows, true, b1.m, tdma_tab());
+      if (op == 3) composite_rows(st, src, dst, rows, true, composite());
       else ortho_rows(st, src, dst, rows, true, b1.m, b1.n, stencil_coef(), op == 4 ? d1 : 0, op == 4 ? d0 : 0, b0.m, sc);
       return dst;
     }

@@ -452,10 +452,16 @@ void split_to_interleaved(hipStream_t s, const double* in, double* out, int m, i
 // ortho_rows: mi composite coefficients (coef: stencil taps [2][n]; null: Chebyshev, mi = n)
 // -> n Chebyshev coefficients of the d1-th derivative; complex rows first times (i k)^d0,
 // k = row mod m0, and divided by sc last, real rows times sc last.
-// composite_rows: from_ortho, m + 2 values -> m (tabp: the tables of tdma_rows_lds).
+// composite_rows: from_ortho, m + 2 values -> m.
 bool row_ops_supported(int n);
 void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int mi, int n, const double* coef,
                 int d1, int d0, int m0, double sc);
-void composite_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int m, const double* tabp);
+struct Composite {
+  int m = 0;
+  // of chains of m + 2 values in slice order: w and l_{t-1} (see composite_rows_kernel; null: Dirichlet)
+  const double* tab = nullptr;
+  double iw[2] = {};  // 1 / (w w)
+};
+void composite_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, const Composite& c);
 
 }  // namespace rbc

@@ -114,12 +114,20 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
   }
 }
 
-// from_ortho of every row (composite_stencil.rs:250-276, linalg.rs:14-57), the recurrences of
-// tdma_rows_lds.  in: m + 2 values per row, out: m.
+// from_ortho of every row (composite_stencil.rs:250-276): the least squares x of S x = q, S the stencil
+// q_t = x_t + l_{t-1} x_{t-1} along a parity chain of one value more than x has.  What S x cannot reach is
+// along w, S^T w = 0 (w_t = -l_t w_{t+1}); with it taken off, r = q - w (w q) / (w w), S x = r is solved from
+// either end: Dirichlet (l = -1, w = 1: tab null) by suffix sums, x_t = -(r_{t+1} + r_{t+2} + ..), from the
+// small coefficients down; Neumann (-1 < l <= 0) by x_t = r_t - l_{t-1} x_{t-1}, tab holding w and l_{t-1} in
+// slice order.  iw: 1 / (w w) of the two chains.  w is taken off twice, the second time what rounding left.
+// Rounding against 64 bits, rows of 257 coefficients that fall off as k^-2: Dirichlet 2e-16, Neumann 1e-16 of
+// the result (dense product 6e-16 and 3e-16; the normal equations S^T S x = S^T q of linalg.rs:14-57, whose
+// condition grows as the square, 1.2e-14 and 1.5e-15).  in: n = m + 2 values per row, out: m.
 template <int SLICE, bool CPLX>
 __global__ __launch_bounds__(WAVE* WAVES) void composite_rows_kernel(const double* __restrict__ in,
                                                                      double* __restrict__ out, long rows, int m, int per,
-                                                                     int bl, const double* __restrict__ tab) {
+                                                                     int bl, const double* __restrict__ tab, double iw0,
+                                                                     double iw1) {
 #pragma clang fp contract(off)
   extern __shared__ double lds[];
   const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x / WAVE;
@@ -142,30 +150,45 @@ __global__ __launch_bounds__(WAVE* WAVES) void composite_rows_kernel(const doubl
     }
   }
   __syncthreads();
-  const int len = p == 0 ? (m + 1) / 2 : m / 2;
+  const int len = p == 0 ? (n + 1) / 2 : n / 2;  // values q of the chain; x has one less
   const int t0 = lane * per, cnt = max(0, min(per, len - t0));
-  double v[SLICE], c0[SLICE], c1[SLICE];
-#define TB(a, q) tab[((size_t)((a) * 2 + p) * per + (q)) * WAVE + lane]
+  double v[SLICE], nw[SLICE], l[SLICE];
 #pragma unroll
   for (int q = 0; q < SLICE; ++q) {
-    c0[q] = TB(0, q);
-    c1[q] = TB(1, q);
+    v[q] = q < cnt ? buf[pad(p + 2 * (t0 + q) + 2)] : 0.0;
+    nw[q] = q < cnt ? 1.0 : 0.0;
+    l[q] = -1.0;
+    if (tab) {
+      nw[q] = tab[((size_t)p * per + q) * WAVE + lane];
+      l[q] = tab[((size_t)(2 + p) * per + q) * WAVE + lane];
+    }
   }
+  const double iw = p ? iw1 : iw0;
 #pragma unroll
-  for (int q = 0; q < SLICE; ++q) {
-    const int j = p + 2 * (t0 + q) + 2;
-    v[q] = q < cnt ? buf[pad(j)] * c0[q] + buf[pad(j + 2)] * c1[q] : 0.0;
+  for (int k = 0; k < 2; ++k) {
+    double s = 0.0, above;
+#pragma unroll
+    for (int q = 0; q < SLICE; ++q)
+      if (q < cnt) s = s + nw[q] * v[q];
+    const double a = wave::lane_value(wave::suffix_sum(s, lane, above), 0) * iw;
+#pragma unroll
+    for (int q = 0; q < SLICE; ++q)
+      if (q < cnt) v[q] = __builtin_fma(-a, nw[q], v[q]);
   }
+  if (tab) {
+    chains::fdma_forward(v, l, lane, t0, cnt);
+  } else {
+    double s = 0.0, above;
 #pragma unroll
-  for (int q = 0; q < SLICE; ++q) {
-    c0[q] = TB(2, q);
-    c1[q] = TB(3, q);
+    for (int q = SLICE - 1; q >= 0; --q) s = s + v[q];
+    wave::suffix_sum(s, lane, above);
+#pragma unroll
+    for (int q = SLICE - 1; q >= 0; --q) {
+      const double r = v[q];
+      v[q] = -above;
+      above = above + r;
+    }
   }
-  chains::tdma_forward(v, c0, c1, lane, t0, cnt);
-#pragma unroll
-  for (int q = 0; q < SLICE; ++q) c0[q] = TB(4, q);
-#undef TB
-  chains::tdma_backward(v, c0, lane, t0, cnt, p, m);
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < SLICE; ++q)
@@ -208,12 +231,13 @@ void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cp
   check("ortho_rows");
 }
 
-void composite_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int m, const double* tabp) {
-  if (!row_ops_supported(m + 2) || !tdma_rows_lds_supported(m)) throw std::invalid_argument("composite_rows: bad length");
+void composite_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, const Composite& c) {
+  const int n = c.m + 2, m = c.m;
+  if (!row_ops_supported(n)) throw std::invalid_argument("composite_rows: bad length");
   if (rows < 1 || rows > 0x3fffffff) throw std::invalid_argument("composite_rows: bad rows");
-  const int per = fdma_rows_lds_per(m), bl = buf_len(m + 2);
-  if (cplx) RBC_ROW_OP(composite_rows_kernel, true, per, in, out, rows, m, per, bl, tabp);
-  else RBC_ROW_OP(composite_rows_kernel, false, per, in, out, rows, m, per, bl, tabp);
+  const int per = fdma_rows_lds_per(n), bl = buf_len(n);
+  if (cplx) RBC_ROW_OP(composite_rows_kernel, true, per, in, out, rows, m, per, bl, c.tab, c.iw[0], c.iw[1]);
+  else RBC_ROW_OP(composite_rows_kernel, false, per, in, out, rows, m, per, bl, c.tab, c.iw[0], c.iw[1]);
   check("composite_rows");
 }
 
