@@ -78,7 +78,11 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
     }
   }
   __syncthreads();
-  if (coef) {  // stencil taps, zero where absent
+  if (coef && d1 == 1) {
+    rowdiff::derive_composite<SLICE>(buf, coef + n + 2, n, per, lane, p);
+  } else if (coef && d1 == 2) {
+    rowdiff::derive2_composite<SLICE>(buf, coef + n + 2, n, per, lane, p);
+  } else if (coef) {  // stencil taps, zero where absent
     double v[MAXQ];
 #pragma unroll
     for (int q = 0; q < MAXQ; ++q) {
@@ -93,7 +97,8 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
     }
     __syncthreads();
   }
-  for (int t = 0; t < d1; ++t) rowdiff::derive<SLICE>(buf, n, per, lane, p);
+  if (!coef)
+    for (int t = 0; t < d1; ++t) rowdiff::derive<SLICE>(buf, n, per, lane, p);
   if constexpr (CPLX) {
     const double ns = sc * sc + 0.0 * 0.0;
     for (int i = threadIdx.x; i < n; i += WAVE * WAVES) {
@@ -220,7 +225,7 @@ bool row_ops_supported(int n) { return n >= 6 && fdma_rows_lds_per(n) <= 16; }
 
 void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int mi, int n, const double* coef,
                 int d1, int d0, int m0, double sc) {
-  if (!row_ops_supported(n) || mi > n || (!coef && mi != n) || d1 < 0 || d0 < 0 || (d0 > 0 && m0 < 1))
+  if (!row_ops_supported(n) || mi > n || (!coef && mi != n) || d1 < 0 || (coef && d1 > 2) || d0 < 0 || (d0 > 0 && m0 < 1))
     throw std::invalid_argument("ortho_rows: bad arguments");
   if (rows < 1 || rows > 0x3fffffff) throw std::invalid_argument("ortho_rows: bad rows");
   const int per = fdma_rows_lds_per(n), bl = buf_len(n);

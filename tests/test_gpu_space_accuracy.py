@@ -43,7 +43,7 @@ def _rounding(got, want):
 
 @pytest.mark.parametrize("kind", [DIRICHLET, NEUMANN])
 @pytest.mark.parametrize("n", [24, 65, 130, 257, 300, 513])
-@pytest.mark.parametrize("op", ["proj"])
+@pytest.mark.parametrize("op", ["ortho", "dy", "dyy", "proj"])
 def test_row_operators_round_as_dense_products(n, kind, op):
     from rustpde_amd import Space2
     print("case rounding", n, kind, op, flush=True)
