@@ -36,7 +36,9 @@ void check(const char* what) {
 // d1 derivatives (ortho.rs:107-125) of the to_ortho stencil (composite_stencil.rs:207-229) of
 // every row, (i k)^d0 (r2c.rs:88-99) applied first and the division by sc last (complex rows;
 // real rows multiply by sc, the caller's reciprocal).  in: mi values per row, out: n.
-template <int SLICE, bool CPLX>
+// COMP: the derivative of a composite row that is formed at once (0: to_ortho, then d1 plain derivatives); the
+// second one's registers would cost the others a block per CU.
+template <int SLICE, bool CPLX, int COMP>
 __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* __restrict__ in, double* __restrict__ out,
                                                                  long rows, int mi, int n, int per, int bl,
                                                                  const double* __restrict__ coef, int d1, int d0, int m0,
@@ -78,9 +80,9 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
     }
   }
   __syncthreads();
-  if (coef && d1 == 1) {
+  if constexpr (COMP == 1) {
     rowdiff::derive_composite<SLICE>(buf, coef + n + 2, n, per, lane, p);
-  } else if (coef && d1 == 2) {
+  } else if constexpr (COMP == 2) {
     rowdiff::derive2_composite<SLICE>(buf, coef + n + 2, n, per, lane, p);
   } else if (coef) {  // stencil taps, zero where absent
     double v[MAXQ];
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(WAVE* WAVES) void ortho_rows_kernel(const double* _
     }
     __syncthreads();
   }
-  if (!coef)
+  if constexpr (COMP == 0)
     for (int t = 0; t < d1; ++t) rowdiff::derive<SLICE>(buf, n, per, lane, p);
   if constexpr (CPLX) {
     const double ns = sc * sc + 0.0 * 0.0;
@@ -213,15 +215,25 @@ __global__ __launch_bounds__(WAVE* WAVES) void composite_rows_kernel(const doubl
 // the slices of a row of n values: at most 16 entries per lane and chain
 bool row_ops_supported(int n) { return n >= 6 && fdma_rows_lds_per(n) <= 16; }
 
-#define RBC_ROW_OP(KERNEL, CPLX, per, ...)                                                                   \
-  do {                                                                                                       \
-    const dim3 grid((unsigned)((CPLX) ? rows : (rows + 1) / 2)), block(WAVE * WAVES);                         \
-    if ((per) <= 2) RBC_LAUNCH((KERNEL<2, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
-    else if ((per) <= 4) RBC_LAUNCH((KERNEL<4, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);      \
-    else if ((per) <= 6) RBC_LAUNCH((KERNEL<6, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__); \
-    else if ((per) <= 8) RBC_LAUNCH((KERNEL<8, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__); \
-    else RBC_LAUNCH((KERNEL<16, CPLX>), grid, block, 2 * bl * sizeof(double), s, __VA_ARGS__);                \
+#define RBC_ROW_OP(KERNEL, blocks, per, PARAMS, ...)                                             \
+  do {                                                                                          \
+    const dim3 grid((unsigned)(blocks)), block(WAVE * WAVES);                                   \
+    const size_t sh = 2 * bl * sizeof(double);                                                  \
+    if ((per) <= 2) RBC_LAUNCH((KERNEL<2, PARAMS>), grid, block, sh, s, __VA_ARGS__);           \
+    else if ((per) <= 4) RBC_LAUNCH((KERNEL<4, PARAMS>), grid, block, sh, s, __VA_ARGS__);      \
+    else if ((per) <= 6) RBC_LAUNCH((KERNEL<6, PARAMS>), grid, block, sh, s, __VA_ARGS__);      \
+    else if ((per) <= 8) RBC_LAUNCH((KERNEL<8, PARAMS>), grid, block, sh, s, __VA_ARGS__);      \
+    else RBC_LAUNCH((KERNEL<16, PARAMS>), grid, block, sh, s, __VA_ARGS__);                     \
   } while (0)
+
+template <bool CPLX, int COMP>
+static void launch_ortho(hipStream_t s, const double* in, double* out, long rows, int mi, int n, int per, int bl,
+                         const double* coef, int d1, int d0, int m0, double sc, double isc) {
+#define RBC_PARAMS CPLX, COMP
+  RBC_ROW_OP(ortho_rows_kernel, CPLX ? rows : (rows + 1) / 2, per, RBC_PARAMS, in, out, rows, mi, n, per, bl, coef, d1, d0,
+             m0, sc, isc);
+#undef RBC_PARAMS
+}
 
 void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cplx, int mi, int n, const double* coef,
                 int d1, int d0, int m0, double sc) {
@@ -231,8 +243,16 @@ void ortho_rows(hipStream_t s, const double* in, double* out, long rows, bool cp
   const int per = fdma_rows_lds_per(n), bl = buf_len(n);
   int ex = 0;
   const double isc = sc > 0.0 && sc != 1.0 && std::frexp(sc, &ex) == 0.5 ? 1.0 / sc : 0.0;
-  if (cplx) RBC_ROW_OP(ortho_rows_kernel, true, per, in, out, rows, mi, n, per, bl, coef, d1, d0, m0, sc, isc);
-  else RBC_ROW_OP(ortho_rows_kernel, false, per, in, out, rows, mi, n, per, bl, coef, d1, 0, 1, sc, 0.0);
+  const int comp = coef ? d1 : 0;
+  if (!cplx) {
+    d0 = 0;
+    m0 = 1;
+  }
+#define RBC_ORTHO(C, D) launch_ortho<C, D>(s, in, out, rows, mi, n, per, bl, coef, d1, d0, m0, sc, C ? isc : 0.0)
+  if (comp == 0) cplx ? RBC_ORTHO(true, 0) : RBC_ORTHO(false, 0);
+  else if (comp == 1) cplx ? RBC_ORTHO(true, 1) : RBC_ORTHO(false, 1);
+  else cplx ? RBC_ORTHO(true, 2) : RBC_ORTHO(false, 2);
+#undef RBC_ORTHO
   check("ortho_rows");
 }
 
@@ -241,8 +261,8 @@ void composite_rows(hipStream_t s, const double* in, double* out, long rows, boo
   if (!row_ops_supported(n)) throw std::invalid_argument("composite_rows: bad length");
   if (rows < 1 || rows > 0x3fffffff) throw std::invalid_argument("composite_rows: bad rows");
   const int per = fdma_rows_lds_per(n), bl = buf_len(n);
-  if (cplx) RBC_ROW_OP(composite_rows_kernel, true, per, in, out, rows, m, per, bl, c.tab, c.iw[0], c.iw[1]);
-  else RBC_ROW_OP(composite_rows_kernel, false, per, in, out, rows, m, per, bl, c.tab, c.iw[0], c.iw[1]);
+  if (cplx) RBC_ROW_OP(composite_rows_kernel, rows, per, true, in, out, rows, m, per, bl, c.tab, c.iw[0], c.iw[1]);
+  else RBC_ROW_OP(composite_rows_kernel, (rows + 1) / 2, per, false, in, out, rows, m, per, bl, c.tab, c.iw[0], c.iw[1]);
   check("composite_rows");
 }
 
