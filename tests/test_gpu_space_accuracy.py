@@ -57,3 +57,31 @@ def test_row_operators_round_as_dense_products(n, kind, op):
                "dyy": lambda v: sp.gradient(v, (0, 2), (1.0, 1.0))}[op](f).real
         want, dense = f.real.astype(LD) @ a.T, f.real @ a.astype(float).T
         assert _rounding(got, want) <= 1.5 * _rounding(dense, want), (k0, _rounding(got, want), _rounding(dense, want))
+
+
+@pytest.mark.parametrize("kind", [DIRICHLET, NEUMANN])
+@pytest.mark.parametrize("n", [33, 65, 130, 257, 513])
+def test_forward_rounds_as_dense_products(n, kind):
+    """Real spaces: dense products along both axes, the one along x as it is (a fast transform along y adds
+    its own rounding)."""
+    from rustpde_amd import Space2
+    print("case forward rounding", n, kind, flush=True)
+    m = n - 1
+    cosines = np.cos(4 * np.arctan(LD(1)) * np.arange(2 * m).astype(LD) / m)
+    t = cosines[(np.arange(n)[:, None] * (m - np.arange(n)[None, :])) % (2 * m)]  # T_k(x_j)
+    c = np.ones(n, dtype=LD)
+    c[0] = c[-1] = 2
+    y = _operators(kind, n)["proj"] @ (LD(2) / m * t / (c[:, None] * c))
+    n0 = 24
+    mx = n0 - 1
+    tx = np.cos(4 * np.arctan(LD(1)) * ((np.arange(n0)[:, None] * (mx - np.arange(n0)[None, :])) % (2 * mx)).astype(LD) / mx)
+    cx = np.ones(n0, dtype=LD)
+    cx[0] = cx[-1] = 2
+    x = LD(2) / mx * tx / (cx[:, None] * cx)
+    rng = np.random.default_rng(n)
+    g, h = np.linspace(0, 1, n0)[:, None], np.linspace(0, 1, n)[None, :]
+    v = sum(np.sin(2 * np.pi * (j + 1) * g + j) * np.sin(np.pi * (j + 1) * h) for j in range(3))
+    v = v + 1e-3 * rng.standard_normal(v.shape)
+    want, dense = x @ (v.astype(LD) @ y.T), x.astype(float) @ (v @ y.astype(float).T)
+    got = Space2((CHEB, n0), (kind, n)).forward(v)
+    assert _rounding(got, want) <= 1.5 * _rounding(dense, want), (_rounding(got, want), _rounding(dense, want))
