@@ -2755,14 +2755,16 @@ class Space {
     const std::string op_name = name;
     if (b1.k == CHEB && (op_name == "S" || op_name == "FO")) return in;
     if ((op_name == "BS" && y_fast(1)) || (op_name == "FS" && y_fast(0))) {  // FFT-based DCT-I
+      // two rows share a transform: of one field only, so that none rounds or fails with its neighbours
+      const int per = b0.n % 2 ? b0.n : (int)rows, nb = (int)(rows / per);
       if (op_name == "BS") {
         const double* coef = stencil_coef();
-        cheb_y_backward(st, in, b1.m, b1.m, out, b1.n, (int)rows, b1.n, coef, band ? band->mask.p : nullptr, 0, 1.0,
-                        nullptr, 0, 0.0);
+        cheb_y_backward(st, in, b1.m, b1.m, out, b1.n, per, b1.n, coef, band ? band->mask.p : nullptr, 0, 1.0,
+                        nullptr, 0, 0.0, nb, (long)per * b1.m, (long)per * b1.n);
         return out;
       }
       double* to = b1.k == CHEB ? out : work(W3);
-      cheb_y_forward(st, in, b1.n, to, b1.n, (int)rows, b1.n, b1.n);
+      cheb_y_forward(st, in, b1.n, to, b1.n, per, b1.n, b1.n, nb, (long)per * b1.n, (long)per * b1.n);
       if (b1.k != CHEB) composite_rows(st, to, out, rows, false, composite());
       return out;
     }
