@@ -1441,8 +1441,10 @@ class Navier {
   // ------------------------------------------------- the confined FP64 step (navier.rs:737-765)
   // The dense operators as parity-class products along x or, on transposed arrays, along y
   // (xgemm.hip), and what lies between them as row kernels (confined.hip): 12 launches, 13 with the
-  // y transforms by DCT, where stencils, derivatives, sums and products of their own took 29.  A
-  // step takes 38 us at 64^2 (105 before), 44 us at 128 x 129 (173), 91 us at 257^2 (205).
+  // y transforms by DCT, where stencils, derivatives, sums and products of their own took 29.  The first
+  // stage is three launches instead of one where its operators, of nx and nx - 2 columns, pad to
+  // different lengths (nx = 65, 66, 129, 130, 257, 258 and the like): 257^2 takes 15.  A step takes 38 us at
+  // 64^2 (105 before), 44 us at 128 x 129 (173), 91 us at 257^2 (205).
   // RBC_OPT_BATCH 0 runs every launch field by field with the same arithmetic.
   bool confined_fused_ok() {
     if (periodic || mixed || solid_on || !use_bands || !xg_ok() || !vel_same || !confined_rows_supported(nx, ny)) return false;
@@ -1462,8 +1464,8 @@ class Navier {
            same_classes(s0.hyp.op, s2.hyp.op);
   }
   // the y transforms of the convective terms by DCT: the dense products are ahead below 200 points (a
-  // step of 128 x 129 53 us against 62 by DCT, periodic 32 against 41) and even at the next fast length
-  // (257^2 91.6 against 91.2, periodic 128 x 257 40.9 against 42.0), whose operations grow faster
+  // step of 128 x 129 44 us against 55 by DCT, periodic 29 against 39) and even at the next fast length
+  // (257^2 91.4 against 90.8, periodic 128 x 257 38.9 against 39.7), whose operations grow faster
   bool confined_dct() const { return use_dct && nb == 1 && ny > 200 && cheb_y_supported(ny); }
   // the products `op` (temp: `opt`) of fields f0 <= f < f1: in [op.cols, N] -> out at row stride ldc
   XGemm field_op(const PackedOp& op, const PackedOp& opt, const double* in, int N, double* out, int ldc, int f0, int f1) {
@@ -1982,9 +1984,9 @@ class Navier {
   }
   // The convective terms by products with the dense x operators, the y stage as in the confined step,
   // where there are no fast transforms (160 x 129, 50 steps and their output: 12.3 ms field by field in
-  // some 45 launches a step, 1.8 ms in seven) and on small grids, whose transforms are bound by their
+  // some 45 launches a step, 1.8 ms in six) and on small grids, whose transforms are bound by their
   // launches and passes: us per step by transforms / products on MI355X, 64 x 65 50.5 / 32.7 (before the
-  // row kernels' lane scans), 512 x 129 60.1 / 52.6, 128 x 257 46.0 / 42.0, 256 x 257
+  // row kernels' lane scans; 24.9 with them), 512 x 129 60.1 / 52.6, 128 x 257 46.0 / 42.0, 256 x 257
   // 51.5 / 51.6, 512 x 257 65 / 78, 256 x 513 68 / 75.
   bool dense_sizes() const {
     if (!periodic) return false;
@@ -2241,9 +2243,10 @@ class Navier {
     if (!use_conv3 || !cheb_y_supported(ny) || by_u.k != CD || by_u.n != ny || by_u.m != ny - 2 ||
         !dirichlet_taps(by_u))
       return false;
-    // one block per x-row runs six transforms in turn, four blocks per CU: below four blocks
-    // per CU the three separate launches are faster (measured at 256 x 257: 14,530 against
-    // 13,880 steps/s; at 1024 x 1025 the one launch wins, 5,558 against 5,465)
+    // One block per x-row runs six transforms in turn, four blocks per CU.  The line was drawn where the
+    // three separate launches were ahead below four blocks per CU (256 x 257 13,880 steps/s against 14,530).
+    // With the other launches as they are now, a step takes, three launches / one: 1024 x 1025 148.9 / 139.7
+    // us, 512 x 513 70.6 / 68.6, 256 x 257 42.8 / 41.4.
     return use_conv3 == 2 || nx >= 4 * device_cus();
   }
   static int device_cus() {
@@ -3407,7 +3410,7 @@ class Adjoint {
   // The three fields in one launch each: the residuals' smoothers, their x-transformed values and
   // derivatives once (the terms above form them 14 times), the terms in one kernel, the right-hand
   // sides by rows; then the step's own divergence, pressure and projection kernels.  Launches bound it: 96 x
-  // 97, ten iterations, their norms and fields take 1.46 ms as replays of a graph of some 33 launches an
+  // 97, ten iterations, their norms and fields take 1.33 ms as replays of a graph of some 33 launches an
   // iteration, 7.33 ms with some 110 launches term by term.
   DBuf SMF, SMB, BCT, LX;   // smoothers' packed products (pf of the three; pb negated), bc transposed
   bool packed3[2] = {};     // the three operators share their classes: one launch

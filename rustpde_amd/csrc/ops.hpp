@@ -241,7 +241,8 @@ void set_zero_entries(hipStream_t s, double* x, int n_idx, long i0, long i1, int
 void ew_update_pres_group(hipStream_t s, double* p, const double* div, const double* phi, const double* nu,
                           double inv_dt, long n, long stride);
 
-// Weighted column sums: out[j] = sum_i v[i, j] * w[i]  (i sequential, as average.rs:25-34)
+// Weighted column sums: out[j] = sum_i v[i, j] * w[i] (average.rs:25-34), every 32nd row summed in turn, then
+// the 32 sums in pairs
 void col_weighted_sum(hipStream_t s, const double* v, int n0, int n1, const double* w, double* out);
 // out (16-byte aligned, pinned host memory): the n values a and b, interleaved
 void read_out(hipStream_t s, const double* a, const double* b, double* out, long n);
@@ -346,12 +347,6 @@ void rhs_rows(hipStream_t s, const ConfinedRows& a, int nb);
 void div_rows(hipStream_t s, const ConfinedRows& a, int nb);
 void proj_rows(hipStream_t s, const ConfinedRows& a, int nb, bool pressure);
 
-// The pressure stage of the periodic step fused per x-wavenumber (one workgroup per k):
-// divergence, Poisson rows (pseu(0,0) = 0), projection of ux and uy, pressure update.
-// Fields are split-plane spectral arrays: ux, uy [2 mx, mu], pres [2 mx, ny], pseu
-// [2 mx, mu]; su / sp are the stencil taps [2][ny] of the velocity / pseudo-pressure y
-// bases; pybp / pdiag the Poisson solver's P_y taps and diagonal sets and ttab the tdma
-// tables of the velocity y basis, all in slice order.  per and bl are set by the call.
 // Right-hand sides of the periodic step formed by the row solves themselves: rhs3_fused's values with its
 // arguments (U: ux, uy, temp, F apart; stencil [2][ny]; cv FP32 when cv32).
 struct StepRhs {
@@ -361,14 +356,19 @@ struct StepRhs {
   long F;
   double kscale, isc, dt;  // isc = 1 / kscale when kscale is a power of two, else 0
 };
-// ux and uy (fields 0 and 1) solved in place, both with the tables bandp, diagp (mx sets)
-// rows of up to four entries a lane (514 points): a step with / without, 64 x 65 25.0 / 27.3 us, 512 x 257
+// ux and uy (fields 0 and 1) solved in place, both with the tables bandp, diagp (mx sets): rows of up to four entries a lane (514 points): a step with / without, 64 x 65 25.0 / 27.3 us, 512 x 257
 // 62.8 / 65.1, 1024 x 513 109 / 116; with eight entries the values in flight cost the kernels their
 // occupancy (1024 x 1025 mixed: 82.6 us in two launches against 72.3 in three)
 constexpr int STEP_SLICE = 4;
 bool step_rows_supported(int ny);
 void step_rows(hipStream_t s, const StepRhs& a, double* X, const double* bandp, const double* diagp);
 
+// The pressure stage of the periodic step fused per x-wavenumber (one workgroup per k):
+// divergence, Poisson rows (pseu(0,0) = 0), projection of ux and uy, pressure update.
+// Fields are split-plane spectral arrays: ux, uy [2 mx, mu], pres [2 mx, ny], pseu
+// [2 mx, mu]; su / sp are the stencil taps [2][ny] of the velocity / pseudo-pressure y
+// bases; pybp / pdiag the Poisson solver's P_y taps and diagonal sets and ttab the tdma
+// tables of the velocity y basis, all in slice order.  per and bl are set by the call.
 struct PressureArgs {
   double *UX, *UY, *P0, *P1;
   const double *su, *sp, *pybp, *pdiag, *ttab;

@@ -6,9 +6,13 @@
 // that the caller's interleaved arrays need no separate split pass).  Each row is two parity
 // chains, one wavefront each (chains.hpp).  The operators are bound by memory: one read of the
 // input and one write of the output.  At fourier_r2c(512) x cheb_dirichlet(513), 8 fields, one
-// d/dx, d/dy, d2/dy2, to_ortho and from_ortho each take 2,842 us in all as split copies, dense
-// FMA products and merge copies per field, and 127 us as one launch per operator over the batch
-// (15 us a launch; the rest is each call's wait).
+// d/dx, d/dy, d2/dy2, to_ortho and from_ortho each take 2,834 us in all as split copies, dense
+// FMA products and merge copies per field, and 114 us as one launch per operator over the batch
+// (13 us a launch; the rest is each call's wait).
+//
+// The dense products' entries were rounded once from long double, so the rows' own forms are chosen for
+// their rounding: derivatives of the composite basis itself (rowdiff.hpp), from_ortho by the stencil's null
+// vector, not the reference's recurrences over intermediate results.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
