@@ -278,7 +278,10 @@ struct PackedOp {
   DBuf buf;
   XOp op;
   size_t stride() const { return buf.n; }
-  void pack(const std::vector<double>& m, int rows, int cols) {  // row-major rows x cols
+  // row-major rows x cols.  couples: what the operator is known to couple, equal parities (0) or opposite
+  // ones (1), where its entries cannot tell: those of an instance with meaningless parameters are NaN, and its
+  // group's other instances share its launches.
+  void pack(const std::vector<double>& m, int rows, int cols, int couples = -1) {
     auto at = [&](int i, int j) { return m[(size_t)i * cols + j]; };
     op = XOp{};
     op.rows = rows;
@@ -287,6 +290,10 @@ struct PackedOp {
     for (int i = 0; i < rows && (same || flip); ++i)
       for (int j = 0; j < cols; ++j)
         if (at(i, j) != 0.0) (((i + j) & 1) ? same : flip) = false;
+    if (couples >= 0 && !std::all_of(m.begin(), m.end(), [](double v) { return std::isfinite(v); })) {
+      same = couples == 0;
+      flip = couples == 1;
+    }
     // mirror signs: column j (fold out) or row i (fold in) symmetric or antisymmetric
     auto mirrored = [&](bool out, int parity) {  // index of parity `parity` symmetric, else antisymmetric
       const int nl = out ? cols : rows, nm = out ? rows : cols;
@@ -525,11 +532,11 @@ static std::unique_ptr<Solver> make_solver(SKind kind, const Basis& b0, const Ba
       LMat H = inverse(M) * g.p;  // (m x n)
       if (ax == 0) {
         upload_op(s->hx, H);
-        s->hxp.pack(H.to_double(), H.r, H.c);
+        s->hxp.pack(H.to_double(), H.r, H.c, 0);
         s->hxl = H;
       } else {
         upload_op(s->hy, H.t());
-        s->hyp.pack(H.to_double(), H.r, H.c);
+        s->hyp.pack(H.to_double(), H.r, H.c, 0);
       }
     }
     return s;
@@ -1097,7 +1104,7 @@ class Navier {
     if (!per) {
       const LMat d = build_axis_op(bx_u, "DS", (ld)scale[0]);
       const LMat m = d * solver[0]->hxl;
-      dhx.pack(m.to_double(), m.r, m.c);
+      dhx.pack(m.to_double(), m.r, m.c, 1);
       if (!share) {
         const LMat fo = build_axis_op(bx_u, "FO", (ld)scale[0]);
         solver[3]->left = {fo * build_axis_op(bx_phi, "DS", (ld)scale[0]), fo * build_axis_op(bx_phi, "S", (ld)scale[0])};
